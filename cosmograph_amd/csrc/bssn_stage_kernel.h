@@ -129,18 +129,21 @@ __device__ __host__ constexpr int stencil_seq(int s) {
 // sits at a position s % 3 != 1:
 // PHI, KK, G11, G12, GAM1, G13, G22, GAM2, G23, G33, GAM3, [ALPHA],
 // [12 dust fluxes, or 4 tiles of three], A11..A33 (everything after the head
-// is FP32).  KG (every field 4 bytes): K and Gamma^i in two two-field tiles
-// at positions 2 and 5 (buffer 2, the larger one), the head
-// PHI, G11, (K, GAM1), G12, G13, (GAM2, GAM3), G22, G23, G33.
+// is FP32).  KG (every field 4 bytes, three buffers of one size): the metric
+// first, then [ALPHA] and K, Gamma^i in two two-field tiles:
+// PHI, G11..G33, [ALPHA], (K, GAM1), (GAM2, GAM3).
 template <bool LA, bool DU = false, bool GRP = false, bool KG = false>
 __device__ __host__ constexpr int stencil_seq_split(int s) {
   constexpr int head[11] = {PHI, KK, G11, G12, GAM1, G13, G22, GAM2, G23, G33, GAM3};
-  constexpr int headk[9] = {PHI, G11, KG0, G12, G13, KG1, G22, G23, G33};
-  constexpr int NH = KG ? 9 : 11;
-  if (s < NH) return KG ? headk[s] : head[s];
+  constexpr int NH = KG ? 7 : 11;
+  if (s < NH) return KG ? (s == 0 ? PHI : G11 + (s - 1)) : head[s];
   if (LA) {
     if (s == NH) return ALPHA;
     s -= 1;
+  }
+  if (KG) {
+    if (s < NH + 2) return s == NH ? KG0 : KG1;
+    s -= 2;
   }
   if (DU && GRP) {
     if (s < NH + NDUST) return FLUXG0 + (s - NH);
@@ -263,7 +266,8 @@ __device__ __forceinline__ void morton_xy(int m, int lx, int ly, int& x, int& y)
 // differentiated, in three LDS buffers.  No registers hold the loads in
 // flight.  Requires nz % 4 == 0 and no stage-1 normalisation (a.normalize is
 // ignored); the launcher falls back to DMA = false otherwise.
-template <typename TS, typename TC, int R, int H, int TI, int TJ, int TK, bool LIVE_ALPHA, int MODE, bool DMA = false>
+template <typename TS, typename TC, int R, int H, int TI, int TJ, int TK, int WPE, bool LIVE_ALPHA, int MODE,
+          bool DMA = false>
 __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, const FrwV fv) {
   constexpr int NT = TI * TJ * TK;
   // Halo along k: H; with DMA staging rounded up so that every 16-byte group
@@ -288,8 +292,22 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
   constexpr int NW = NT / 64;                                   // waves per block
   constexpr int NPR = HV / 2, NQD = HV4 / 4;                    // FP64 pairs, FP32 quads per tile
   constexpr int CPR = (NPR + 63) / 64, CQD = (NQD + 63) / 64;   // chunks per field
-  constexpr int P64 = CPR * 1024, P32 = SPLIT ? CQD * 1024 : P64;  // staging buffer bytes
   constexpr bool M32 = (MODE & MODE_M32) != 0;                  // metric in the storage type
+  constexpr bool CONS = (MODE & MODE_CONS) != 0;
+  constexpr bool DUST = (MODE & MODE_DUST) != 0;
+  constexpr int KO_ORDER = (H > R) ? 2 * R : 0;
+  // axis-only tiles: the points within H along one axis of the tile's own
+  // (x part: HI x TJ x TK, y part: TI x HJ x TK, z part: TI x TJ x HK4)
+  constexpr int FGX = HI * TJ * TK, FGY = TI * HJ * TK, FGZ = TI * TJ * HK4;
+  // every field 4 bytes, no KO: K and the Gamma^i, which only have first
+  // derivatives, go two to a tile, each field in the same three parts, where
+  // that loads clearly less than two full tiles (the halo of 3 of order 6)
+  constexpr int NCR = FGX + FGY + FGZ, NQK = 2 * NCR / 4, CKG = (NQK + 63) / 64;
+  constexpr bool KGRP = DMA && M32 && KO_ORDER == 0 && !CONS && CKG <= CPR;
+  // staging buffers: split precision has two of an FP64 tile and one of an
+  // FP32 tile; otherwise all three hold any tile
+  constexpr int CB = KGRP && CKG > CQD ? CKG : CQD;
+  constexpr int P64 = (M32 ? CB : CPR) * 1024, P32 = (M32 ? CB : SPLIT ? CQD : CPR) * 1024;
   constexpr bool MQ = M32 && (MODE & MODE_MQ) != 0;             // ... as 32-bit fixed point
   // metric tiles hold the fixed-point words (FP32 compute); with FP64
   // compute (constraint mode) they hold the scaled FP64 values instead
@@ -304,11 +322,10 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
   constexpr int N64 = M32 ? 0 : SPLIT ? 7 : (LIVE_ALPHA ? NF : NF - 1);  // FP64-stored fields updated (ALPHA last)
   constexpr int N32 = M32 ? (LIVE_ALPHA ? NF : NF - 1) : SPLIT ? (LIVE_ALPHA ? NF - 7 : NF - 8) : 0;  // FP32 ones
   // every field 4 bytes, frozen lapse: stage 4 of the accumulator-free form
-  // also prefetches a2 of the first NA2 fields, in the groups (16 lanes, 64
-  // points, one field) of the staging LDS left after the _p/_f groups (a
-  // 52 KB layout with every a2, issued from one loop with _p/_f, measured
-  // stage 4 0.21 ms faster but stages 1-3 0.12 ms slower at 256^3)
-  constexpr int LSTAGE = 2 * P64 + P32;
+  // also prefetches a2 of the last NA2 fields, in the groups (16 lanes, 64
+  // points, one field) of the block's share of LDS left after the _p/_f groups
+  constexpr int LBLOCK = (160 / (WPE > 2 ? WPE : 3)) * 1024 / 4096 * 4096;  // one block per SIMD wave
+  constexpr int LSTAGE = M32 && NT == 256 && 2 * P64 + P32 < LBLOCK ? LBLOCK : 2 * P64 + P32;
   constexpr bool PF2 = PF && M32 && !LIVE_ALPHA;
   constexpr int CPF = (2 * N32 + 3) / 4;                        // _p/_f chunks of the FP32 fields
   constexpr int NA2_ = PF2 ? (LSTAGE / (NW * 1024) - N64 - CPF) * 4 : 0;
@@ -412,8 +429,6 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
                                                                                                  : a.s_in);
   };
   auto RD = [&](int q, int slot) -> TS* { return (TS*)a.dreg + ((long)q * 4 + slot) * a.rstride; };
-  constexpr bool CONS = (MODE & MODE_CONS) != 0;
-  constexpr bool DUST = (MODE & MODE_DUST) != 0;
   const bool norm = !DMA && a.normalize != 0;
 
   // stage-1 unit-determinant factor at the halo points (bssn.cc:75-99):
@@ -607,8 +622,18 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
   const double i1 = a.inv_dx, i2 = a.inv_dx2;
   const TC idx1 = (TC)a.inv_dx;
   TC dg[3][6];      // d_k gamma_ij
-  TC T1[6];         // gamma^{kl} d_k d_l gamma_ij
-  TC dphi[3], ddphi[6], dal[3], ddal[6], dK[3], dG[3][3];
+  // conformal Ricci tensor, accumulated as its inputs arrive:
+  // -1/2 gamma^{kl} d_k d_l gamma_ij per metric field, the d_j Gamma^k terms
+  // per Gamma^k, the rest in curvature()
+  TC ric[6] = {TC(0), TC(0), TC(0), TC(0), TC(0), TC(0)};
+  // (split precision: the d_j Gamma^k terms in a sum of their own, because
+  // its DMA staging has two Gamma^k before the last metric field and the
+  // register path none, and both shall add in the same order)
+  constexpr bool SEPG = sizeof(TS) == 4 && !M32;
+  TC ricG[SEPG ? 6 : 1];
+#pragma unroll
+  for (int q = 0; q < (SEPG ? 6 : 1); ++q) ricG[q] = TC(0);
+  TC dphi[3], ddphi[6], dal[3], ddal[6], dK[3];
   TC dA[3][6];      // d_j A_kl, constraint mode only
   TC ddust[NDUST];  // sum_i d_i of the dust fluxes
 #pragma unroll
@@ -616,24 +641,19 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
   TC ko[NF];
 #pragma unroll
   for (int f = 0; f < NF; ++f) ko[f] = TC(0);
-  const bool use_ko = a.use_ko != 0;
-  constexpr int KO_ORDER = (H > R) ? 2 * R : 0;
 
   // stencil fields in order; A_ij only when KO is active or for the
   // constraints; the dust fluxes only in the dust stage
   constexpr bool FLUXES = DUST && !CONS;
-  // 4-byte DMA staging: the three fluxes of a quantity share one LDS tile,
-  // each with the halo of its own derivative axis only (x part: HI x TJ x
-  // TK, y part: TI x HJ x TK, z part: TI x TJ x HK4)
+  // 4-byte DMA staging: the three fluxes of a quantity share one axis-only
+  // tile, each with the halo of its own derivative axis
   constexpr bool FGRP = DMA && FLUXES && SPLIT;
-  constexpr int FGX = HI * TJ * TK, FGY = TI * HJ * TK, FGZ = TI * TJ * HK4;
-  // every field 4 bytes, no KO: K and the Gamma^i, which only have first
-  // derivatives, go two to a tile, each field in the same three parts, where
-  // such a tile fits the larger staging buffers (the halo of 3 of order 6)
-  constexpr bool KGRP = DMA && M32 && KO_ORDER == 0 && !CONS &&
-                        (2 * (FGX + FGY + FGZ) / 4 + 63) / 64 <= (HV / 2 + 63) / 64;
-  constexpr int NSEQ = (LIVE_ALPHA ? 18 : 17) - (KGRP ? 2 : 0) + (FLUXES ? (FGRP ? NDUST : NFLUX) : 0);
-  const int nseq = (use_ko || CONS) ? NSEQ : NSEQ - 6;
+  // position after which every field curvature() needs is differentiated:
+  // the last of the metric fields and ALPHA in the staging order
+  constexpr int MID = SPLIT && DMA && !KGRP ? (LIVE_ALPHA ? 11 : 9) : (LIVE_ALPHA ? 7 : 6);
+  // (a halo beyond the derivatives' is there for KO only, which differentiates A_ij too)
+  constexpr int NSEQ = (LIVE_ALPHA ? 18 : 17) - (KGRP ? 2 : 0) + (FLUXES ? (FGRP ? NDUST : NFLUX) : 0) -
+                       (KO_ORDER || CONS ? 0 : 6);
   if constexpr (!LIVE_ALPHA) {
 #pragma unroll
     for (int d = 0; d < 3; ++d) dal[d] = TC(0);
@@ -641,13 +661,151 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
     for (int d = 0; d < 6; ++d) ddal[d] = TC(0);
   }
 
+  // -1/2 gamma^{kl} d_k d_l of metric component f into the Ricci tensor
+  auto add_lap = [&](int f, TC e00, TC e01, TC e02, TC e11, TC e12, TC e22) {
+    if (f < 6)
+      ric[f < 6 ? f : 0] -= TC(0.5) * (gi[0] * e00 + gi[3] * e11 + gi[5] * e22) +
+                            (gi[1] * e01 + gi[2] * e02 + gi[4] * e12);
+  };
+  // 1/2 (gamma_ki d_j Gamma^k + gamma_kj d_i Gamma^k) of one k
+  auto add_dG = [&](int k, TC d0, TC d1, TC d2) {
+    const TC d[3] = {d0, d1, d2};
+#pragma unroll
+    for (int I = 0; I < 3; ++I)
+#pragma unroll
+      for (int J = I; J < 3; ++J)
+        (SEPG ? ricG[SEPG ? sy(I, J) : 0] : ric[sy(I, J)]) += I == J ? GM(k, I) * d[I] : TC(0.5) * (GM(k, I) * d[J] + GM(k, J) * d[I]);
+  };
+  // Everything that needs the first derivatives of the metric, formed as soon
+  // as the last of DIFFgamma_ij, DIFFphi (and DIFFalpha) is differentiated:
+  // after it the Christoffel symbols and d_k gamma_ij are dead, and while the
+  // remaining fields are staged only the sums below stay live.  The kernels
+  // are bound by how many waves their registers allow: with the whole
+  // algebra after the last field, the FP64 kernel held 256 VGPRs and spilled
+  // 188 B (0.421 ms per stage at 128^3, order 4; now 242, no spill, 0.285
+  // ms), the fixed-point one 157 (1.62 ms at 256^3, order 6; now 126, four
+  // waves, 1.535 ms).
+  TC GL[3][6], G[3][6], Gd[3];
+  TC Ac[6], AijAij = TC(0), second[3];  // A^ij, A_ij A^ij, Gamma^i_jk A^jk + 6 A^ij d_j phi
+  TC DDa[6], DDaTR = TC(0);             // (D_i D_j alpha)^TF and its trace (without e^{-4 phi})
+  auto curvature = [&]() {
+    // Christoffels (bssn_macros.h:221-229):  GL_ijk = 1/2(d_j g_ki + d_k g_ji - d_i g_jk),
+    // G^i_jk = gamma^{im} GL_mjk
+  #pragma unroll
+    for (int I = 0; I < 3; ++I)
+  #pragma unroll
+      for (int J = 0; J < 3; ++J)
+  #pragma unroll
+        for (int Kx = J; Kx < 3; ++Kx)
+          GL[I][sy(J, Kx)] = TC(0.5) * (dg[J][sy(Kx, I)] + dg[Kx][sy(J, I)] - dg[I][sy(J, Kx)]);
+  #pragma unroll
+    for (int I = 0; I < 3; ++I)
+  #pragma unroll
+      for (int s = 0; s < 6; ++s) G[I][s] = GI(I, 0) * GL[0][s] + GI(I, 1) * GL[1][s] + GI(I, 2) * GL[2][s];
+  #pragma unroll
+    for (int I = 0; I < 3; ++I)
+      Gd[I] = G[I][0] * gi[0] + G[I][3] * gi[3] + G[I][5] * gi[5] + TC(2) * (G[I][1] * gi[1] + G[I][2] * gi[2] + G[I][4] * gi[4]);
+
+    // D_i D_j phi (bssn.cc:592-602)
+    TC DDphi[6];
+  #pragma unroll
+    for (int s = 0; s < 6; ++s) DDphi[s] = ddphi[s] - (G[0][s] * dphi[0] + G[1][s] * dphi[1] + G[2][s] * dphi[2]);
+
+    // (D_i D_j alpha)^TF and its trace (bssn.cc:604-626)
+  #pragma unroll
+    for (int q = 0; q < 6; ++q) DDa[q] = TC(0);
+    if constexpr (LIVE_ALPHA) {
+      TC gild[3];
+  #pragma unroll
+      for (int I = 0; I < 3; ++I) gild[I] = GI(I, 0) * dphi[0] + GI(I, 1) * dphi[1] + GI(I, 2) * dphi[2];
+  #pragma unroll
+      for (int I = 0; I < 3; ++I)
+  #pragma unroll
+        for (int J = I; J < 3; ++J) {
+          const int s = sy(I, J);
+          TC acc = TC(0);
+  #pragma unroll
+          for (int m = 0; m < 3; ++m)
+            acc += (G[m][s] + TC(2) * ((m == I ? dphi[J] : TC(0)) + (m == J ? dphi[I] : TC(0)) - GM(I, J) * gild[m])) * dal[m];
+          DDa[s] = ddal[s] - acc;
+        }
+      DDaTR = gi[0] * DDa[0] + gi[3] * DDa[3] + gi[5] * DDa[5] + TC(2) * (gi[1] * DDa[1] + gi[2] * DDa[2] + gi[4] * DDa[4]);
+  #pragma unroll
+      for (int s = 0; s < 6; ++s) DDa[s] -= TC(1.0 / 3.0) * (v[G11 + s] + (diag6(s) ? TC(1) : TC(0))) * DDaTR;
+    }
+
+    // conformal Ricci (bssn_macros.h:248-277).  TERM4 is regrouped as
+    //   sum_{K,M} X[K][I][M] Y[J][K][M] + (I<->J),
+    //   X[K][I][M] = gamma^{ML} G^K_{LI},  Y[J][K][M] = GL_{J,KM} + 1/2 GL_{K,MJ}
+  #pragma unroll
+    for (int Kx = 0; Kx < 3; ++Kx) {
+      TC X[3][3], Y[3][3];
+  #pragma unroll
+      for (int I = 0; I < 3; ++I)
+  #pragma unroll
+        for (int M = 0; M < 3; ++M)
+          X[I][M] = GI(M, 0) * G[Kx][sy(0, I)] + GI(M, 1) * G[Kx][sy(1, I)] + GI(M, 2) * G[Kx][sy(2, I)];
+  #pragma unroll
+      for (int J = 0; J < 3; ++J)
+  #pragma unroll
+        for (int M = 0; M < 3; ++M) Y[J][M] = GL[J][sy(Kx, M)] + TC(0.5) * GL[Kx][sy(M, J)];
+  #pragma unroll
+      for (int I = 0; I < 3; ++I)
+  #pragma unroll
+        for (int J = I; J < 3; ++J) {
+          const TC z = X[I][0] * Y[J][0] + X[I][1] * Y[J][1] + X[I][2] * Y[J][2];
+          if (I == J) ric[sy(I, J)] += TC(2) * z;
+          else ric[sy(I, J)] += z + (X[J][0] * Y[I][0] + X[J][1] * Y[I][1] + X[J][2] * Y[I][2]);
+        }
+    }
+    {
+      // phi part (bssn.cc:639-655)
+      const TC expression =
+          gi[0] * (DDphi[0] + TC(2) * dphi[0] * dphi[0]) + gi[3] * (DDphi[3] + TC(2) * dphi[1] * dphi[1]) +
+          gi[5] * (DDphi[5] + TC(2) * dphi[2] * dphi[2]) +
+          TC(2) * (gi[1] * (DDphi[1] + TC(2) * dphi[0] * dphi[1]) + gi[2] * (DDphi[2] + TC(2) * dphi[0] * dphi[2]) +
+                   gi[4] * (DDphi[4] + TC(2) * dphi[1] * dphi[2]));
+  #pragma unroll
+      for (int I = 0; I < 3; ++I)
+  #pragma unroll
+        for (int J = I; J < 3; ++J) {
+          const int s = sy(I, J);
+          TC t3 = TC(0);
+  #pragma unroll
+          for (int k = 0; k < 3; ++k) t3 += Gd[k] * (GL[I][sy(J, k)] + GL[J][sy(I, k)]);
+          ric[s] += TC(0.5) * t3 - TC(2) * (DDphi[s] - TC(2) * dphi[I] * dphi[J] + GM(I, J) * expression);
+        }
+    }
+
+    // A^ij and A_ij A^ij (bssn.cc:463-472)
+  #pragma unroll
+    for (int I = 0; I < 3; ++I)
+  #pragma unroll
+      for (int J = I; J < 3; ++J) {
+        TC acc = TC(0);
+  #pragma unroll
+        for (int p = 0; p < 3; ++p) {
+          const TC w = GI(I, p);
+          acc += w * (GI(J, 0) * AM(p, 0) + GI(J, 1) * AM(p, 1) + GI(J, 2) * AM(p, 2));
+        }
+        Ac[sy(I, J)] = acc;
+      }
+    AijAij = Ac[0] * v[A11] + Ac[3] * v[A22] + Ac[5] * v[A33] +
+             TC(2) * (Ac[1] * v[A12] + Ac[2] * v[A13] + Ac[4] * v[A23]);
+  #pragma unroll
+    for (int I = 0; I < 3; ++I)
+      second[I] = G[I][0] * Ac[0] + G[I][3] * Ac[3] + G[I][5] * Ac[5] +
+                  TC(2) * (G[I][1] * Ac[1] + G[I][2] * Ac[2] + G[I][4] * Ac[4]) +
+                  TC(6) * (Ac[sy(I, 0)] * dphi[0] + Ac[sy(I, 1)] * dphi[1] + Ac[sy(I, 2)] * dphi[2]);
+  };
+
   // derivatives of field f, staged in the LDS tile BUF, at this thread's
   // point, folded into the per-point tensors (a macro: the same code as a
   // lambda allocates registers differently and spills)
 #define CG_DERIVE(f, BUF) \
     if (mfield<M32>(f)) {                                                                                               \
       const double* __restrict__ L = reinterpret_cast<const double*>(BUF);                                               \
-      if (KO_ORDER && use_ko) ko[f] = (TC)(a.ko_pref * ko_sum<KO_ORDER, double>(L, c, SI, SJ, SK));                      \
+      if (KO_ORDER) ko[f] = (TC)(a.ko_pref * ko_sum<KO_ORDER, double>(L, c, SI, SJ, SK));                      \
       const double d0 = fd1<R>(L, c, SI) * i1, d1 = fd1<R>(L, c, SJ) * i1, d2 = fd1<R>(L, c, SK) * i1;                   \
       const double e00 = fd2<R>(L, c, SI) * i2, e11 = fd2<R>(L, c, SJ) * i2, e22 = fd2<R>(L, c, SK) * i2;                \
       const double e01 = fdm<R>(L, c, SI, SJ) * i2, e02 = fdm<R>(L, c, SI, SK) * i2,                                     \
@@ -658,13 +816,12 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
         ddphi[3] = (TC)e11; ddphi[4] = (TC)e12; ddphi[5] = (TC)e22;                                                      \
       } else {                                                                                                           \
         dg[0][f] = (TC)d0; dg[1][f] = (TC)d1; dg[2][f] = (TC)d2;                                                         \
-        T1[f] = gi[0] * (TC)e00 + gi[3] * (TC)e11 + gi[5] * (TC)e22 +                                                    \
-                TC(2) * (gi[1] * (TC)e01 + gi[2] * (TC)e02 + gi[4] * (TC)e12);                                           \
+        add_lap(f, (TC)e00, (TC)e01, (TC)e02, (TC)e11, (TC)e12, (TC)e22);                                                \
       }                                                                                                                  \
     } else {                                                                                                             \
       const TC* __restrict__ L = reinterpret_cast<const TC*>(BUF);                                                       \
       const int* __restrict__ LQ = reinterpret_cast<const int*>(BUF);                                                    \
-      if (KO_ORDER && use_ko && f < NF) {                                                                                \
+      if (KO_ORDER && f < NF) {                                                                                \
         if (MQW && (f <= G33 || f == PHI))                                                                               \
           ko[f] = (TC)(a.ko_pref * a.msc[f < 7 ? f : 0] * ko_sumq<KO_ORDER>(LQ, c4, SI4, SJ4, SK));                      \
         else                                                                                                             \
@@ -682,7 +839,7 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
           ddphi[0] = e00; ddphi[1] = e01; ddphi[2] = e02; ddphi[3] = e11; ddphi[4] = e12; ddphi[5] = e22;                \
         } else {                                                                                                         \
           dg[0][f] = d0; dg[1][f] = d1; dg[2][f] = d2;                                                                   \
-          T1[f] = gi[0] * e00 + gi[3] * e11 + gi[5] * e22 + TC(2) * (gi[1] * e01 + gi[2] * e02 + gi[4] * e12);          \
+          add_lap(f, e00, e01, e02, e11, e12, e22);                                                                      \
         }                                                                                                                \
       } else if (M32 && (f <= G33 || f == PHI)) {                                                                        \
         const TC idx2 = (TC)a.inv_dx2;                                                                                   \
@@ -695,7 +852,7 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
           ddphi[0] = e00; ddphi[1] = e01; ddphi[2] = e02; ddphi[3] = e11; ddphi[4] = e12; ddphi[5] = e22;                \
         } else {                                                                                                         \
           dg[0][f] = d0; dg[1][f] = d1; dg[2][f] = d2;                                                                   \
-          T1[f] = gi[0] * e00 + gi[3] * e11 + gi[5] * e22 + TC(2) * (gi[1] * e01 + gi[2] * e02 + gi[4] * e12);          \
+          add_lap(f, e00, e01, e02, e11, e12, e22);                                                                      \
         }                                                                                                                \
       } else if (f == ALPHA) {                                                                                           \
         const TC idx2 = (TC)a.inv_dx2;                                                                                   \
@@ -706,9 +863,7 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
       } else if (f == KK) {                                                                                              \
         dK[0] = fd1<R>(L, c4, SI4) * idx1; dK[1] = fd1<R>(L, c4, SJ4) * idx1; dK[2] = fd1<R>(L, c4, SK) * idx1;          \
       } else if (f >= GAM1 && f <= GAM3) {                                                                               \
-        const int kk = f - GAM1;                                                                                         \
-        dG[0][kk] = fd1<R>(L, c4, SI4) * idx1; dG[1][kk] = fd1<R>(L, c4, SJ4) * idx1;                                    \
-        dG[2][kk] = fd1<R>(L, c4, SK) * idx1;                                                                            \
+        add_dG(f - GAM1, fd1<R>(L, c4, SI4) * idx1, fd1<R>(L, c4, SJ4) * idx1, fd1<R>(L, c4, SK) * idx1);                \
       } else if (CONS && f >= A11 && f <= A33) {                                                                         \
         const int q = f - A11;                                                                                           \
         dA[0][q] = fd1<R>(L, c4, SI4) * idx1; dA[1][q] = fd1<R>(L, c4, SJ4) * idx1; dA[2][q] = fd1<R>(L, c4, SK) * idx1; \
@@ -723,9 +878,11 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
           dd[h][2] = fd1<R>(L, h * (FGX + FGY + FGZ) + cz, 1) * idx1;                                                    \
         }                                                                                                                \
         if (f == KG0) {                                                                                                  \
-          _Pragma("unroll") for (int d = 0; d < 3; ++d) { dK[d] = dd[0][d]; dG[d][0] = dd[1][d]; }                      \
+          _Pragma("unroll") for (int d = 0; d < 3; ++d) dK[d] = dd[0][d];                                               \
+          add_dG(0, dd[1][0], dd[1][1], dd[1][2]);                                                                       \
         } else {                                                                                                         \
-          _Pragma("unroll") for (int d = 0; d < 3; ++d) { dG[d][1] = dd[0][d]; dG[d][2] = dd[1][d]; }                   \
+          add_dG(1, dd[0][0], dd[0][1], dd[0][2]);                                                                       \
+          add_dG(2, dd[1][0], dd[1][1], dd[1][2]);                                                                       \
         }                                                                                                                \
       } else if (FGRP && f >= FLUXG0) {                                                                                  \
         /* the three fluxes of quantity q, each along its own axis, summed in the order x, y, z */                       \
@@ -804,8 +961,8 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
     // then its x, y and z parts as a flux tile; the second field's register
     // is 4 * rstride elements after the first's (the launcher keeps
     // 5 * rstride * 4 bytes below 2^32)
-    constexpr int NCR = FGX + FGY + FGZ, NQK = 2 * NCR / 4, CKG = (NQK + 63) / 64, MKG = (CKG + NW - 1) / NW;
-    static_assert(!KGRP || (FGX % 4 == 0 && FGY % 4 == 0 && CKG <= CPR), "two-field tiles: whole quads, buffer 2");
+    constexpr int MKG = (CKG + NW - 1) / NW;
+    static_assert(!KGRP || (FGX % 4 == 0 && FGY % 4 == 0), "two-field tiles: whole quads");
     auto kchunk = [&](int m) { const int ch = wv + m * NW; return ch < CKG ? ch : CKG - 1; };
     unsigned koff[KGRP ? MKG : 1];
     if constexpr (KGRP) {
@@ -848,28 +1005,30 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
       return SPLIT ? stencil_seq_split<LIVE_ALPHA, FLUXES, FGRP, KGRP>(s) : stencil_seq<LIVE_ALPHA, FLUXES>(s);
     };
     dma(seq(0), 0);
-    if (nseq > 1) dma(seq(1), 1);
-#pragma unroll
-    for (int s = 0; s < NSEQ; ++s) {
-      if (s < nseq) {
-        // position s has landed for this wave once at most the chunks of
-        // position s + 1 are outstanding; for every wave after the barrier
-        const int f1 = seq(s + 1 < NSEQ ? s + 1 : 0);
-        if (s + 1 < nseq) {
-          if (!SPLIT || mfield<M32>(f1)) dma_wait_barrier<MPR>();
-          else if (KGRP && f1 >= KG0) dma_wait_barrier<MKG>();
-          else if (FGRP && f1 >= FLUXG0) dma_wait_barrier<MFG>();
-          else dma_wait_barrier<MQD>();
-        } else {
-          dma_wait_barrier<0>();
-        }
-        // buffer (s + 2) % 3 was last read at position s - 1, before the barrier
-        if (s + 2 < nseq) dma(seq(s + 2 < NSEQ ? s + 2 : 0), (s + 2) % 3);
-        const int f = seq(s);
-        const void* const buf = s % 3 == 0 ? (const void*)lb0 : s % 3 == 1 ? (const void*)lb1 : (const void*)lb2;
-        if (valid) { CG_DERIVE(f, buf); }
+    dma(seq(1), 1);
+    auto stage_field = [&](const int s) {
+      // position s has landed for this wave once at most the chunks of
+      // position s + 1 are outstanding; for every wave after the barrier
+      const int f1 = seq(s + 1 < NSEQ ? s + 1 : 0);
+      if (s + 1 < NSEQ) {
+        if (!SPLIT || mfield<M32>(f1)) dma_wait_barrier<MPR>();
+        else if (KGRP && f1 >= KG0) dma_wait_barrier<MKG>();
+        else if (FGRP && f1 >= FLUXG0) dma_wait_barrier<MFG>();
+        else dma_wait_barrier<MQD>();
+      } else {
+        dma_wait_barrier<0>();
       }
-    }
+      // buffer (s + 2) % 3 was last read at position s - 1, before the barrier
+      if (s + 2 < NSEQ) dma(seq(s + 2 < NSEQ ? s + 2 : 0), (s + 2) % 3);
+      const int f = seq(s);
+      const void* const buf = s % 3 == 0 ? (const void*)lb0 : s % 3 == 1 ? (const void*)lb1 : (const void*)lb2;
+      if (valid) { CG_DERIVE(f, buf); }
+    };
+#pragma unroll
+    for (int s = 0; s <= MID; ++s) stage_field(s);
+    if (valid) curvature();
+#pragma unroll
+    for (int s = MID + 1; s < NSEQ; ++s) stage_field(s);
     // Every point value has arrived by now (the last staging wait drained
     // the vector memory counter).  The compiler does not see the asm waits:
     // touching the values here puts its own waits for them here, where they
@@ -930,18 +1089,20 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
     store(0, PHI);
     __syncthreads();
 
+    auto stage_field = [&](const int s) {
+      const bool more = s + 1 < NSEQ;
+      const int fn = stencil_seq<LIVE_ALPHA, FLUXES>(more ? s + 1 : 0);
+      if (more) fetch(fn);
+      const int f = stencil_seq<LIVE_ALPHA, FLUXES>(s);
+      if (valid) { CG_DERIVE(f, ldsraw[s & 1]); }
+      if (more) store((s + 1) & 1, fn);
+      __syncthreads();
+    };
   #pragma unroll
-    for (int s = 0; s < NSEQ; ++s) {
-      if (s < nseq) {
-        const bool more = (s + 1) < nseq;
-        const int fn = stencil_seq<LIVE_ALPHA, FLUXES>((s + 1) < NSEQ ? s + 1 : 0);
-        if (more) fetch(fn);
-        const int f = stencil_seq<LIVE_ALPHA, FLUXES>(s);
-        if (valid) { CG_DERIVE(f, ldsraw[s & 1]); }
-        if (more) store((s + 1) & 1, fn);
-        __syncthreads();
-      }
-    }
+    for (int s = 0; s <= MID; ++s) stage_field(s);
+    if (valid) curvature();
+  #pragma unroll
+    for (int s = MID + 1; s < NSEQ; ++s) stage_field(s);
   }
 #undef CG_DERIVE
   // Threads outside the grid (ragged edge tiles) skip the algebra but stay
@@ -1083,121 +1244,12 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
       }
     }
 
-    // A^ij and A_ij A^ij (bssn.cc:463-472)
-    TC Ac[6];
+    if constexpr (SEPG) {
   #pragma unroll
-    for (int I = 0; I < 3; ++I)
-  #pragma unroll
-      for (int J = I; J < 3; ++J) {
-        TC acc = TC(0);
-  #pragma unroll
-        for (int p = 0; p < 3; ++p) {
-          const TC w = GI(I, p);
-          acc += w * (GI(J, 0) * AM(p, 0) + GI(J, 1) * AM(p, 1) + GI(J, 2) * AM(p, 2));
-        }
-        Ac[sy(I, J)] = acc;
-      }
-    const TC AijAij = Ac[0] * v[A11] + Ac[3] * v[A22] + Ac[5] * v[A33] +
-                      TC(2) * (Ac[1] * v[A12] + Ac[2] * v[A13] + Ac[4] * v[A23]);
-
-    // Christoffels (bssn_macros.h:221-229):  GL_ijk = 1/2(d_j g_ki + d_k g_ji - d_i g_jk),
-    // G^i_jk = gamma^{im} GL_mjk
-    TC GL[3][6], G[3][6];
-  #pragma unroll
-    for (int I = 0; I < 3; ++I)
-  #pragma unroll
-      for (int J = 0; J < 3; ++J)
-  #pragma unroll
-        for (int Kx = J; Kx < 3; ++Kx)
-          GL[I][sy(J, Kx)] = TC(0.5) * (dg[J][sy(Kx, I)] + dg[Kx][sy(J, I)] - dg[I][sy(J, Kx)]);
-  #pragma unroll
-    for (int I = 0; I < 3; ++I)
-  #pragma unroll
-      for (int s = 0; s < 6; ++s) G[I][s] = GI(I, 0) * GL[0][s] + GI(I, 1) * GL[1][s] + GI(I, 2) * GL[2][s];
-    TC Gd[3];
-  #pragma unroll
-    for (int I = 0; I < 3; ++I)
-      Gd[I] = G[I][0] * gi[0] + G[I][3] * gi[3] + G[I][5] * gi[5] + TC(2) * (G[I][1] * gi[1] + G[I][2] * gi[2] + G[I][4] * gi[4]);
-
-    // D_i D_j phi (bssn.cc:592-602)
-    TC DDphi[6];
-  #pragma unroll
-    for (int s = 0; s < 6; ++s) DDphi[s] = ddphi[s] - (G[0][s] * dphi[0] + G[1][s] * dphi[1] + G[2][s] * dphi[2]);
-
-    // (D_i D_j alpha)^TF and its trace (bssn.cc:604-626)
-    TC DDa[6], DDaTR = TC(0);
-  #pragma unroll
-    for (int q = 0; q < 6; ++q) DDa[q] = TC(0);
-    if constexpr (LIVE_ALPHA) {
-      TC gild[3];
-  #pragma unroll
-      for (int I = 0; I < 3; ++I) gild[I] = GI(I, 0) * dphi[0] + GI(I, 1) * dphi[1] + GI(I, 2) * dphi[2];
-  #pragma unroll
-      for (int I = 0; I < 3; ++I)
-  #pragma unroll
-        for (int J = I; J < 3; ++J) {
-          const int s = sy(I, J);
-          TC acc = TC(0);
-  #pragma unroll
-          for (int m = 0; m < 3; ++m)
-            acc += (G[m][s] + TC(2) * ((m == I ? dphi[J] : TC(0)) + (m == J ? dphi[I] : TC(0)) - GM(I, J) * gild[m])) * dal[m];
-          DDa[s] = ddal[s] - acc;
-        }
-      DDaTR = gi[0] * DDa[0] + gi[3] * DDa[3] + gi[5] * DDa[5] + TC(2) * (gi[1] * DDa[1] + gi[2] * DDa[2] + gi[4] * DDa[4]);
-  #pragma unroll
-      for (int s = 0; s < 6; ++s) DDa[s] -= TC(1.0 / 3.0) * (v[G11 + s] + (diag6(s) ? TC(1) : TC(0))) * DDaTR;
+      for (int q = 0; q < 6; ++q) ric[q] += ricG[q];
     }
     const TC em4phi = exp(TC(-4) * phi);
     DDaTR *= em4phi;
-
-    // conformal Ricci (bssn_macros.h:248-277).  TERM4 is regrouped as
-    //   sum_{K,M} X[K][I][M] Y[J][K][M] + (I<->J),
-    //   X[K][I][M] = gamma^{ML} G^K_{LI},  Y[J][K][M] = GL_{J,KM} + 1/2 GL_{K,MJ}
-    TC Z[3][3];
-  #pragma unroll
-    for (int I = 0; I < 3; ++I)
-  #pragma unroll
-      for (int J = 0; J < 3; ++J) Z[I][J] = TC(0);
-  #pragma unroll
-    for (int Kx = 0; Kx < 3; ++Kx) {
-      TC X[3][3], Y[3][3];
-  #pragma unroll
-      for (int I = 0; I < 3; ++I)
-  #pragma unroll
-        for (int M = 0; M < 3; ++M)
-          X[I][M] = GI(M, 0) * G[Kx][sy(0, I)] + GI(M, 1) * G[Kx][sy(1, I)] + GI(M, 2) * G[Kx][sy(2, I)];
-  #pragma unroll
-      for (int J = 0; J < 3; ++J)
-  #pragma unroll
-        for (int M = 0; M < 3; ++M) Y[J][M] = GL[J][sy(Kx, M)] + TC(0.5) * GL[Kx][sy(M, J)];
-  #pragma unroll
-      for (int I = 0; I < 3; ++I)
-  #pragma unroll
-        for (int J = 0; J < 3; ++J) Z[I][J] += X[I][0] * Y[J][0] + X[I][1] * Y[J][1] + X[I][2] * Y[J][2];
-    }
-    TC ric[6];
-    {
-      // phi part (bssn.cc:639-655)
-      const TC expression =
-          gi[0] * (DDphi[0] + TC(2) * dphi[0] * dphi[0]) + gi[3] * (DDphi[3] + TC(2) * dphi[1] * dphi[1]) +
-          gi[5] * (DDphi[5] + TC(2) * dphi[2] * dphi[2]) +
-          TC(2) * (gi[1] * (DDphi[1] + TC(2) * dphi[0] * dphi[1]) + gi[2] * (DDphi[2] + TC(2) * dphi[0] * dphi[2]) +
-                   gi[4] * (DDphi[4] + TC(2) * dphi[1] * dphi[2]));
-  #pragma unroll
-      for (int I = 0; I < 3; ++I)
-  #pragma unroll
-        for (int J = I; J < 3; ++J) {
-          const int s = sy(I, J);
-          TC t2 = TC(0), t3 = TC(0);
-  #pragma unroll
-          for (int k = 0; k < 3; ++k) {
-            t2 += GM(k, I) * dG[J][k] + GM(k, J) * dG[I][k];
-            t3 += Gd[k] * (GL[I][sy(J, k)] + GL[J][sy(I, k)]);
-          }
-          const TC U = TC(-0.5) * T1[s] + TC(0.5) * t2 + TC(0.5) * t3 + (Z[I][J] + Z[J][I]);
-          ric[s] = U - TC(2) * (DDphi[s] - TC(2) * dphi[I] * dphi[J] + GM(I, J) * expression);
-        }
-    }
     const TC ricci = em4phi * (ric[0] * gi[0] + ric[3] * gi[3] + ric[5] * gi[5] +
                                TC(2) * (ric[1] * gi[1] + ric[2] * gi[2] + ric[4] * gi[4]));
     const TC e4phi = exp(TC(4) * phi);
@@ -1317,12 +1369,9 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
       // bssn_macros.h:340-361
     #pragma unroll
       for (int I = 0; I < 3; ++I) {
-        const TC second = G[I][0] * Ac[0] + G[I][3] * Ac[3] + G[I][5] * Ac[5] +
-                          TC(2) * (G[I][1] * Ac[1] + G[I][2] * Ac[2] + G[I][4] * Ac[4]) +
-                          TC(6) * (Ac[sy(I, 0)] * dphi[0] + Ac[sy(I, 1)] * dphi[1] + Ac[sy(I, 2)] * dphi[2]);
         rhs[GAM1 + I] = TC(-2) * (Ac[sy(I, 0)] * dal[0] + Ac[sy(I, 1)] * dal[1] + Ac[sy(I, 2)] * dal[2]) +
                         TC(2) * alpha *
-                            (second - TC(2.0 / 3.0) * (GI(I, 0) * dK[0] + GI(I, 1) * dK[1] + GI(I, 2) * dK[2]) -
+                            (second[I] - TC(2.0 / 3.0) * (GI(I, 0) * dK[0] + GI(I, 1) * dK[1] + GI(I, 2) * dK[2]) -
                              TC(8) * PI * (GI(I, 0) * Si[0] + GI(I, 1) * Si[1] + GI(I, 2) * Si[2])) -
                         ko[GAM1 + I];
       }
@@ -1560,7 +1609,7 @@ stage_kernel(const StageArgs a) {
   const int b = blockIdx.x;
   const int t = (b & 7) * a.per_xcd + (b >> 3);  // consecutive tiles stay on one XCD
   if (t >= (a.tile_count ? a.tile_count : a.ntx * a.nty * a.ntz)) return;
-  stage_body<TS, TC, R, H, TI, TJ, TK, LIVE_ALPHA, MODE, DMA>(
+  stage_body<TS, TC, R, H, TI, TJ, TK, WPE, LIVE_ALPHA, MODE, DMA>(
       a, a.tile_base + t, FrwV{a.phi_F, a.K_F, a.rho_F, a.S_F, a.H_frw, a.phi_F_next});
 }
 
@@ -1597,7 +1646,7 @@ stage_kernel_batch(const BatchArgs ba) {
   }
   CDouble* const f = (CDouble*)ba.frw + (long)r * FRW_N;
   const StageArgs a = ((CArgs*)ba.tab)[r];
-  stage_body<TS, TC, R, H, TI, TJ, TK, LIVE_ALPHA, 0, DMA>(a, g - ts[r], FrwV{f[0], f[1], f[2], f[3], f[4], f[5]});
+  stage_body<TS, TC, R, H, TI, TJ, TK, WPE, LIVE_ALPHA, 0, DMA>(a, g - ts[r], FrwV{f[0], f[1], f[2], f[3], f[4], f[5]});
 }
 
 // ------------------------------------------------------------ variants

@@ -324,8 +324,8 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
   // every field 4 bytes, frozen lapse: stage 4 of the accumulator-free form
   // also prefetches a2 of the last NA2 fields, in the groups (16 lanes, 64
   // points, one field) of the block's share of LDS left after the _p/_f groups
-  constexpr int LBLOCK = (160 / (WPE > 2 ? WPE : 3)) * 1024 / 4096 * 4096;  // one block per SIMD wave
-  constexpr int LSTAGE = M32 && NT == 256 && 2 * P64 + P32 < LBLOCK ? LBLOCK : 2 * P64 + P32;
+  constexpr int LBLOCK = (160 * NW / 4 / (WPE > 2 ? WPE : 3)) / NW * NW * 1024;  // WPE waves per SIMD share 160 KB
+  constexpr int LSTAGE = M32 && 2 * P64 + P32 < LBLOCK ? LBLOCK : 2 * P64 + P32;
   constexpr bool PF2 = PF && M32 && !LIVE_ALPHA;
   constexpr int CPF = (2 * N32 + 3) / 4;                        // _p/_f chunks of the FP32 fields
   constexpr int NA2_ = PF2 ? (LSTAGE / (NW * 1024) - N64 - CPF) * 4 : 0;
@@ -573,13 +573,19 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
   if constexpr (DMA) {
     if (a.matter == MATTER_STATIC) Dpt = (TC)ldo((const TS*)a.DIFFD, idx);
   }
-  // dust fluid with the epilogue prefetch: its stage input, RK4 inputs and
-  // lagged state at the point, loaded after the staging and waited for
+  // dust fluid: its stage input at the point, with the point values
+  TS pdi[DUST ? NDUST : 1];
+  if constexpr (DUST) {
+#pragma unroll
+    for (int q = 0; q < NDUST; ++q) pdi[q] = ldo((const TS*)RD(q, a.s_in), idx);
+  }
+  // dust fluid with the epilogue prefetch: its RK4 inputs and lagged state
+  // at the point, loaded after the staging and waited for
   // before the prefetch is issued (vector memory operations retire in order:
   // waiting for them in the algebra would also wait for the prefetch)
   static_assert(!PFD || MQ, "the prefetching dust kernels hold the metric as fixed-point words");
   constexpr int ND = PFD ? NDUST : 1;
-  TS pdi[ND], pdp[ND], pd1[ND], pd2[ND], pdl[ND];
+  TS pdp[ND], pd1[ND], pd2[ND], pdl[ND];
   int plw[PFD ? 7 : 1];
   auto dust_preload = [&]() {
     if constexpr (PFD) {
@@ -587,7 +593,6 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
       const bool lag = a.lag_mode != 0;
 #pragma unroll
       for (int q = 0; q < NDUST; ++q) {
-        pdi[q] = ldo((const TS*)RD(q, a.s_in), idx);
         pdp[q] = rk ? ldo((const TS*)RD(q, a.s_p), idx) : TS(0);
         pd1[q] = f1 ? ldo((const TS*)RD(q, a.s_f), idx) : TS(0);
         pd2[q] = f2 ? ldo((const TS*)RD(q, a.s_a2), idx) : TS(0);
@@ -597,7 +602,7 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
       for (int q = 0; q < 6; ++q) plw[q] = lag ? ldo((const int*)RS(q, a.s_lag_met), idx) : 0;
       plw[6] = lag ? ldo((const int*)RS(PHI, a.s_lag), idx) : 0;
 #pragma unroll
-      for (int q = 0; q < NDUST; ++q) asm volatile("" ::"v"(pdi[q]), "v"(pdp[q]), "v"(pd1[q]), "v"(pd2[q]), "v"(pdl[q]));
+      for (int q = 0; q < NDUST; ++q) asm volatile("" ::"v"(pdp[q]), "v"(pd1[q]), "v"(pd2[q]), "v"(pdl[q]));
 #pragma unroll
       for (int q = 0; q < 7; ++q) asm volatile("" ::"v"(plw[q]));
     }
@@ -688,7 +693,32 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
   TC GL[3][6], G[3][6], Gd[3];
   TC Ac[6], AijAij = TC(0), second[3];  // A^ij, A_ij A^ij, Gamma^i_jk A^jk + 6 A^ij d_j phi
   TC DDa[6], DDaTR = TC(0);             // (D_i D_j alpha)^TF and its trace (without e^{-4 phi})
+  // dust fluid: D, S_j, the Lorentz factor W and the momentum force's
+  // v^i v^j (4 gamma_ij d_k phi + d_k gamma_ij), which reads d_k gamma_ij too
+  TC Dc = TC(0), Sc[3] = {TC(0), TC(0), TC(0)}, Wc = TC(1), force[3];
   auto curvature = [&]() {
+    if constexpr (DUST) {
+      // Dust::getDustData at the point (dust.cc:177-200)
+      const TC ph = (TC)(phi_c + fv.phi), em4 = exp(TC(-4) * ph), e6 = exp(TC(6) * ph);
+      Dc = (TC)pdi[0];
+  #pragma unroll
+      for (int j = 0; j < 3; ++j) Sc[j] = (TC)pdi[DUST ? 1 + j : 0];
+      const TC giSS = em4 * (gi[0] * Sc[0] * Sc[0] + gi[3] * Sc[1] * Sc[1] + gi[5] * Sc[2] * Sc[2] +
+                             TC(2) * (gi[1] * Sc[0] * Sc[1] + gi[2] * Sc[0] * Sc[2] + gi[4] * Sc[1] * Sc[2]));
+      Wc = sqrt(TC(1) + giSS / Dc / Dc);
+      TC vc[3];
+  #pragma unroll
+      for (int i = 0; i < 3; ++i) vc[i] = em4 / e6 * (GI(i, 0) * Sc[0] + GI(i, 1) * Sc[1] + GI(i, 2) * Sc[2]);
+      // dust.cc:139-150
+  #pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        const TC dp4 = TC(4) * dphi[k];
+        force[k] = vc[0] * vc[0] * (dp4 * GM(0, 0) + dg[k][0]) + vc[1] * vc[1] * (dp4 * GM(1, 1) + dg[k][3]) +
+                   vc[2] * vc[2] * (dp4 * GM(2, 2) + dg[k][5]) +
+                   TC(2) * (vc[0] * vc[1] * (dp4 * GM(0, 1) + dg[k][1]) + vc[0] * vc[2] * (dp4 * GM(0, 2) + dg[k][2]) +
+                            vc[1] * vc[2] * (dp4 * GM(1, 2) + dg[k][4]));
+      }
+    }
     // Christoffels (bssn_macros.h:221-229):  GL_ijk = 1/2(d_j g_ki + d_k g_ji - d_i g_jk),
     // G^i_jk = gamma^{im} GL_mjk
   #pragma unroll
@@ -1122,24 +1152,11 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
     // sources (components/static/static.cc:28-35, components/Lambda/lambda.cc:32-41)
     TC DIFFr = TC(0), DIFFS = TC(0);
     TC Si[3] = {TC(0), TC(0), TC(0)}, STF[6] = {TC(0), TC(0), TC(0), TC(0), TC(0), TC(0)};
-    TC Dc = TC(0), Sc[3] = {TC(0), TC(0), TC(0)}, Wc = TC(1), vc[3] = {TC(0), TC(0), TC(0)};
     if (a.matter == MATTER_STATIC) {
       const TC D = DMA ? Dpt : (TC)ldo((const TS*)a.DIFFD, idx);
       DIFFr = exp((TC)(-6.0 * (phi_c + fv.phi))) * D + rhoF * expm1(TC(-6) * v[PHI]);
     }
     if constexpr (DUST) {
-      // Dust::getDustData at the point (dust.cc:177-200)
-      Dc = PFD ? (TC)pdi[0] : (TC)ldo((const TS*)RD(0, a.s_in), idx);
-  #pragma unroll
-      for (int j = 0; j < 3; ++j) Sc[j] = PFD ? (TC)pdi[1 + j] : (TC)ldo((const TS*)RD(1 + j, a.s_in), idx);
-      {
-        const TC em4 = exp(TC(-4) * phi), e6 = exp(TC(6) * phi);
-        const TC giSS = em4 * (gi[0] * Sc[0] * Sc[0] + gi[3] * Sc[1] * Sc[1] + gi[5] * Sc[2] * Sc[2] +
-                               TC(2) * (gi[1] * Sc[0] * Sc[1] + gi[2] * Sc[0] * Sc[2] + gi[4] * Sc[1] * Sc[2]));
-        Wc = sqrt(TC(1) + giSS / Dc / Dc);
-  #pragma unroll
-        for (int i = 0; i < 3; ++i) vc[i] = em4 / e6 * (GI(i, 0) * Sc[0] + GI(i, 1) * Sc[1] + GI(i, 2) * Sc[2]);
-      }
       // Dust::addBSSNSrc (dust.cc:226-264): D, S_i of this stage with W,
       // detg, g_ij of the state the previous populateDerivedFields saw
       TC Wl = Wc, detg = exp(TC(6) * phi), e4l = exp(TC(4) * phi);
@@ -1209,14 +1226,7 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
       drhs[0] = ddust[0];
       const TC pre = TC(0.5) * alpha * Wc * Dc * exp(TC(4) * phi);
 #pragma unroll
-      for (int k = 0; k < 3; ++k) {
-        const TC dp4 = TC(4) * dphi[k];
-        const TC acc = vc[0] * vc[0] * (dp4 * GM(0, 0) + dg[k][0]) + vc[1] * vc[1] * (dp4 * GM(1, 1) + dg[k][3]) +
-                       vc[2] * vc[2] * (dp4 * GM(2, 2) + dg[k][5]) +
-                       TC(2) * (vc[0] * vc[1] * (dp4 * GM(0, 1) + dg[k][1]) + vc[0] * vc[2] * (dp4 * GM(0, 2) + dg[k][2]) +
-                                vc[1] * vc[2] * (dp4 * GM(1, 2) + dg[k][4]));
-        drhs[1 + k] = ddust[1 + k] + (pre * acc - Wc * Dc * dal[k]);
-      }
+      for (int k = 0; k < 3; ++k) drhs[1 + k] = ddust[1 + k] + (pre * force[k] - Wc * Dc * dal[k]);
 #pragma unroll
       for (int q = 0; q < NDUST; ++q) {
         const double cc = (double)drhs[q];
@@ -1235,7 +1245,7 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
           // accumulator-free form: K3Finalize's accumulator from the three stage outputs
           const double a1 = PFD ? (double)pd1[qq] : (double)ldo((const TS*)fr, idx);
           const double a2 = PFD ? (double)pd2[qq] : (double)ldo((const TS*)RD(q, a.s_a2), idx);
-          const double a3 = PFD ? (double)pdi[qq] : (double)ldo((const TS*)RD(q, a.s_in), idx);
+          const double a3 = (double)pdi[q];
           fo = ((a1 - p) + 2.0 * (a2 - p) + (a3 - p)) * (1.0 / 3.0);
         }
         const double inc = a.cf * cc;

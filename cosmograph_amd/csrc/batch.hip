@@ -97,20 +97,17 @@ static bool batch_norm_stage1(const cg_batch* b) {
   return false;
 }
 
+// as pick_variant, over the tiles of all grids
 static const StageVariant* batch_pick(const cg_batch* b) {
   const StageVariant* best = nullptr;
-  int best_score = -1;
+  double least = 0.0;
   for (const auto& v : stage_variants()) {
     if (!batch_fits(b, v)) continue;
-    int score = 0;
-    if (b->req_ti) {
-      if (v.ti != b->req_ti || v.tj != b->req_tj || v.tk != b->req_tk) continue;
-      score += 100;
-    } else if (v.ti == 4 && v.tj == 8 && v.tk == 8) {
-      score += 100;
-    }
-    score += (v.wpe == (b->prec == CG_FP64 ? 2 : 3)) ? 10 : (v.wpe == 1 ? 5 : 0);
-    if (score > best_score) { best = &v; best_score = score; }
+    if (b->req_ti && (v.ti != b->req_ti || v.tj != b->req_tj || v.tk != b->req_tk)) continue;
+    double pts = 0.0;
+    for (auto* c : b->m) pts += tiled_points(c, v);
+    const double t = pts * variant_weight(v, batch_dma_fits(b, v));
+    if (!best || t < least) { best = &v; least = t; }
   }
   return best;
 }

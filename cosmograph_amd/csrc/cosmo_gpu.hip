@@ -470,6 +470,36 @@ bool dma_fits(const cg_ctx* c, const StageVariant& v) {
   return c->p.nz % 4 == 0 && c->p.nz >= kh && c->p.nz > v.tk + kh - 2;
 }
 
+double tiled_points(const cg_ctx* c, const StageVariant& v) {
+  auto up = [](int n, int t) { return (double)((n + t - 1) / t * t); };
+  return up(c->p.nx, v.ti) * up(c->p.ny, v.tj) * up(c->p.nz, v.tk);
+}
+
+// Relative time per tiled point, measured with the autotuner on grids whose
+// extents are multiples of 16 (ms per stage):
+//   LDS-DMA: 4x4x16 is the fastest tile, or within 2% of it: rows of 64 or
+//     128 bytes along k, and the smallest halo of the 256-point tiles.  128^3
+//     FP64, order 4: 4x4x16 0.283, 2x8x16 0.278, 4x8x8 0.314; order 6: 0.329,
+//     0.336, 0.368.  256^3 fixed point, order 6: 1.51, 4x8x8 1.79.  96^3
+//     FP64, order 8: 0.217, 8x8x8 0.242.
+//   Register staging: FP64 order 4 0.372, 0.377, 4x8x8 0.386; order 6 0.453,
+//     0.464, 0.455; split order 6 (101x90x118) 0.208, 0.256, 0.217; order 8
+//     (LDS-bound occupancy): FP64 4x4x16 0.343, 4x8x8 0.360, 8x8x8 0.273,
+//     split 0.334, 0.210, 0.247.
+//   Halo 5 (KO at order 8), FP64, 96^3: 8x8x8 0.457 (DMA), 0.537 (register),
+//     4x8x8 0.650.
+double variant_weight(const StageVariant& v, bool dma) {
+  const bool f64 = v.prec == CG_FP64;
+  double w;
+  if (v.ti == 4 && v.tj == 4) w = 1.0;
+  else if (v.ti == 2) w = dma ? 1.02 : f64 ? 1.03 : 1.2;
+  else if (v.ti == 8) w = dma ? 1.15 : v.halo >= 4 && f64 ? 0.8 : 1.3;
+  else w = dma ? 1.15 : v.halo >= 4 && !f64 ? 0.7 : 1.04;
+  if (!dma) w *= 1.35;  // register staging against LDS-DMA: 1.31 to 1.65 in the figures above
+  // a register budget for one wave per SIMD only pays where nothing else fits
+  return v.wpe == 1 ? 1.02 * w : w;
+}
+
 // tile order 3 (Morton columns) needs power-of-two tile counts along i and j
 bool morton_fits(int ntx, int nty) { return ntx > 0 && nty > 0 && !(ntx & (ntx - 1)) && !(nty & (nty - 1)); }
 
@@ -491,22 +521,17 @@ static bool variant_matches(const cg_ctx* c, const StageVariant& v) {
          v.dust == (c->p.matter == CG_MATTER_DUST) && variant_fits(c, v);
 }
 
-// default: the requested tile, else the 4x8x8 tile with the register budget
-// of 3 (FP32) / 2 (FP64) waves per SIMD when compiled, else any fitting tile
+// The variant without an autotuner run: among those that fit (and have the
+// requested tile, if any), the one with the least estimated time of a stage,
+// the points of all its tiles (padding included) times variant_weight.
 static const StageVariant* pick_variant(const cg_ctx* c) {
   const StageVariant* best = nullptr;
-  int best_score = -1;
+  double least = 0.0;
   for (const auto& v : stage_variants()) {
     if (!variant_matches(c, v)) continue;
-    int score = 0;
-    if (c->req_ti) {
-      if (v.ti != c->req_ti || v.tj != c->req_tj || v.tk != c->req_tk) continue;
-      score += 100;
-    } else if (v.ti == 4 && v.tj == 8 && v.tk == 8) {
-      score += 100;
-    }
-    score += (v.wpe == (c->prec == CG_FP64 ? 2 : 3)) ? 10 : (v.wpe == 1 ? 5 : 0);
-    if (score > best_score) { best = &v; best_score = score; }
+    if (c->req_ti && (v.ti != c->req_ti || v.tj != c->req_tj || v.tk != c->req_tk)) continue;
+    const double t = tiled_points(c, v) * variant_weight(v, c->dma_allowed && c->dma_pick && dma_fits(c, v));
+    if (!best || t < least) { best = &v; least = t; }
   }
   return best;
 }

@@ -286,6 +286,40 @@ __global__ void k_dust_finalize(TS* __restrict__ dreg, long rstride, int rp, int
   }
 }
 
+// Uploads and downloads of FP32 fields: the caller's FP64 values and the
+// device's FP32 ones are converted here, through a device buffer of at most
+// kIoValues.  Bound by the host link: a 256^3 field moves 134 MB instead of
+// 67, but the conversion on the host (a 67 MB vector filled and read by one
+// thread) cost more than both: 256^3 into pinned memory 20.3 -> 2.5 ms, into
+// a new array 24.0 -> 13.0 ms, upload 18.7 -> 4.7 ms.
+constexpr long kIoValues = 4l << 20;  // 32 MB
+// Small pageable arrays stay with the host loop: the runtime's copy of twice
+// the bytes out of pageable memory costs more than converting them (48^3
+// download 0.066 ms against 0.045, 96^3 0.438 against 0.358, 128^3 equal);
+// pinned ones go through the device at every size (48^3 0.038 ms against 0.041).
+inline bool io_on_device(const void* host, size_t n) {
+  if (n >= (2u << 20)) return true;
+  hipPointerAttribute_t at{};
+  if (hipPointerGetAttributes(&at, host) != hipSuccess) {
+    (void)hipGetLastError();  // not an address the runtime knows: pageable
+    return false;
+  }
+  return at.type == hipMemoryTypeHost;
+}
+inline unsigned io_blocks(size_t n) { return (unsigned)((n + 1023) / 1024); }
+__global__ void __launch_bounds__(256) k_widen(const float* __restrict__ src, long n, double* __restrict__ dst) {
+  const long b = (long)blockIdx.x * 1024 + threadIdx.x;
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+    if (b + q * 256 < n) dst[b + q * 256] = (double)src[b + q * 256];
+}
+__global__ void __launch_bounds__(256) k_narrow(const double* __restrict__ src, long n, float* __restrict__ dst) {
+  const long b = (long)blockIdx.x * 1024 + threadIdx.x;
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+    if (b + q * 256 < n) dst[b + q * 256] = (float)src[b + q * 256];
+}
+
 // numNaNs (math.h:1524-1541): NaN test of the float-rounded value
 template <typename TS>
 __global__ void k_num_nans(const TS* __restrict__ f, long n, unsigned long long* count) {
@@ -599,14 +633,6 @@ int cg_create(const cg_params* params, cg_ctx** out) {
     HIPCHK(c, hipMalloc((void**)&c->met, (size_t)7 * 4 * pad * sizeof(double)));
     HIPCHK(c, hipMemsetAsync(c->met, 0, (size_t)7 * 4 * pad * sizeof(double), c->stream));
   }
-  HIPCHK(c, hipMalloc(&c->DIFFD, (size_t)pad * c->ts));
-  HIPCHK(c, hipMemsetAsync(c->DIFFD, 0, (size_t)pad * c->ts, c->stream));
-  HIPCHK(c, hipMalloc(&c->nan_dev, sizeof(unsigned)));
-  HIPCHK(c, hipMemsetAsync(c->nan_dev, 0, sizeof(unsigned), c->stream));
-  if (c->mq) {
-    HIPCHK(c, hipMalloc((void**)&c->mq_sat, sizeof(unsigned)));
-    HIPCHK(c, hipMemsetAsync(c->mq_sat, 0, sizeof(unsigned), c->stream));
-  }
   // partial rows: one per tile of any compiled stage variant, or one per
   // 256-point block of the elementwise kernels
   long rows = (c->npts + 255) / 256;
@@ -615,11 +641,30 @@ int cg_create(const cg_params* params, cg_ctx** out) {
     rows = nt > rows ? nt : rows;
   }
   c->ext_rows = rows;
-  HIPCHK(c, hipMalloc((void**)&c->ext_part, (size_t)rows * EXT_W * sizeof(double)));
-  HIPCHK(c, hipMalloc((void**)&c->ext_mid, (size_t)(kExtMid + 1) * EXT_W * sizeof(double)));
-  HIPCHK(c, hipMalloc((void**)&c->ext, 4 * sizeof(double)));
-  HIPCHK(c, hipMemsetAsync(c->ext, 0, 4 * sizeof(double), c->stream));
-  HIPCHK(c, hipMalloc((void**)&c->nan_cnt, sizeof(unsigned long long)));
+  if (c->ts == 4) c->io_n = (size_t)std::min(c->npts, kIoValues);
+  // the counters, scratch rows and staging of a context share one
+  // allocation: what starts as zero first, each part on a 256-byte boundary
+  size_t total = 0, zeroed = 0;
+  auto part = [&](size_t bytes) {
+    const size_t at = total;
+    total += (bytes + 255) / 256 * 256;
+    return at;
+  };
+  const size_t oD = part((size_t)pad * c->ts), oNan = part(sizeof(unsigned)), oSat = part(sizeof(unsigned)),
+               oExt = part(4 * sizeof(double)), oCnt = part(sizeof(unsigned long long));
+  zeroed = total;
+  const size_t oMid = part((size_t)(kExtMid + 1) * EXT_W * sizeof(double)),
+               oPart = part((size_t)rows * EXT_W * sizeof(double)), oIo = part(c->io_n * sizeof(double));
+  HIPCHK(c, hipMalloc((void**)&c->arena, total));
+  HIPCHK(c, hipMemsetAsync(c->arena, 0, zeroed, c->stream));
+  c->DIFFD = c->arena + oD;
+  c->nan_dev = (unsigned*)(c->arena + oNan);
+  if (c->mq) c->mq_sat = (unsigned*)(c->arena + oSat);
+  c->ext = (double*)(c->arena + oExt);
+  c->nan_cnt = (unsigned long long*)(c->arena + oCnt);
+  c->ext_mid = (double*)(c->arena + oMid);
+  c->ext_part = (double*)(c->arena + oPart);
+  if (c->io_n) c->io = (double*)(c->arena + oIo);
   c->nxf = n_xfields(p.shift);
   if (c->nxf) {
     HIPCHK(c, hipMalloc((void**)&c->xreg, (size_t)c->nxf * 4 * pad * sizeof(double)));
@@ -641,21 +686,15 @@ int cg_destroy(cg_ctx* c) {
   if (c->stream) (void)hipStreamSynchronize(c->stream);
   for (auto& e : c->ev) { (void)hipEventDestroy(e.first); (void)hipEventDestroy(e.second); }
   if (c->regs) (void)hipFree(c->regs);
-  if (c->DIFFD) (void)hipFree(c->DIFFD);
   if (c->met) (void)hipFree(c->met);
   if (c->cons) (void)hipFree(c->cons);
   if (c->cons_part) (void)hipFree(c->cons_part);
   if (c->obuf) (void)hipFree(c->obuf);
-  if (c->nan_dev) (void)hipFree(c->nan_dev);
-  if (c->ext) (void)hipFree(c->ext);
-  if (c->ext_part) (void)hipFree(c->ext_part);
-  if (c->ext_mid) (void)hipFree(c->ext_mid);
-  if (c->nan_cnt) (void)hipFree(c->nan_cnt);
   if (c->dreg) (void)hipFree(c->dreg);
   if (c->flux) (void)hipFree(c->flux);
   if (c->rho_src) (void)hipFree(c->rho_src);
   if (c->xreg) (void)hipFree(c->xreg);
-  if (c->mq_sat) (void)hipFree(c->mq_sat);
+  if (c->arena) (void)hipFree(c->arena);
   mq_free(c);
   bardeen_free(c);
   if (c->stream) (void)hipStreamDestroy(c->stream);
@@ -779,10 +818,19 @@ int cg_field_upload(cg_ctx* c, const char* name, const double* host, size_t n) {
   if (esz == 8) {
     HIPCHK(c, hipMemcpyAsync(d, host, n * 8, hipMemcpyHostToDevice, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
-  } else {
+  } else if (!io_on_device(host, n)) {
     std::vector<float> tmp(n);
     for (size_t x = 0; x < n; ++x) tmp[x] = (float)host[x];
     HIPCHK(c, hipMemcpyAsync(d, tmp.data(), n * 4, hipMemcpyHostToDevice, c->stream));
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+  } else {
+    for (size_t at = 0; at < n; at += c->io_n) {
+      const size_t m = n - at < c->io_n ? n - at : c->io_n;
+      HIPCHK(c, hipMemcpyAsync(c->io, host + at, m * 8, hipMemcpyHostToDevice, c->stream));
+      hipLaunchKernelGGL(k_narrow, dim3(io_blocks(m)), dim3(256), 0, c->stream, (const double*)c->io, (long)m,
+                         (float*)d + at);
+      HIPCHK(c, hipGetLastError());
+    }
     HIPCHK(c, hipStreamSynchronize(c->stream));
   }
   return CG_OK;
@@ -808,11 +856,19 @@ int cg_field_download(cg_ctx* c, const char* name, double* host, size_t n) {
   if (esz == 8) {
     HIPCHK(c, hipMemcpyAsync(host, d, n * 8, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
-  } else {
+  } else if (!io_on_device(host, n)) {
     std::vector<float> tmp(n);
     HIPCHK(c, hipMemcpyAsync(tmp.data(), d, n * 4, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     for (size_t x = 0; x < n; ++x) host[x] = (double)tmp[x];
+  } else {
+    for (size_t at = 0; at < n; at += c->io_n) {
+      const size_t m = n - at < c->io_n ? n - at : c->io_n;
+      hipLaunchKernelGGL(k_widen, dim3(io_blocks(m)), dim3(256), 0, c->stream, (const float*)d + at, (long)m, c->io);
+      HIPCHK(c, hipGetLastError());
+      HIPCHK(c, hipMemcpyAsync(host + at, c->io, m * 8, hipMemcpyDeviceToHost, c->stream));
+    }
+    HIPCHK(c, hipStreamSynchronize(c->stream));
   }
   return CG_OK;
 }

@@ -130,6 +130,9 @@ struct cg_ctx {
   bool mq = false;
   int mq_exp[7] = {-40, -40, -40, -40, -40, -40, -40};
   double* mq_tmp = nullptr;               // FP64 staging of one field (lazy)
+  double* io = nullptr;                   // FP64 staging of FP32 uploads and downloads, io_n values
+  size_t io_n = 0;
+  char* arena = nullptr;                  // holds DIFFD, nan_dev, mq_sat, ext, nan_cnt, ext_mid, ext_part, io
   unsigned* mq_part = nullptr;            // per-block maxima (lazy)
   unsigned* mq_sat = nullptr;             // count of saturated words written by the stage kernels
   double* cons = nullptr;                 // [CONS_N][pad] per-point constraint values (lazy)

@@ -27,7 +27,6 @@
 // evolution loop); FP32-split registers are widened into the workspace
 // first.  The workspace (about 60 FP64 arrays) is allocated on first use.
 #include <hip/hip_runtime.h>
-#include <hipfft/hipfft.h>
 
 #include <cmath>
 #include <cstring>
@@ -35,6 +34,7 @@
 #include <vector>
 
 #include "bssn_stage.h"
+#include "fftplan.h"
 #include "runtime.h"
 #include "stencil.h"
 
@@ -56,8 +56,8 @@ struct BrdWork {
   double* arr = nullptr;        // [W_N][pad]
   double2* spec = nullptr;      // [nx][ny][nz/2+1]
   double* part = nullptr;       // reduction partials
-  hipfftHandle r2c = 0, c2r = 0;
-  bool plans = false;
+  FftPlan r2c, c2r;             // held while the workspace is
+  bool ready = false;           // everything above allocated
   bool valid = false;           // potentials of the last call present
 };
 
@@ -400,12 +400,6 @@ double ml_d2adt2(double t, double OL) {
   return a * H * H - (1.0 - OL) * 3.0 / 2.0 / a / a;
 }
 
-#define FFTCHK(ctx, expr)                                                                          \
-  do {                                                                                             \
-    hipfftResult r_ = (expr);                                                                      \
-    if (r_ != HIPFFT_SUCCESS) return fail(ctx, CG_ERR_HIP, std::string(#expr) + " failed: " + std::to_string((int)r_)); \
-  } while (0)
-
 struct Red {
   cg_ctx* c;
   BrdWork* w;
@@ -457,12 +451,12 @@ int bardeen_t(cg_ctx* c, BrdWork* w, const BrdIn& in, double t, int use_ml, doub
   int rc = 0;
   const double box = c->p.nx * c->p.dx;  // H_LEN_FRAC
   auto invlap = [&](int q) -> int {
-    FFTCHK(c, hipfftExecD2Z(w->r2c, W + (long)q * pad, (hipfftDoubleComplex*)w->spec));
+    FFTCHK(c, w->r2c.d2z(W + (long)q * pad, w->spec));
     const long nm = (long)c->p.nx * c->p.ny * (c->p.nz / 2 + 1);
     hipLaunchKernelGGL(k_inv_lap_modes, dim3((unsigned)((nm + kBT - 1) / kBT)), blk, 0, c->stream, w->spec, c->p.nx,
                        c->p.ny, c->p.nz, box, (double)n);
     HIPCHK(c, hipGetLastError());
-    FFTCHK(c, hipfftExecZ2D(w->c2r, (hipfftDoubleComplex*)w->spec, W + (long)q * pad));
+    FFTCHK(c, w->c2r.z2d(w->spec, W + (long)q * pad));
     return CG_OK;
   };
 
@@ -588,10 +582,6 @@ const int kBrdIdx[] = {W_PHI, W_PSI, W_A, W_DTA, W_D2TA, W_B, W_DTB, W_D2TB, W_E
 void bardeen_free(cg_ctx* c) {
   BrdWork* w = c->brd;
   if (!w) return;
-  if (w->plans) {
-    (void)hipfftDestroy(w->r2c);
-    (void)hipfftDestroy(w->c2r);
-  }
   if (w->arr) (void)hipFree(w->arr);
   if (w->spec) (void)hipFree(w->spec);
   if (w->part) (void)hipFree(w->part);
@@ -633,20 +623,19 @@ int cg_bardeen(cg_ctx* c, double elapsed_t, int use_ml_scale_factor, double omeg
   const int rout = c->sC;
   if (int rc = rhs_at(c, rin, rout)) return rc;
   const long pad = c->rstride, n = c->npts;
+  if (c->brd && !c->brd->ready) bardeen_free(c);  // an earlier call ran out of memory on the way
   if (!c->brd) {
     BrdWork* w = new BrdWork();
     c->brd = w;
     HIPCHK(c, hipMalloc((void**)&w->arr, (size_t)W_N * pad * sizeof(double)));
     HIPCHK(c, hipMalloc((void**)&w->spec, (size_t)c->p.nx * c->p.ny * (c->p.nz / 2 + 1) * sizeof(double2)));
     HIPCHK(c, hipMalloc((void**)&w->part, kRedBlocks * sizeof(double)));
-    FFTCHK(c, hipfftPlan3d(&w->r2c, c->p.nx, c->p.ny, c->p.nz, HIPFFT_D2Z));
-    FFTCHK(c, hipfftPlan3d(&w->c2r, c->p.nx, c->p.ny, c->p.nz, HIPFFT_Z2D));
-    w->plans = true;
+    if (int rc = w->r2c.take(c, HIPFFT_D2Z, c->stream)) return rc;
+    if (int rc = w->c2r.take(c, HIPFFT_Z2D, c->stream)) return rc;
+    w->ready = true;
   }
   BrdWork* w = c->brd;
   w->valid = false;
-  FFTCHK(c, hipfftSetStream(w->r2c, c->stream));
-  FFTCHK(c, hipfftSetStream(w->c2r, c->stream));
   // inputs in FP64: the metric registers directly, the storage-type ones
   // widened into the workspace in split precision
   BrdIn in{};

@@ -27,7 +27,6 @@
 // Reductions are per-block partials in a fixed order, summed on the host in
 // block order: the result is deterministic.
 #include <hip/hip_runtime.h>
-#include <hipfft/hipfft.h>
 
 #include <algorithm>
 #include <cmath>
@@ -35,6 +34,7 @@
 #include <vector>
 
 #include "../../include/cosmo_gpu.h"
+#include "fftplan.h"
 #include "runtime.h"
 
 using namespace cg;
@@ -178,23 +178,14 @@ struct Scratch {
   double* work = nullptr;
   double2* spec = nullptr;
   double* part = nullptr;
-  hipfftHandle r2c = 0, c2r = 0;
-  bool have_r2c = false, have_c2r = false;
+  FftPlan r2c, c2r;
   ~Scratch() {
-    if (have_r2c) (void)hipfftDestroy(r2c);
-    if (have_c2r) (void)hipfftDestroy(c2r);
     for (void* p : {(void*)u, (void*)drho, (void*)work, (void*)spec, (void*)part})
       if (p) (void)hipFree(p);
   }
 };
 
 }  // namespace
-
-#define FFTCHK(ctx, expr)                                                                          \
-  do {                                                                                             \
-    hipfftResult r_ = (expr);                                                                      \
-    if (r_ != HIPFFT_SUCCESS) return fail(ctx, CG_ERR_HIP, std::string(#expr) + ": hipFFT error " + std::to_string((int)r_)); \
-  } while (0)
 
 int cg_ics_static_dust(cg_ctx* c, const double* modes, size_t n_modes, double rms, double tol, int max_iter,
                        double* shift, int* iters) {
@@ -212,12 +203,8 @@ int cg_ics_static_dust(cg_ctx* c, const double* modes, size_t n_modes, double rm
   HIPCHK(c, hipMalloc((void**)&w.work, n * sizeof(double)));
   HIPCHK(c, hipMalloc((void**)&w.spec, nspec * sizeof(double2)));
   HIPCHK(c, hipMalloc((void**)&w.part, 2 * kB * sizeof(double)));
-  FFTCHK(c, hipfftPlan3d(&w.r2c, nx, ny, nz, HIPFFT_D2Z));
-  w.have_r2c = true;
-  FFTCHK(c, hipfftPlan3d(&w.c2r, nx, ny, nz, HIPFFT_Z2D));
-  w.have_c2r = true;
-  FFTCHK(c, hipfftSetStream(w.r2c, s));
-  FFTCHK(c, hipfftSetStream(w.c2r, s));
+  if (int rc = w.r2c.take(c, HIPFFT_D2Z, s)) return rc;
+  if (int rc = w.c2r.take(c, HIPFFT_Z2D, s)) return rc;
   std::vector<double> part(2 * kB);
   auto sums = [&](double* s0, double* s1) -> int {
     HIPCHK(c, hipMemcpyAsync(part.data(), w.part, part.size() * sizeof(double), hipMemcpyDeviceToHost, s));
@@ -235,7 +222,7 @@ int cg_ics_static_dust(cg_ctx* c, const double* modes, size_t n_modes, double rm
   const int gh = (int)(((long)nx * ny + kT - 1) / kT);
   hipLaunchKernelGGL(k_hermitize, dim3(gh), dim3(kT), 0, s, w.spec, nx, ny, nzc, 0);
   if (nz / 2 != 0) hipLaunchKernelGGL(k_hermitize, dim3(gh), dim3(kT), 0, s, w.spec, nx, ny, nzc, nz / 2);
-  FFTCHK(c, hipfftExecZ2D(w.c2r, (hipfftDoubleComplex*)w.spec, w.drho));
+  FFTCHK(c, w.c2r.z2d(w.spec, w.drho));
   hipLaunchKernelGGL(k_sum, dim3(kB), dim3(kT), 0, s, w.drho, n, w.part);
   double tot = 0.0, sq = 0.0;
   if (int rc = sums(&tot, nullptr)) return rc;
@@ -257,9 +244,9 @@ int cg_ics_static_dust(cg_ctx* c, const double* modes, size_t n_modes, double rm
     if (int rc = sums(&s0, &s1)) return rc;
     cs = s0 / s1;
     hipLaunchKernelGGL(k_rhs, dim3(kB), dim3(kT), 0, s, w.u, w.drho, cs, n, w.work);
-    FFTCHK(c, hipfftExecD2Z(w.r2c, w.work, (hipfftDoubleComplex*)w.spec));
+    FFTCHK(c, w.r2c.d2z(w.work, w.spec));
     hipLaunchKernelGGL(k_green, dim3(gb), dim3(kT), 0, s, w.spec, nx, ny, nz, wx, wy, wz, 1.0 / (double)n);
-    FFTCHK(c, hipfftExecZ2D(w.c2r, (hipfftDoubleComplex*)w.spec, w.work));
+    FFTCHK(c, w.c2r.z2d(w.spec, w.work));
     hipLaunchKernelGGL(k_update, dim3(kB), dim3(kT), 0, s, w.u, w.work, n, w.part);
     HIPCHK(c, hipMemcpyAsync(part.data(), w.part, part.size() * sizeof(double), hipMemcpyDeviceToHost, s));
     HIPCHK(c, hipStreamSynchronize(s));
@@ -389,16 +376,14 @@ int cg_power_spectrum(cg_ctx* c, const char* name, double* out, int nbins) {
   HIPCHK(c, hipMalloc((void**)&w.work, n * sizeof(double)));
   HIPCHK(c, hipMalloc((void**)&w.spec, nspec * sizeof(double2)));
   HIPCHK(c, hipMalloc((void**)&w.part, (size_t)kBlocks * nbins * (sizeof(double) + sizeof(unsigned))));
-  FFTCHK(c, hipfftPlan3d(&w.r2c, nx, ny, nz, HIPFFT_D2Z));
-  w.have_r2c = true;
-  FFTCHK(c, hipfftSetStream(w.r2c, s));
+  if (int rc = w.r2c.take(c, HIPFFT_D2Z, s)) return rc;
   const int nb = (int)std::min<long>(4096, (n + 255) / 256);
   if (esz == 8)
     hipLaunchKernelGGL(k_to_double<double>, dim3(nb), dim3(256), 0, s, (const double*)d, n, w.work);
   else
     hipLaunchKernelGGL(k_to_double<float>, dim3(nb), dim3(256), 0, s, (const float*)d, n, w.work);
   HIPCHK(c, hipGetLastError());
-  FFTCHK(c, hipfftExecD2Z(w.r2c, w.work, (hipfftDoubleComplex*)w.spec));
+  FFTCHK(c, w.r2c.d2z(w.work, w.spec));
   double* pf = w.part;
   unsigned* pn = reinterpret_cast<unsigned*>(w.part + (size_t)kBlocks * nbins);
   const size_t shmem = (size_t)nbins * (sizeof(double) + sizeof(unsigned));

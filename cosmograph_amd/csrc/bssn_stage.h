@@ -143,6 +143,11 @@ struct StageArgs {
 // pass 1: 2q + {sum (val - mean)^2, sum (scaled - mean scaled)^2}
 constexpr int CONS_ROW_W = 30;
 constexpr int CONS_ROW_W1 = 10;
+// pass 2, one pass for everything: 8q + {the six of pass 0, the block's
+// sum (val - its mean)^2, sum (scaled - its mean)^2}, then the number of points
+constexpr int CONS_ROW_F = 41;
+// tile of the constraint kernel's LDS-DMA form
+constexpr int CONS_DMA_TI = 4, CONS_DMA_TJ = 4, CONS_DMA_TK = 16;
 // the 5 constraints' value, scale, scaled of one point
 constexpr int CONS_PT = 15;
 
@@ -170,7 +175,7 @@ struct BatchArgs {
 // bssn.cc:903-938) and the sources DIFFr, DIFFS of the evaluated state
 enum { CONS_H = 0, CONS_M = 3, CONS_G = 6, CONS_A = 9, CONS_S = 12, CONS_RICCI = 15, CONS_AIJAIJ = 16,
        CONS_MI = 17, CONS_RHO = 20, CONS_SRCS = 21, CONS_N = 22 };
-int launch_constraints(int prec, int order, bool live_alpha, bool dust, const StageArgs& a, hipStream_t s);
+int launch_constraints(int prec, int order, bool live_alpha, bool dust, bool dma, const StageArgs& a, hipStream_t s);
 
 // BSSN::setExtraFieldData (bssn.cc:165-170) partial sums, one row per
 // workgroup: sum w*DIFFK, sum w, sum w*DIFFphi, sum w*DIFFr, min DIFFK with
@@ -229,13 +234,12 @@ __device__ __forceinline__ double wave_max(double v) {
 // the grid.  Every thread of the block must call this: it holds barriers.
 __device__ __forceinline__ void block_cons_put(double* row, int pass, const double* means, bool on,
                                                const double cv[CONS_PT]) {
-  __shared__ double sh[16][CONS_ROW_W];
+  __shared__ double sh[16][CONS_ROW_W + 1], tot[CONS_ROW_W + 1];
   const int wv = threadIdx.x >> 6, nw = (int)(blockDim.x >> 6);
-  const int w = pass == 0 ? CONS_ROW_W : CONS_ROW_W1;
+  auto first = [&]() {  // sums and maxima (pass 0)
 #pragma unroll
-  for (int q = 0; q < 5; ++q) {
-    const double v = on ? cv[3 * q] : 0.0, sc = on ? cv[3 * q + 1] : 0.0, sd = on ? cv[3 * q + 2] : 0.0;
-    if (pass == 0) {
+    for (int q = 0; q < 5; ++q) {
+      const double v = on ? cv[3 * q] : 0.0, sc = on ? cv[3 * q + 1] : 0.0, sd = on ? cv[3 * q + 2] : 0.0;
       const double r0 = wave_sum(v), r1 = wave_sum(sc), r2 = wave_sum(sd), r3 = wave_sum(v * v);
       // the reference's `if (fabs(C) > max)` from 0: NaN never wins
       const double r4 = wave_max(on && fabs(v) > 0.0 ? fabs(v) : 0.0);
@@ -244,19 +248,46 @@ __device__ __forceinline__ void block_cons_put(double* row, int pass, const doub
         sh[wv][6 * q] = r0; sh[wv][6 * q + 1] = r1; sh[wv][6 * q + 2] = r2;
         sh[wv][6 * q + 3] = r3; sh[wv][6 * q + 4] = r4; sh[wv][6 * q + 5] = r5;
       }
-    } else {
-      const double d0 = on ? v - means[2 * q] : 0.0, d1 = on ? sd - means[2 * q + 1] : 0.0;
+    }
+  };
+  // squared deviations from m[2q], m[2q + 1]
+  auto second = [&](auto m) {
+#pragma unroll
+    for (int q = 0; q < 5; ++q) {
+      const double d0 = on ? cv[3 * q] - m(2 * q) : 0.0, d1 = on ? cv[3 * q + 2] - m(2 * q + 1) : 0.0;
       const double r0 = wave_sum(d0 * d0), r1 = wave_sum(d1 * d1);
       if ((threadIdx.x & 63) == 0) { sh[wv][2 * q] = r0; sh[wv][2 * q + 1] = r1; }
     }
-  }
-  __syncthreads();
-  if ((int)threadIdx.x < w) {
-    const int col = threadIdx.x;
-    const bool ismax = pass == 0 && (col % 6) >= 4;
+  };
+  auto column = [&](int col, bool ismax) {
     double acc = sh[0][col];
     for (int k = 1; k < nw; ++k) acc = ismax ? (sh[k][col] > acc ? sh[k][col] : acc) : acc + sh[k][col];
-    row[col] = acc;
+    return acc;
+  };
+  const int col = (int)threadIdx.x;
+  if (pass == 0) {
+    first();
+    __syncthreads();
+    if (col < CONS_ROW_W) row[col] = column(col, (col % 6) >= 4);
+  } else if (pass == 1) {
+    second([&](int q) { return means[q]; });
+    __syncthreads();
+    if (col < CONS_ROW_W1) row[col] = column(col, false);
+  } else {
+    first();
+    const unsigned long long on_mask = __ballot(on);
+    if ((threadIdx.x & 63) == 0) sh[wv][CONS_ROW_W] = (double)__popcll(on_mask);
+    __syncthreads();
+    if (col <= CONS_ROW_W) {
+      const double x = column(col, col < CONS_ROW_W && (col % 6) >= 4);
+      tot[col] = x;
+      row[col < CONS_ROW_W ? col / 6 * 8 + col % 6 : CONS_ROW_F - 1] = x;
+    }
+    __syncthreads();
+    const double rn = 1.0 / tot[CONS_ROW_W];
+    second([&](int q) { return tot[q / 2 * 6 + (q & 1) * 2] * rn; });
+    __syncthreads();
+    if (col < CONS_ROW_W1) row[col / 2 * 8 + 6 + (col & 1)] = column(col, false);
   }
 }
 

@@ -639,7 +639,10 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
 #pragma unroll
   for (int q = 0; q < (SEPG ? 6 : 1); ++q) ricG[q] = TC(0);
   TC dphi[3], ddphi[6], dal[3], ddal[6], dK[3];
-  TC dA[3][6];      // d_j A_kl, constraint mode only
+  // constraint mode: gamma^{mn} d_n A_mI and the rest of the momentum
+  // constraint's covariant derivative, its A_mI d_n phi term, and the trace
+  // that scales the Gamma^I constraint
+  TC mdiv[3] = {TC(0), TC(0), TC(0)}, mphi[3], gscale[3];
   TC ddust[NDUST];  // sum_i d_i of the dust fluxes
 #pragma unroll
   for (int q = 0; q < NDUST; ++q) ddust[q] = TC(0);
@@ -680,6 +683,12 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
 #pragma unroll
       for (int J = I; J < 3; ++J)
         (SEPG ? ricG[SEPG ? sy(I, J) : 0] : ric[sy(I, J)]) += I == J ? GM(k, I) * d[I] : TC(0.5) * (GM(k, I) * d[J] + GM(k, J) * d[I]);
+  };
+  // d_n of A_ab (component q) into the momentum constraint's divergence
+  auto add_dA = [&](int q, TC d0, TC d1, TC d2) {
+    const int sa = q < 3 ? 0 : q < 5 ? 1 : 2, sb = q == 0 ? 0 : q == 1 || q == 3 ? 1 : 2;
+    mdiv[sb] += GI(sa, 0) * d0 + GI(sa, 1) * d1 + GI(sa, 2) * d2;
+    if (sa != sb) mdiv[sa] += GI(sb, 0) * d0 + GI(sb, 1) * d1 + GI(sb, 2) * d2;
   };
   // Everything that needs the first derivatives of the metric, formed as soon
   // as the last of DIFFgamma_ij, DIFFphi (and DIFFalpha) is differentiated:
@@ -827,6 +836,23 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
       second[I] = G[I][0] * Ac[0] + G[I][3] * Ac[3] + G[I][5] * Ac[5] +
                   TC(2) * (G[I][1] * Ac[1] + G[I][2] * Ac[2] + G[I][4] * Ac[4]) +
                   TC(6) * (Ac[sy(I, 0)] * dphi[0] + Ac[sy(I, 1)] * dphi[1] + Ac[sy(I, 2)] * dphi[2]);
+    if constexpr (CONS) {
+  #pragma unroll
+      for (int I = 0; I < 3; ++I) {
+        mphi[I] = TC(0);
+  #pragma unroll
+        for (int n = 0; n < 3; ++n)
+  #pragma unroll
+          for (int m = 0; m < 3; ++m) {
+            mphi[I] += GI(m, n) * AM(m, I) * dphi[n];
+            mdiv[I] -= GL[m][sy(n, I)] * Ac[sy(m, n)];
+          }
+  #pragma unroll
+        for (int m = 0; m < 3; ++m) mdiv[I] -= Gd[m] * AM(m, I);
+        gscale[I] = gi[0] * G[I][0] - gi[3] * G[I][3] - gi[5] * G[I][5] -
+                    TC(2) * (gi[1] * G[I][1] + gi[2] * G[I][2] + gi[4] * G[I][4]);
+      }
+    }
   };
 
   // derivatives of field f, staged in the LDS tile BUF, at this thread's
@@ -896,7 +922,7 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
         add_dG(f - GAM1, fd1<R>(L, c4, SI4) * idx1, fd1<R>(L, c4, SJ4) * idx1, fd1<R>(L, c4, SK) * idx1);                \
       } else if (CONS && f >= A11 && f <= A33) {                                                                         \
         const int q = f - A11;                                                                                           \
-        dA[0][q] = fd1<R>(L, c4, SI4) * idx1; dA[1][q] = fd1<R>(L, c4, SJ4) * idx1; dA[2][q] = fd1<R>(L, c4, SK) * idx1; \
+        add_dA(q, fd1<R>(L, c4, SI4) * idx1, fd1<R>(L, c4, SJ4) * idx1, fd1<R>(L, c4, SK) * idx1);                       \
       } else if (KGRP && f >= KG0) {                                                                                     \
         /* two first-derivative fields in three parts each; the same points as the full tile */                         \
         const int cx = ((li + H) * TJ + lj) * TK + lk, cy = FGX + (li * HJ + lj + H) * TK + lk;                          \
@@ -1283,7 +1309,9 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
       const long cs = a.cons_stride;
       auto put = [&](int q, double val) {
         if (q < CONS_PT) cv[q] = val;
-        if (!a.cons_rows) co[(long)q * cs + idx] = val;
+        // with rows, only the arrays cg_field_download reads
+        if (!a.cons_rows || (co && (q == CONS_RICCI || q == CONS_AIJAIJ || q == CONS_RHO || q == CONS_SRCS)))
+          co[(long)q * cs + idx] = val;
       };
       const double rr = (double)DIFFr + fv.rho;
       const double e5 = exp(5.0 * (double)phi), e6 = exp(6.0 * (double)phi);
@@ -1295,20 +1323,7 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
       double M2 = 0, Ms2 = 0;
   #pragma unroll
       for (int I = 0; I < 3; ++I) {
-        double t6 = 0, td = 0;
-  #pragma unroll
-        for (int n = 0; n < 3; ++n)
-  #pragma unroll
-          for (int m = 0; m < 3; ++m) {
-            t6 += GI(m, n) * AM(m, I) * dphi[n];
-            td += GI(m, n) * dA[n][sy(m, I)];
-          }
-  #pragma unroll
-        for (int m = 0; m < 3; ++m) td -= Gd[m] * AM(m, I);
-  #pragma unroll
-        for (int n = 0; n < 3; ++n)
-  #pragma unroll
-          for (int m = 0; m < 3; ++m) td -= GL[m][sy(n, I)] * Ac[sy(m, n)];
+        const double t6 = mphi[I], td = mdiv[I];
         const double PI8S = 8.0 * 3.14159265358979323846 * (double)Si[I];
         const double MI = e6 * (-2.0 / 3.0 * dK[I] - PI8S + 6.0 * t6 + td);
         const double MS = e6 * (fabs(2.0 / 3.0 * dK[I]) + fabs(PI8S) + 6.0 * fabs(t6) + fabs(td));
@@ -1322,12 +1337,8 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
       double G2 = 0, Gs2 = 0;
   #pragma unroll
       for (int I = 0; I < 3; ++I) {
-        const double tr = gi[0] * G[I][0] + gi[3] * G[I][3] + gi[5] * G[I][5] +
-                          2.0 * (gi[1] * G[I][1] + gi[2] * G[I][2] + gi[4] * G[I][4]);
-        const double gc_ = v[GAM1 + I] - tr;
-        const double gs_ = fabs((double)v[GAM1 + I]) +
-                           fabs(gi[0] * G[I][0] - gi[3] * G[I][3] - gi[5] * G[I][5] -
-                                2.0 * (gi[1] * G[I][1] + gi[2] * G[I][2] + gi[4] * G[I][4]));
+        const double gc_ = v[GAM1 + I] - Gd[I];
+        const double gs_ = fabs((double)v[GAM1 + I]) + fabs((double)gscale[I]);
         G2 += gc_ * gc_;
         Gs2 += gs_ * gs_;
       }
@@ -1598,7 +1609,8 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
   }  // valid
   if constexpr (CONS) {
     if (a.cons_rows)
-      block_cons_put(a.cons_rows + (long)(t - a.tile_base) * CONS_ROW_W, a.cons_pass, a.cons_means, valid, cv);
+      block_cons_put(a.cons_rows + (long)(t - a.tile_base) * (a.cons_pass == 2 ? CONS_ROW_F : CONS_ROW_W), a.cons_pass,
+                     a.cons_means, valid, cv);
     return;
   }
 
@@ -1688,9 +1700,20 @@ int stage_info_t(int* vgprs, int* spills, int* lds) {
   return 0;
 }
 
+// The constraint kernel (FP64 algebra from any storage).  FP64 storage has an
+// LDS-DMA form on the 4x4x16 tile, for the grids the stage kernels use it on;
+// 4x8x8 with register staging otherwise.  Bound by the FP64 algebra at 2 waves
+// per SIMD (256 VGPRs).
 template <typename TS, int R, bool LA, int MODE = MODE_CONS>
-int cons_launch_t(const StageArgs& a, hipStream_t s) {
-  hipLaunchKernelGGL((stage_kernel<TS, double, R, R, 4, 8, 8, 1, LA, MODE>), dim3(8 * a.per_xcd), dim3(256), 0, s, a);
+int cons_launch_t(const StageArgs& a, bool dma, hipStream_t s) {
+  if constexpr (sizeof(TS) == 8) {
+    if (dma) {
+      hipLaunchKernelGGL((stage_kernel<TS, double, R, R, CONS_DMA_TI, CONS_DMA_TJ, CONS_DMA_TK, 2, LA, MODE, true>),
+                         dim3(8 * a.per_xcd), dim3(CONS_DMA_TI * CONS_DMA_TJ * CONS_DMA_TK), 0, s, a);
+      return (int)hipGetLastError();
+    }
+  }
+  hipLaunchKernelGGL((stage_kernel<TS, double, R, R, 4, 8, 8, 2, LA, MODE>), dim3(8 * a.per_xcd), dim3(256), 0, s, a);
   return (int)hipGetLastError();
 }
 

@@ -67,6 +67,28 @@ __device__ __forceinline__ void st(const RegTable& t, int f, int s, long x, doub
   }
 }
 
+// det(gamma) = 1 and A_ij trace free at one point
+__device__ __forceinline__ void normalise(double v[NF]) {
+  // BSSN::set_DIFFgamma_Aij_norm (bssn.cc:61-119)
+  double g11 = v[G11], g12 = v[G12], g13 = v[G13], g22 = v[G22], g23 = v[G23], g33 = v[G33];
+  double omd = -1.0 * (g11 + g22 + g33 - g12 * g12 - g13 * g13 - g23 * g23 + g11 * g22 + g11 * g33 + g22 * g33 -
+                       g23 * g23 * g11 - g13 * g13 * g22 - g12 * g12 * g33 + 2.0 * g12 * g13 * g23 + g11 * g22 * g33);
+  double tn = -1.0 * expm1(log1p(-1.0 * omd) / 3.0);
+  g11 = (g11 + tn) / (1.0 - tn); g22 = (g22 + tn) / (1.0 - tn); g33 = (g33 + tn) / (1.0 - tn);
+  g12 = g12 / (1.0 - tn); g13 = g13 / (1.0 - tn); g23 = g23 / (1.0 - tn);
+  v[G11] = g11; v[G12] = g12; v[G13] = g13; v[G22] = g22; v[G23] = g23; v[G33] = g33;
+  double i11 = 1.0 + g22 + g33 - g23 * g23 + g22 * g33, i22 = 1.0 + g11 + g33 - g13 * g13 + g11 * g33;
+  double i33 = 1.0 + g11 + g22 - g12 * g12 + g11 * g22, i12 = g13 * g23 - g12 * (1.0 + g33);
+  double i13 = g12 * g23 - g13 * (1.0 + g22), i23 = g12 * g13 - g23 * (1.0 + g11);
+  double trA = i11 * v[A11] + i22 * v[A22] + i33 * v[A33] + 2.0 * (i12 * v[A12] + i13 * v[A13] + i23 * v[A23]);
+  v[A11] = (v[A11] - 1.0 / 3.0 * (1.0 + g11) * trA) / (1.0 - tn);
+  v[A22] = (v[A22] - 1.0 / 3.0 * (1.0 + g22) * trA) / (1.0 - tn);
+  v[A33] = (v[A33] - 1.0 / 3.0 * (1.0 + g33) * trA) / (1.0 - tn);
+  v[A12] = (v[A12] - 1.0 / 3.0 * g12 * trA) / (1.0 - tn);
+  v[A13] = (v[A13] - 1.0 / 3.0 * g13 * trA) / (1.0 - tn);
+  v[A23] = (v[A23] - 1.0 / 3.0 * g23 * trA) / (1.0 - tn);
+}
+
 // Elementwise kernels run 256 threads per block; threads past the end keep
 // going with point 0 and store nothing, so whole blocks reach the
 // setExtraFieldData reduction (one partial row per block, see bssn_stage.h).
@@ -80,35 +102,36 @@ __global__ void k_step_init(RegTable t, int rp, int ra, int rf, long n, int norm
   double v[NF];
   for (int f = 0; f < NF; ++f) {
     v[f] = ld<TS, MT>(t, f, rp, x);
-    if (valid) st<TS, MT>(t, f, rf, x, 0.0);
+    if (valid && rf >= 0) st<TS, MT>(t, f, rf, x, 0.0);  // rf < 0: nothing reads _f after this call
   }
   // BSSN::stepInit calls setExtraFieldData before the normalisation, which
   // leaves DIFFphi and DIFFK alone (bssn.cc:219-226); DIFFr is not touched
   if (ext_part) block_ext_put(ext_part, blockIdx.x, valid, v[PHI], v[KK], 0.0, phiF);
   if (!valid) return;
-  if (normalize) {
-    // BSSN::set_DIFFgamma_Aij_norm (bssn.cc:61-119)
-    double g11 = v[G11], g12 = v[G12], g13 = v[G13], g22 = v[G22], g23 = v[G23], g33 = v[G33];
-    double omd = -1.0 * (g11 + g22 + g33 - g12 * g12 - g13 * g13 - g23 * g23 + g11 * g22 + g11 * g33 + g22 * g33 -
-                         g23 * g23 * g11 - g13 * g13 * g22 - g12 * g12 * g33 + 2.0 * g12 * g13 * g23 + g11 * g22 * g33);
-    double tn = -1.0 * expm1(log1p(-1.0 * omd) / 3.0);
-    g11 = (g11 + tn) / (1.0 - tn); g22 = (g22 + tn) / (1.0 - tn); g33 = (g33 + tn) / (1.0 - tn);
-    g12 = g12 / (1.0 - tn); g13 = g13 / (1.0 - tn); g23 = g23 / (1.0 - tn);
-    v[G11] = g11; v[G12] = g12; v[G13] = g13; v[G22] = g22; v[G23] = g23; v[G33] = g33;
-    double i11 = 1.0 + g22 + g33 - g23 * g23 + g22 * g33, i22 = 1.0 + g11 + g33 - g13 * g13 + g11 * g33;
-    double i33 = 1.0 + g11 + g22 - g12 * g12 + g11 * g22, i12 = g13 * g23 - g12 * (1.0 + g33);
-    double i13 = g12 * g23 - g13 * (1.0 + g22), i23 = g12 * g13 - g23 * (1.0 + g11);
-    double trA = i11 * v[A11] + i22 * v[A22] + i33 * v[A33] + 2.0 * (i12 * v[A12] + i13 * v[A13] + i23 * v[A23]);
-    v[A11] = (v[A11] - 1.0 / 3.0 * (1.0 + g11) * trA) / (1.0 - tn);
-    v[A22] = (v[A22] - 1.0 / 3.0 * (1.0 + g22) * trA) / (1.0 - tn);
-    v[A33] = (v[A33] - 1.0 / 3.0 * (1.0 + g33) * trA) / (1.0 - tn);
-    v[A12] = (v[A12] - 1.0 / 3.0 * g12 * trA) / (1.0 - tn);
-    v[A13] = (v[A13] - 1.0 / 3.0 * g13 * trA) / (1.0 - tn);
-    v[A23] = (v[A23] - 1.0 / 3.0 * g23 * trA) / (1.0 - tn);
-  }
+  if (normalize) normalise(v);
   for (int f = 0; f < NF; ++f) st<TS, MT>(t, f, ra, x, v[f]);
 }
 
+
+// the normalised DIFFgamma_ij and A_ij of register rp into register rn, the
+// only fields that differ from rp after stepInit
+template <typename TS, typename MT>
+__global__ void k_norm_copy(RegTable t, int rp, int rn, long n) {
+  const long x = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (x >= n) return;
+  double v[NF];
+#pragma unroll
+  for (int q = 0; q < 6; ++q) {
+    v[G11 + q] = ld<TS, MT>(t, G11 + q, rp, x);
+    v[A11 + q] = ld<TS, MT>(t, A11 + q, rp, x);
+  }
+  normalise(v);
+#pragma unroll
+  for (int q = 0; q < 6; ++q) {
+    st<TS, MT>(t, G11 + q, rn, x, v[G11 + q]);
+    st<TS, MT>(t, A11 + q, rn, x, v[A11 + q]);
+  }
+}
 
 template <typename TS>
 __device__ __forceinline__ double diff_r(const SrcArgs& s, double dphi, long x) {
@@ -339,74 +362,41 @@ constexpr int kStats = 6;  // sum val, sum scale, sum scaled, sum val^2, max|val
 
 __device__ __forceinline__ double red_max(double a, double b) { return b > a ? b : a; }
 
-__global__ void k_cons_partial(const double* __restrict__ cons, long stride, long n, double* __restrict__ part) {
-  __shared__ double sh[kRedThreads];
+// Rows of the constraint kernel's one-pass mode (CONS_ROW_F columns per
+// workgroup) into one row: column c of the output is the sum, or for 8q + 4,
+// 8q + 5 the max, over the rows.  pass 1 combines only 8q + 6, 8q + 7: the
+// workgroups' squared deviations move to the mean of all points, tot holding
+// pass 0's totals:  sum (x - m)^2 = sum_b [ sum (x - m_b)^2 + n_b (m_b - m)^2 ].
+// Thread (lane, r) of a block takes column lane of rows lo + r, lo + r + 16,
+// ...; a fixed order, so the result is deterministic.
+constexpr int kFinThreads = 1024, kFinBlocks = 128;
+__global__ void __launch_bounds__(kFinThreads) k_cons_fin(const double* __restrict__ rows, long n, int pass,
+                                                          const double* __restrict__ tot, double* __restrict__ out) {
+  __shared__ double sh[kFinThreads / 64][64];
+  const int col = threadIdx.x & 63, r = threadIdx.x >> 6;
   const long per = (n + gridDim.x - 1) / gridDim.x;
   const long lo = (long)blockIdx.x * per, hi = lo + per < n ? lo + per : n;
-  for (int c = 0; c < 5; ++c) {
-    const double* val = cons + (long)(3 * c) * stride;
-    const double* sca = val + stride;
-    const double* scd = val + 2 * stride;
-    double acc[kStats] = {0, 0, 0, 0, 0, 0};
-    for (long x = lo + threadIdx.x; x < hi; x += kRedThreads) {
-      const double v = val[x], sc = sca[x], sd = scd[x];
-      acc[0] += v; acc[1] += sc; acc[2] += sd; acc[3] += v * v;
-      acc[4] = red_max(acc[4], fabs(v)); acc[5] = red_max(acc[5], fabs(sd));
-    }
-    for (int q = 0; q < kStats; ++q) {
-      sh[threadIdx.x] = acc[q];
-      __syncthreads();
-      for (int w = kRedThreads / 2; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w)
-          sh[threadIdx.x] = q < 4 ? sh[threadIdx.x] + sh[threadIdx.x + w] : red_max(sh[threadIdx.x], sh[threadIdx.x + w]);
-        __syncthreads();
+  const int c8 = col & 7;
+  const bool dev = col < CONS_ROW_F - 1 && c8 >= 6, ismax = col < CONS_ROW_F - 1 && (c8 == 4 || c8 == 5);
+  // the column of the sum a deviation column belongs to: 6 -> value, 7 -> scaled
+  const int src = dev ? col - c8 + (c8 == 6 ? 0 : 2) : 0;
+  const double mean = dev && pass == 1 && tot ? tot[src] / tot[CONS_ROW_F - 1] : 0.0;
+  double acc = 0.0;
+  if (col < CONS_ROW_F && (pass == 1) == dev)
+    for (long x = lo + r; x < hi; x += kFinThreads / 64) {
+      const double* row = rows + x * CONS_ROW_F;
+      double v = row[col];
+      if (dev && tot) {
+        const double nb = row[CONS_ROW_F - 1], d = row[src] / nb - mean;
+        v += nb * (d * d);
       }
-      if (threadIdx.x == 0) part[((long)blockIdx.x * 5 + c) * kStats + q] = sh[0];
-      __syncthreads();
-    }
-  }
-}
-
-// second pass: sum (val - mean)^2 and (scaled - mean_scaled)^2
-__global__ void k_cons_var(const double* __restrict__ cons, long stride, long n, const double* __restrict__ means,
-                           double* __restrict__ part) {
-  __shared__ double sh[kRedThreads];
-  const long per = (n + gridDim.x - 1) / gridDim.x;
-  const long lo = (long)blockIdx.x * per, hi = lo + per < n ? lo + per : n;
-  for (int c = 0; c < 5; ++c) {
-    const double* val = cons + (long)(3 * c) * stride;
-    const double* scd = val + 2 * stride;
-    const double m0 = means[2 * c], m1 = means[2 * c + 1];
-    double a0 = 0, a1 = 0;
-    for (long x = lo + threadIdx.x; x < hi; x += kRedThreads) {
-      const double d0 = val[x] - m0, d1 = scd[x] - m1;
-      a0 += d0 * d0;
-      a1 += d1 * d1;
-    }
-    for (int q = 0; q < 2; ++q) {
-      sh[threadIdx.x] = q ? a1 : a0;
-      __syncthreads();
-      for (int w = kRedThreads / 2; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) sh[threadIdx.x] += sh[threadIdx.x + w];
-        __syncthreads();
-      }
-      if (threadIdx.x == 0) part[((long)blockIdx.x * 5 + c) * 2 + q] = sh[0];
-      __syncthreads();
-    }
-  }
-}
-
-// one block: combine nb partial rows of width w in block order; columns whose
-// index mod kStats is set in maxmask take the max, the others the sum
-__global__ void k_combine(const double* __restrict__ part, int nb, int w, unsigned maxmask, double* __restrict__ out) {
-  for (int col = threadIdx.x; col < w; col += blockDim.x) {
-    const bool ismax = (maxmask >> (col % kStats)) & 1u;
-    double acc = 0.0;
-    for (int b = 0; b < nb; ++b) {
-      const double v = part[(long)b * w + col];
       acc = ismax ? red_max(acc, v) : acc + v;
     }
-    out[col] = acc;
+  sh[r][col] = acc;
+  __syncthreads();
+  if (r == 0 && col < CONS_ROW_F && (pass == 1) == dev) {
+    for (int k = 1; k < kFinThreads / 64; ++k) acc = ismax ? red_max(acc, sh[k][col]) : acc + sh[k][col];
+    out[(long)blockIdx.x * CONS_ROW_F + col] = acc;
   }
 }
 
@@ -1417,36 +1407,34 @@ int cg_kernel_info(const cg_ctx* cc, int* vgprs, int* scratch, int* lds, int* ti
   return rc ? CG_ERR_HIP : CG_OK;
 }
 
-// the per-point constraint pass (prepBSSNOutput's set_bd_values on every
-// point, sims/sim.cc:214-231, with the constraint values of
-// setConstraintCalcs) into c->cons
-// The register the constraint pass reads: _a as the reference's output step
+// the constraint passes' own bounds on the grid (their 4x8x8 tile)
+static int cons_fits(cg_ctx* c) {
+  if (c->p.nx <= 4 + c->R - 2 || c->p.ny <= 8 + c->R - 2 || c->p.nz <= 8 + c->R - 2)
+    return fail(c, CG_ERR_ARG, "grid too small for the constraint kernel tile");
+  return CG_OK;
+}
+static int spare_slot(const cg_ctx* c) { return c->sC == 3 ? 2 : 3; }  // of the two stage registers
+
+// The register the SVT pass reads: _a as the reference's output step
 // sees it, after stepInit, i.e. the normalised _p when the last call was a
-// fused step.  The momentum constraint differentiates A_ij, so the
-// normalised register is materialised (into the spare stage register and the
-// dead _f) rather than normalised on the fly.  Allocates nothing.
+// fused step, materialised into the spare stage register.  Allocates nothing.
 int cg::cons_input(cg_ctx* c, int* rin_out) {
   // the pending K4Finalize averages read the dust source this pass rewrites
   if (int rc = ext_resolve(c)) return rc;
-  if (c->p.nx <= 4 + c->R - 2 || c->p.ny <= 8 + c->R - 2 || c->p.nz <= 8 + c->R - 2)
-    return fail(c, CG_ERR_ARG, "grid too small for the constraint kernel tile");
+  if (int rc = cons_fits(c)) return rc;
   int rin = c->sA;
   if (c->a_is_p) {
-    rin = (c->sC == 3) ? 2 : 3;  // the spare of the two stage registers
+    rin = spare_slot(c);
     const int bs = 256;
     const long nbk = (c->npts + bs - 1) / bs;
-    if (c->prec == CG_FP64)
-      hipLaunchKernelGGL((k_step_init<double, double>), dim3(nbk), dim3(bs), 0, c->stream, reg_table(c), c->sP, rin,
-                         c->sF, c->npts, c->p.normalize_metric, (double*)nullptr, 0.0);
-    else if (c->mq)
-      hipLaunchKernelGGL((k_step_init<float, int>), dim3(nbk), dim3(bs), 0, c->stream, reg_table(c), c->sP, rin,
-                         c->sF, c->npts, c->p.normalize_metric, (double*)nullptr, 0.0);
-    else if (c->met32)
-      hipLaunchKernelGGL((k_step_init<float, float>), dim3(nbk), dim3(bs), 0, c->stream, reg_table(c), c->sP, rin,
-                         c->sF, c->npts, c->p.normalize_metric, (double*)nullptr, 0.0);
-    else
-      hipLaunchKernelGGL((k_step_init<float, double>), dim3(nbk), dim3(bs), 0, c->stream, reg_table(c), c->sP, rin,
-                         c->sF, c->npts, c->p.normalize_metric, (double*)nullptr, 0.0);
+    auto init = [&](auto ts, auto mt) {
+      hipLaunchKernelGGL((k_step_init<decltype(ts), decltype(mt)>), dim3(nbk), dim3(bs), 0, c->stream, reg_table(c),
+                         c->sP, rin, -1, c->npts, c->p.normalize_metric, (double*)nullptr, 0.0);
+    };
+    if (c->prec == CG_FP64) init(double(), double());
+    else if (c->mq) init(float(), int());
+    else if (c->met32) init(float(), float());
+    else init(float(), double());
     HIPCHK(c, hipGetLastError());
     if (c->dreg && dust_reg_init(c, c->sP, rin, c->sF)) return CG_ERR_HIP;
   }
@@ -1454,33 +1442,86 @@ int cg::cons_input(cg_ctx* c, int* rin_out) {
   return CG_OK;
 }
 
-// arguments of a constraint pass over register rin with the 4x8x8 tile of
-// the constraint kernel; dust: sources from this state itself
-// (initDustStep's populate, sims/dust.cc:53-63)
-static StageArgs cons_args(cg_ctx* c, int rin) {
-  StageArgs a = make_args(c, 0, rin, c->sP, c->sF, c->sC, 0);
-  a.ntx = (c->p.nx + 3) / 4;
-  a.nty = (c->p.ny + 7) / 8;
-  a.ntz = (c->p.nz + 7) / 8;
+// Arguments of a constraint pass over the state the reference's output step
+// sees (_a after stepInit).  The momentum constraint differentiates A_ij, so
+// after a fused step the normalised DIFFgamma_ij and A_ij are materialised in
+// the spare stage register and read from there, the other fields from _p.
+// Dust: sources from this state itself (initDustStep's populate,
+// sims/dust.cc:53-63).
+static int cons_args(cg_ctx* c, StageArgs* out, bool* dma) {
+  if (int rc = ext_resolve(c)) return rc;
+  if (int rc = cons_fits(c)) return rc;
+  StageArgs a = make_args(c, 0, c->a_is_p ? c->sP : c->sA, c->sP, c->sF, c->sC, 0);
+  if (c->a_is_p && c->p.normalize_metric) {
+    a.s_in_norm = spare_slot(c);
+    const int bs = 256;
+    const long nbk = (c->npts + bs - 1) / bs;
+    auto copy = [&](auto ts, auto mt) {
+      hipLaunchKernelGGL((k_norm_copy<decltype(ts), decltype(mt)>), dim3(nbk), dim3(bs), 0, c->stream, reg_table(c),
+                         c->sP, a.s_in_norm, c->npts);
+    };
+    if (c->prec == CG_FP64) copy(double(), double());
+    else if (c->mq) copy(float(), int());
+    else if (c->met32) copy(float(), float());
+    else copy(float(), double());
+    HIPCHK(c, hipGetLastError());
+  }
+  // the DMA form's conditions are those of the stage kernels (dma_fits)
+  StageVariant v{};
+  v.prec = c->prec;
+  v.halo = c->R;
+  v.tk = CONS_DMA_TK;
+  v.launch_dma = [](const StageArgs&, hipStream_t) { return 0; };
+  *dma = c->prec == CG_FP64 && c->dma_allowed && dma_fits(c, v) && c->p.nx > CONS_DMA_TI + c->R - 2 &&
+         c->p.ny > CONS_DMA_TJ + c->R - 2;
+  const int ti = *dma ? CONS_DMA_TI : 4, tj = *dma ? CONS_DMA_TJ : 8, tk = *dma ? CONS_DMA_TK : 8;
+  a.ntx = (c->p.nx + ti - 1) / ti;
+  a.nty = (c->p.ny + tj - 1) / tj;
+  a.ntz = (c->p.nz + tk - 1) / tk;
+  if (a.tile_order == 3 && !morton_fits(a.ntx, a.nty)) a.tile_order = 0;
   a.per_xcd = (a.ntx * a.nty * a.ntz + 7) / 8;
-  return a;
+  *out = a;
+  return CG_OK;
 }
 
-static int cons_eval(cg_ctx* c) {
-  int rin;
-  if (int rc = cons_input(c, &rin)) return rc;
-  const long pad = c->rstride;
-  const int nb = 1024;
-  if (!c->cons) {
-    HIPCHK(c, hipMalloc((void**)&c->cons, (size_t)CONS_N * pad * sizeof(double)));
-    HIPCHK(c, hipMalloc((void**)&c->cons_part, (size_t)nb * 5 * kStats * sizeof(double) + 64 * sizeof(double)));
+// the constraint pass over every point (prepBSSNOutput's set_bd_values,
+// sims/sim.cc:214-231, with the constraint values of setConstraintCalcs):
+// every per-point array into c->cons, or with rows only the ones
+// cg_field_download reads and one row per workgroup
+static int cons_eval(cg_ctx* c, bool rows) {
+  StageArgs a;
+  bool dma;
+  if (int rc = cons_args(c, &a, &dma)) return rc;
+  const long pad = c->rstride, tiles = (long)a.ntx * a.nty * a.ntz;
+  if (!c->cons) HIPCHK(c, hipMalloc((void**)&c->cons, (size_t)CONS_N * pad * sizeof(double)));
+  if (rows && c->cons_tiles < tiles) {
+    if (c->cons_part) (void)hipFree(c->cons_part);
+    c->cons_part = nullptr;
+    c->cons_tiles = 0;
+    HIPCHK(c, hipMalloc((void**)&c->cons_part, (size_t)(tiles + kFinBlocks + 1) * CONS_ROW_F * sizeof(double)));
+    c->cons_tiles = tiles;
   }
-  StageArgs a = cons_args(c, rin);
   a.cons = c->cons;
   a.cons_stride = pad;
-  int rc = launch_constraints(c->prec, c->p.stencil_order, alpha_live(c), c->dreg != nullptr, a, c->stream);
+  if (rows) {
+    a.cons_rows = c->cons_part;
+    a.cons_pass = 2;
+  }
+  int rc = launch_constraints(c->prec, c->p.stencil_order, alpha_live(c), c->dreg != nullptr, dma, a, c->stream);
   if (rc) return fail(c, CG_ERR_HIP, std::string("constraint launch: ") + hipGetErrorString((hipError_t)rc));
   c->cons_valid = true;
+  c->cons_rows_last = tiles;
+  if (!rows) return CG_OK;
+  // totals, then the squared deviations from the means they give
+  double* part = c->cons_part + tiles * CONS_ROW_F;
+  double* fin = part + (long)kFinBlocks * CONS_ROW_F;
+  for (int pass = 0; pass < 2; ++pass) {
+    hipLaunchKernelGGL(k_cons_fin, dim3(kFinBlocks), dim3(kFinThreads), 0, c->stream, (const double*)c->cons_part, tiles,
+                       pass, (const double*)(pass ? fin : nullptr), part);
+    hipLaunchKernelGGL(k_cons_fin, dim3(1), dim3(kFinThreads), 0, c->stream, (const double*)part, (long)kFinBlocks, pass,
+                       (const double*)nullptr, fin);
+  }
+  HIPCHK(c, hipGetLastError());
   return CG_OK;
 }
 
@@ -1508,30 +1549,20 @@ static void cons_stats(const cg_ctx* c, const double* tot, const double* means, 
 
 int cg_constraints(cg_ctx* c, double H[8], double M[8], double G[7], double A[7], double S[7]) {
   if (!c) return CG_ERR_ARG;
-  if (int rc = cons_eval(c)) return rc;
-  const long pad = c->rstride;
-  const int nb = 1024;
-  double* part = c->cons_part;
-  double* fin = part + (size_t)nb * 5 * kStats;  // 30 + 10 + 10 doubles
-  hipLaunchKernelGGL(k_cons_partial, dim3(nb), dim3(kRedThreads), 0, c->stream, c->cons, pad, c->npts, part);
-  hipLaunchKernelGGL(k_combine, dim3(1), dim3(64), 0, c->stream, part, nb, 5 * kStats, 0x30u, fin);
-  HIPCHK(c, hipGetLastError());
-  double tot[5 * kStats];
-  HIPCHK(c, hipMemcpyAsync(tot, fin, sizeof tot, hipMemcpyDeviceToHost, c->stream));
+  if (int rc = cons_eval(c, true)) return rc;
+  double row[CONS_ROW_F];
+  HIPCHK(c, hipMemcpyAsync(row, c->cons_part + (c->cons_rows_last + kFinBlocks) * CONS_ROW_F, sizeof row,
+                           hipMemcpyDeviceToHost, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
   const double N = (double)c->npts;
-  double means[10];
+  double tot[5 * kStats], means[10], var[10];
   for (int q = 0; q < 5; ++q) {
+    for (int k = 0; k < kStats; ++k) tot[q * kStats + k] = row[8 * q + k];
     means[2 * q] = tot[q * kStats + 0] / N;      // BSSN_NORMALIZE_MEAN
     means[2 * q + 1] = tot[q * kStats + 2] / N;
+    var[2 * q] = row[8 * q + 6];
+    var[2 * q + 1] = row[8 * q + 7];
   }
-  HIPCHK(c, hipMemcpyAsync(fin + 30, means, sizeof means, hipMemcpyHostToDevice, c->stream));
-  hipLaunchKernelGGL(k_cons_var, dim3(nb), dim3(kRedThreads), 0, c->stream, c->cons, pad, c->npts, fin + 30, part);
-  hipLaunchKernelGGL(k_combine, dim3(1), dim3(64), 0, c->stream, part, nb, 10, 0u, fin + 40);
-  HIPCHK(c, hipGetLastError());
-  double var[10];
-  HIPCHK(c, hipMemcpyAsync(var, fin + 40, sizeof var, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
   cons_stats(c, tot, means, var, H, M, G, A, S);
   return CG_OK;
 }
@@ -1540,9 +1571,9 @@ int cg_constraints_noalloc(cg_ctx* c, double H[8], double M[8], double G[7], dou
   if (!c) return CG_ERR_ARG;
   double* sc = (c->p.device >= 0 && c->p.device < kNaDevices) ? g_scratch_dev[c->p.device] : nullptr;
   if (!sc) return fail(c, CG_ERR_STATE, "no constraint scratch on this device (device ordinal >= 64)");
-  int rin;
-  if (int rc = cons_input(c, &rin)) return rc;
-  StageArgs a = cons_args(c, rin);
+  StageArgs a;
+  bool dma;
+  if (int rc = cons_args(c, &a, &dma)) return rc;
   double* acc0 = sc + kNaTot;             // pass-0 totals [CONS_ROW_W]
   double* acc1 = acc0 + CONS_ROW_W;       // pass-1 totals [CONS_ROW_W1]
   double* dmeans = acc1 + CONS_ROW_W1;    // [10]
@@ -1556,7 +1587,7 @@ int cg_constraints_noalloc(cg_ctx* c, double H[8], double M[8], double G[7], dou
       a.tile_base = base;
       a.tile_count = std::min(kNaRows, total - base);
       a.per_xcd = (a.tile_count + 7) / 8;
-      int rc = launch_constraints(c->prec, c->p.stencil_order, alpha_live(c), c->dreg != nullptr, a, c->stream);
+      int rc = launch_constraints(c->prec, c->p.stencil_order, alpha_live(c), c->dreg != nullptr, dma, a, c->stream);
       if (rc) return fail(c, CG_ERR_HIP, std::string("constraint launch: ") + hipGetErrorString((hipError_t)rc));
       hipLaunchKernelGGL(k_rows_fold, dim3(1), dim3(kFoldThreads), 0, c->stream, (const double*)sc, a.tile_count,
                          CONS_ROW_W, pass == 0 ? CONS_ROW_W : CONS_ROW_W1, pass, base == 0 ? 1 : 0,
@@ -1645,7 +1676,7 @@ int cg_constraint_strip(cg_ctx* c, int axis, long n1, long n2, double* H, double
   const long nx = c->p.nx, ny = c->p.ny, nz = c->p.nz;
   const long ext[3] = {nx, ny, nz};
   if ((long)n != ext[axis - 1]) return fail(c, CG_ERR_ARG, "a strip holds the grid's extent along its axis");
-  if (int rc = cons_eval(c)) return rc;
+  if (int rc = cons_eval(c, false)) return rc;
   // set1DConstraintOutput passes the running index as i for every axis
   // (bssn.cc:918-934), so the points are (x, n1, n2) with x wrapped in i
   const long base = wrap_index(n1, ny) * nz + wrap_index(n2, nz), run = ny * nz;

@@ -136,7 +136,8 @@ struct cg_ctx {
   unsigned* mq_part = nullptr;            // per-block maxima (lazy)
   unsigned* mq_sat = nullptr;             // count of saturated words written by the stage kernels
   double* cons = nullptr;                 // [CONS_N][pad] per-point constraint values (lazy)
-  double* cons_part = nullptr;            // reduction partials
+  double* cons_part = nullptr;            // one row per workgroup of a constraint pass, then the partial totals
+  long cons_tiles = 0, cons_rows_last = 0;  // rows it has room for; rows of the last pass
   bool cons_valid = false;                // ricci_a / AijAij_a filled
   double* obuf = nullptr;                 // device staging of strips and partial sums (lazy)
   size_t obuf_n = 0;

@@ -1316,8 +1316,8 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
       const double rr = (double)DIFFr + fv.rho;
       const double e5 = exp(5.0 * (double)phi), e6 = exp(6.0 * (double)phi);
       // hamiltonianConstraintScale (bssn.cc:1086-1100)
-      const double Hs = (e5 / 8.0) * sqrt((double)ricci * ricci + (double)AijAij * AijAij +
-                                          pow(2.0 / 3.0 * (double)K * K, 2) + pow(16.0 * 3.14159265358979323846 * rr, 2));
+      const double k2 = 2.0 / 3.0 * (double)K * K, r16 = 16.0 * 3.14159265358979323846 * rr;
+      const double Hs = (e5 / 8.0) * sqrt((double)ricci * ricci + (double)AijAij * AijAij + k2 * k2 + r16 * r16);
       put(CONS_H, Hc); put(CONS_H + 1, Hs); put(CONS_H + 2, Hc / Hs);
       // BSSN_MI / BSSN_MI_SCALE (bssn_macros.h:487-527)
       double M2 = 0, Ms2 = 0;

@@ -1092,6 +1092,22 @@ static int step_init_t(cg_ctx* c) {
   return rc;
 }
 
+// DIFFgamma_ij and A_ij of slot rp, normalised, into slot rn
+static int norm_copy(cg_ctx* c, int rp, int rn) {
+  const int bs = 256;
+  const long nbk = (c->npts + bs - 1) / bs;
+  auto copy = [&](auto ts, auto mt) {
+    hipLaunchKernelGGL((k_norm_copy<decltype(ts), decltype(mt)>), dim3(nbk), dim3(bs), 0, c->stream, reg_table(c), rp,
+                       rn, c->npts);
+  };
+  if (c->prec == CG_FP64) copy(double(), double());
+  else if (c->mq) copy(float(), int());
+  else if (c->met32) copy(float(), float());
+  else copy(float(), double());
+  HIPCHK(c, hipGetLastError());
+  return CG_OK;
+}
+
 // Dust::stepInit's register part (dust.cc:65-73) into slot ra
 static int dust_reg_init(cg_ctx* c, int rp, int ra, int rf) {
   const int bs = 256;
@@ -1252,8 +1268,7 @@ int cg_rk4_steps(cg_ctx* c, int nsteps) {
   // (its DIFFgamma_ij from the normalised copy when that stage read one)
   int prev_in = 0, prev_met = 0, prev_norm = 0;
   double prev_phiF = 0.0;
-  // Accumulator-free form (no _f sweeps; the KO path with normalisation
-  // keeps the reference's accumulator)
+  // Accumulator-free form (no _f sweeps)
   const bool incr = fused_incr(c) && c->incr_pick;
   auto stage = [&](int n, int rin, int rout, int normalize, int in_norm = -1, int norm_out = -1, int sf = 1,
                    int sa2 = -1) -> int {
@@ -1294,8 +1309,15 @@ int cg_rk4_steps(cg_ctx* c, int nsteps) {
     // fixed-point metric: exponents checked every kMqCheck steps (a field's
     // words stay below 2^MQ_BITS; twice that saturates)
     if (c->mq && s % kMqCheck == 0 && (rc = mq_check(c))) return rc;
-    const bool pre = !ko_norm && c->p.normalize_metric && s + 1 < nsteps && c->var &&
+    const bool pre = c->p.normalize_metric && s + 1 < nsteps && c->var &&
                      c->dma_allowed && c->dma_pick && dma_fits(c, *c->var);
+    if (ko_norm && !have_norm) {
+      // KO needs normalised A_ij at halo points, which stage 1 does not form
+      // on the fly: the copy is materialised where no stage 4 wrote one
+      if ((rc = norm_copy(c, 0, Y))) return rc;
+      have_norm = true;
+      norm_slot = Y;
+    }
     if (incr) {
       // a1, a2, a3 rotate over slots 1..3 so that the normalised copy of the
       // last stage 4 (written over a1) is the next stage 1's input
@@ -1318,28 +1340,19 @@ int cg_rk4_steps(cg_ctx* c, int nsteps) {
       }
       continue;
     }
-    if (ko_norm) {
-      // KO needs normalised A_ij at halo points: materialise stepInit first
-      c->a_is_p = false; c->sA = X; c->sC = Y;
-      if ((rc = cg_step_init(c))) return rc;
-      if ((rc = stage(1, X, Y, 0))) return rc;
-      if ((rc = stage(2, Y, X, 0))) return rc;
-    } else {
-      // stepInit's setExtraFieldData equals the last K4Finalize's unless the
-      // state changed in between; only the ConformalFLRW lapse reads it
-      if (flrw && !c->ext_fresh && (rc = ext_from_state(c))) return rc;
-      if ((rc = have_norm ? stage(1, 0, X, 0, Y) : stage(1, 0, X, c->p.normalize_metric))) return rc;
-      if ((rc = stage(2, X, Y, 0))) return rc;
-    }
-    const int in3 = ko_norm ? X : Y, out3 = ko_norm ? Y : X;
-    if ((rc = stage(3, in3, out3, 0))) return rc;
-    if ((rc = stage(4, out3, 0, 0, -1, pre ? Y : -1))) return rc;
+    // stepInit's setExtraFieldData equals the last K4Finalize's unless the
+    // state changed in between; only the ConformalFLRW lapse reads it
+    if (flrw && !c->ext_fresh && (rc = ext_from_state(c))) return rc;
+    if ((rc = have_norm ? stage(1, 0, X, 0, Y) : stage(1, 0, X, c->p.normalize_metric))) return rc;
+    if ((rc = stage(2, X, Y, 0))) return rc;
+    if ((rc = stage(3, Y, X, 0))) return rc;
+    if ((rc = stage(4, X, 0, 0, -1, pre ? Y : -1))) return rc;
     have_norm = pre;
-    c->sA = 0; c->sC = out3; c->a_is_p = true;
+    c->sA = 0; c->sC = X; c->a_is_p = true;
     c->ext_fresh = flrw;
     if (!flrw) {
       c->ext_lazy = true;
-      c->ext_lazy_in = out3;
+      c->ext_lazy_in = X;
       c->ext_lazy_src = src4;
       c->ext_lazy_phiF = c->frw.g_phi;
     }
@@ -1454,17 +1467,7 @@ static int cons_args(cg_ctx* c, StageArgs* out, bool* dma) {
   StageArgs a = make_args(c, 0, c->a_is_p ? c->sP : c->sA, c->sP, c->sF, c->sC, 0);
   if (c->a_is_p && c->p.normalize_metric) {
     a.s_in_norm = spare_slot(c);
-    const int bs = 256;
-    const long nbk = (c->npts + bs - 1) / bs;
-    auto copy = [&](auto ts, auto mt) {
-      hipLaunchKernelGGL((k_norm_copy<decltype(ts), decltype(mt)>), dim3(nbk), dim3(bs), 0, c->stream, reg_table(c),
-                         c->sP, a.s_in_norm, c->npts);
-    };
-    if (c->prec == CG_FP64) copy(double(), double());
-    else if (c->mq) copy(float(), int());
-    else if (c->met32) copy(float(), float());
-    else copy(float(), double());
-    HIPCHK(c, hipGetLastError());
+    if (int rc = norm_copy(c, c->sP, a.s_in_norm)) return rc;
   }
   // the DMA form's conditions are those of the stage kernels (dma_fits)
   StageVariant v{};
@@ -1826,7 +1829,7 @@ int cg_autotune(cg_ctx* c, int reps, char* report, size_t report_len) {
             if (st == 1 && c->p.normalize_metric) {
               // steady state of the fused step: the normalised copy with
               // DMA staging (slot 2 stands in), on the fly without
-              if (d == 1 && !ko_norm_path(c)) a.s_in_norm = 2;
+              if (d == 1 || ko_norm_path(c)) a.s_in_norm = 2;
               else a.normalize = 1;
             }
             a.rho_out = nullptr;  // dust: DIFFr_a keeps the last real stage's source

@@ -323,7 +323,7 @@ __global__ void k_to_double(const T* __restrict__ f, long n, double* __restrict_
 // half spectrum [nx][ny][nz/2+1]: |F|^2 of each mode into bin
 // floor(|p|), counted twice for 0 < pz < nz/2 (the mode and its conjugate)
 // and once at pz = 0 and pz = nz/2.  One row of nbins sums and counts per
-// block (LDS atomics), summed on the host in block order.
+// block (LDS atomics), summed in block order by k_power_sum.
 constexpr int kPowThreads = 256;
 __global__ void __launch_bounds__(kPowThreads) k_power_bins(const double2* __restrict__ spec, int nx, int ny, int nz,
                                                            int nbins, double* __restrict__ part_f,
@@ -354,6 +354,24 @@ __global__ void __launch_bounds__(kPowThreads) k_power_bins(const double2* __res
   }
 }
 
+// out[2 bin], out[2 bin + 1]: sum and count of a bin over the blocks' rows.
+// One wave per bin: lane l adds rows l, l + 64, ..., then a fixed tree.
+__global__ void __launch_bounds__(64) k_power_sum(const double* __restrict__ part_f, const unsigned* __restrict__ part_n,
+                                                  int blocks, int nbins, double* __restrict__ out) {
+  const int q = blockIdx.x;
+  double f = 0.0, c = 0.0;
+  for (int b = threadIdx.x; b < blocks; b += 64) {
+    f += part_f[(long)b * nbins + q];
+    c += (double)part_n[(long)b * nbins + q];
+  }
+  f = wave_sum(f);
+  c = wave_sum(c);
+  if (threadIdx.x == 0) {
+    out[2 * q] = f;
+    out[2 * q + 1] = c;
+  }
+}
+
 }  // namespace
 
 int cg_power_spectrum(cg_ctx* c, const char* name, double* out, int nbins) {
@@ -375,7 +393,7 @@ int cg_power_spectrum(cg_ctx* c, const char* name, double* out, int nbins) {
   Scratch w;
   HIPCHK(c, hipMalloc((void**)&w.work, n * sizeof(double)));
   HIPCHK(c, hipMalloc((void**)&w.spec, nspec * sizeof(double2)));
-  HIPCHK(c, hipMalloc((void**)&w.part, (size_t)kBlocks * nbins * (sizeof(double) + sizeof(unsigned))));
+  HIPCHK(c, hipMalloc((void**)&w.part, (size_t)nbins * (kBlocks * (sizeof(double) + sizeof(unsigned)) + 2 * sizeof(double))));
   if (int rc = w.r2c.take(c, HIPFFT_D2Z, s)) return rc;
   const int nb = (int)std::min<long>(4096, (n + 255) / 256);
   if (esz == 8)
@@ -384,25 +402,18 @@ int cg_power_spectrum(cg_ctx* c, const char* name, double* out, int nbins) {
     hipLaunchKernelGGL(k_to_double<float>, dim3(nb), dim3(256), 0, s, (const float*)d, n, w.work);
   HIPCHK(c, hipGetLastError());
   FFTCHK(c, w.r2c.d2z(w.work, w.spec));
-  double* pf = w.part;
-  unsigned* pn = reinterpret_cast<unsigned*>(w.part + (size_t)kBlocks * nbins);
+  double* sums = w.part;
+  double* pf = sums + 2 * (size_t)nbins;
+  unsigned* pn = reinterpret_cast<unsigned*>(pf + (size_t)kBlocks * nbins);
   const size_t shmem = (size_t)nbins * (sizeof(double) + sizeof(unsigned));
   hipLaunchKernelGGL(k_power_bins, dim3(kBlocks), dim3(kPowThreads), shmem, s, w.spec, nx, ny, nz, nbins, pf, pn);
+  hipLaunchKernelGGL(k_power_sum, dim3(nbins), dim3(64), 0, s, (const double*)pf, (const unsigned*)pn, kBlocks, nbins,
+                     sums);
   HIPCHK(c, hipGetLastError());
-  std::vector<double> hf((size_t)kBlocks * nbins);
-  std::vector<unsigned> hn((size_t)kBlocks * nbins);
-  HIPCHK(c, hipMemcpyAsync(hf.data(), pf, hf.size() * sizeof(double), hipMemcpyDeviceToHost, s));
-  HIPCHK(c, hipMemcpyAsync(hn.data(), pn, hn.size() * sizeof(unsigned), hipMemcpyDeviceToHost, s));
+  std::vector<double> h(2 * (size_t)nbins);
+  HIPCHK(c, hipMemcpyAsync(h.data(), sums, h.size() * sizeof(double), hipMemcpyDeviceToHost, s));
   HIPCHK(c, hipStreamSynchronize(s));
-  for (int q = 0; q < nbins; ++q) {
-    double f = 0.0;
-    unsigned long long cnt = 0;
-    for (int b = 0; b < kBlocks; ++b) {
-      f += hf[(size_t)b * nbins + q];
-      cnt += hn[(size_t)b * nbins + q];
-    }
-    out[q] = cnt ? f / (double)cnt : 0.0;  // utils/Fourier.h:209-220
-  }
+  for (int q = 0; q < nbins; ++q) out[q] = h[2 * q + 1] > 0.0 ? h[2 * q] / h[2 * q + 1] : 0.0;  // utils/Fourier.h:209-220
   return CG_OK;
 }
 

@@ -230,12 +230,13 @@ int mq_check(cg_ctx* c);
 void mq_free(cg_ctx* c);
 // a "Bardeen_<name>" array of the last cg_bardeen (err 1: unknown name, 4: not computed)
 const double* bardeen_field(const cg_ctx* c, const std::string& name, int* err);
-// KO at orders 2/8 with metric normalisation materialises stepInit's _a
+// KO at orders 2/8 with metric normalisation needs stepInit's DIFFgamma_ij
+// and A_ij materialised before stage 1
 inline bool ko_norm_path(const cg_ctx* c) {
   return c->p.ko_coeff != 0.0 && c->p.normalize_metric && (c->p.stencil_order == 2 || c->p.stencil_order == 8);
 }
 // fused steps may run in the accumulator-free form (StageArgs::incr)
-inline bool fused_incr(const cg_ctx* c) { return !ko_norm_path(c) && !c->keep_accumulator; }
+inline bool fused_incr(const cg_ctx* c) { return !c->keep_accumulator; }
 // stage slots of an accumulator-free fused step whose stage 1 reads the
 // normalised copy in slot n (1..3), or n = 0 with none: a1, a2, a3 follow n
 // in the rotation 1 -> 2 -> 3 -> 1, and stage 4 writes the next copy over a1

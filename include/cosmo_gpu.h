@@ -283,8 +283,7 @@ int cg_set_dma(cg_ctx* ctx, int on);
  * 17 of RK4Register.h:118-176 (the dust fluid's registers included).  The
  * result differs from the reference's accumulation by rounding (about one
  * unit in the last place of _p per step).  The autotuner times both forms
- * and keeps the faster; without it the accumulator-free form runs.  KO at
- * orders 2 and 8 with metric normalisation always uses the reference's form.
+ * and keeps the faster; without it the accumulator-free form runs.
  * keep = 1: the reference's accumulator. */
 int cg_set_fused_accumulator(cg_ctx* ctx, int keep);
 

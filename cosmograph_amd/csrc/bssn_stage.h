@@ -21,6 +21,8 @@ enum { MODE_STAGE = 0, MODE_CONS = 1, MODE_DUST = 2, MODE_DUST_CONS = 3 };
 // (with bit 2): the conformal metric in 32-bit fixed point instead, value =
 // integer word x 2^e with one power-of-two scale per field
 enum { MODE_M32 = 4, MODE_M32_CONS = 5, MODE_MQ = 8, MODE_MQ_STAGE = 12, MODE_MQ_CONS = 13 };
+// bit 4: the shift build's fused stages, which add the gauge pass's terms
+enum { MODE_SHIFT = 16 };
 // fixed-point metric word (MODE_MQ): value / 2^e rounded to the nearest
 // integer, saturated at MQ_WMAX = 2^30 - 1 in magnitude.  After each
 // exponent check the host keeps |word| below 2^MQ_BITS = 2^29, so a field
@@ -135,6 +137,14 @@ struct StageArgs {
   // and the count of saturated words
   double msc[7], minv[7];
   float msd1[7], msd2[7];
+  // shift build, fused stages (MODE_SHIFT): the gauge pass's terms of every
+  // field's right-hand side lie in slot s_add, at this point read before
+  // anything is written there; with the Gamma driver the auxB^i registers
+  // (auxB: slot 0 of auxB^1; null otherwise) are stepped here too, their
+  // right-hand side being 3/4 of the complete d_t Gamma^i minus eta auxB^i
+  int s_add;
+  double* auxB;
+  double gd_eta;
   unsigned int* mq_sat;
 };
 
@@ -310,6 +320,7 @@ struct StageVariant {
 };
 
 std::vector<StageVariant>& stage_variants();
+std::vector<StageVariant>& shift_variants();  // MODE_SHIFT kernels (LDS-DMA form only)
 struct StageVariantReg {
   explicit StageVariantReg(const StageVariant& v) { stage_variants().push_back(v); }
 };

@@ -295,6 +295,7 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
   constexpr bool M32 = (MODE & MODE_M32) != 0;                  // metric in the storage type
   constexpr bool CONS = (MODE & MODE_CONS) != 0;
   constexpr bool DUST = (MODE & MODE_DUST) != 0;
+  constexpr bool SHIFT = (MODE & MODE_SHIFT) != 0;
   constexpr int KO_ORDER = (H > R) ? 2 * R : 0;
   // axis-only tiles: the points within H along one axis of the tile's own
   // (x part: HI x TJ x TK, y part: TI x HJ x TK, z part: TI x TJ x HK4)
@@ -315,7 +316,7 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
   static_assert(!MQ || sizeof(TS) == 4, "the fixed-point metric shares the 4-byte storage");
   // epilogue prefetch: the stage kernels, and with every field in 4 bytes
   // the dust ones too (which then load the fluid's point values first)
-  constexpr bool PF = DMA && ((MODE & ~(MODE_M32 | MODE_MQ)) == 0 ||
+  constexpr bool PF = DMA && ((MODE & ~(MODE_M32 | MODE_MQ | MODE_SHIFT)) == 0 ||
                               (M32 && (MODE & ~(MODE_M32 | MODE_MQ | MODE_DUST)) == 0));
   constexpr bool PFD = PF && (MODE & MODE_DUST) != 0;
   constexpr int F32 = M32 ? 0 : 7;                              // first field of the FP32 prefetch chunks
@@ -1456,6 +1457,10 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
         // use instead (a few registers per field).
         constexpr int AHEAD = PF ? 4 : 2;
         double a2v[NF], a3m[7], pv[NF], qv[NF];
+        // the gauge pass's terms (upwind advection, hence the K term, is zero
+        // beyond order 4) and the Gamma driver's registers
+        double addv[SHIFT ? NF : 1], bin[SHIFT ? 3 : 1], bp[SHIFT ? 3 : 1], bf[SHIFT ? 3 : 1];
+        auto has_add = [](int g) { return SHIFT && !(g == KK && R > 2); };
         auto pre = [&](int g) {
           if (g >= NF || st == 0 || (g == ALPHA && !LIVE_ALPHA)) return;
           // a storage-type word as FP64 (fixed-point metric words scaled)
@@ -1463,6 +1468,17 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
             if (MQ && g < 7) return (double)ldo((const int*)RS(g, slot), idx) * a.msc[g < 7 ? g : 0];
             return (double)ldo((const TS*)RS(g, slot), idx);
           };
+          if constexpr (SHIFT) {
+            if (has_add(g))
+              addv[g] = mfield<M32>(g) ? ldo((const double*)RM(g, a.s_add), idx) : (double)ldo((const TS*)RS(g, a.s_add), idx);
+            if (g >= GAM1 && g <= GAM3 && a.auxB) {
+              const int i = g >= GAM1 && g <= GAM3 ? g - GAM1 : 0;
+              const double* xb = a.auxB + (long)i * 4 * a.rstride;
+              bin[i] = ldo(xb + (long)a.s_in * a.rstride, idx);
+              bp[i] = ldo(xb + (long)a.s_p * a.rstride, idx);
+              bf[i] = st >= 2 ? ldo(xb + (long)a.s_f * a.rstride, idx) : 0.0;
+            }
+          }
           if constexpr (!PF) {
             const bool m = mfield<M32>(g);
             pv[g] = m ? ldo((const double*)RM(g, a.s_p), idx) : lw(a.s_p);
@@ -1488,7 +1504,16 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
         for (int f = 0; f < NF; ++f) {
           pre(f + AHEAD);
           if (f == ALPHA && !LIVE_ALPHA) continue;  // lapse registers stay identically zero
-          const double cc = (double)rhs[f];
+          const double cc = has_add(f) ? (double)rhs[f] + addv[SHIFT ? f : 0] : (double)rhs[f];
+          if constexpr (SHIFT) {
+            if (f >= GAM1 && f <= GAM3 && a.auxB) {
+              const int i = f >= GAM1 && f <= GAM3 ? f - GAM1 : 0;
+              double* xb = a.auxB + (long)i * 4 * a.rstride;
+              const double cb = 0.75 * cc - a.gd_eta * bin[i], inc = a.cf * cb;
+              sto(xb + (long)a.s_out * a.rstride, idx, st == 4 ? bf[i] + (inc + bp[i]) : bp[i] + a.ca * cb);
+              if (st != 4) sto(xb + (long)a.s_f * a.rstride, idx, bf[i] + inc);
+            }
+          }
           if (mfield<M32>(f)) {
             double* __restrict__ o = RM(f, a.s_out);
             if (st == 0) {
@@ -1576,8 +1601,12 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
           }
         }
       };
-      if (a.incr) epilogue(std::true_type{});
-      else epilogue(std::false_type{});
+      if constexpr (SHIFT) {
+        epilogue(std::false_type{});  // four slots hold p, f, the input and the terms
+      } else {
+        if (a.incr) epilogue(std::true_type{});
+        else epilogue(std::false_type{});
+      }
       if (DMA && st == 4 && a.s_norm_out >= 0) {
         // set_DIFFgamma_Aij_norm (bssn.cc:61-119) of the new state, as the
         // next step's stepInit applies it to _a (DMA kernels only: the

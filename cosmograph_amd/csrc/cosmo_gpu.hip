@@ -981,29 +981,45 @@ StageArgs make_args(cg_ctx* c, int stage, int rin, int rp, int rf, int rout, int
 }
 }  // namespace cg
 
-static int launch(cg_ctx* c, StageArgs a) {
+// the stage kernel of the shift build's fused steps, or null where the grid,
+// the order or the gauge has none (the method sequence then runs)
+static const StageVariant* shift_variant(const cg_ctx* c) {
+  if (!gauge_fusable(c)) return nullptr;
+  for (const auto& v : shift_variants())
+    if (v.prec == c->prec && v.order == c->p.stencil_order && v.halo == c->H && v.live_alpha == alpha_live(c) &&
+        variant_fits(c, v) && dma_fits(c, v))
+      return &v;
+  return nullptr;
+}
+
+// var: the kernel to launch (null: the context's own choice)
+static int launch(cg_ctx* c, StageArgs a, const StageVariant* var = nullptr) {
   hipEvent_t e0 = nullptr, e1 = nullptr;
   if (c->timing) {
     HIPCHK(c, hipEventCreate(&e0));
     HIPCHK(c, hipEventCreate(&e1));
     HIPCHK(c, hipEventRecord(e0, c->stream));
   }
-  const bool live = alpha_live(c);
-  if (!c->var || c->var->live_alpha != live) {
-    c->var = pick_variant(c);
-    if (!c->var) return fail(c, CG_ERR_ARG, "no stage kernel variant fits this grid/order");
+  const bool fixed = var != nullptr;
+  if (!fixed) {
+    const bool live = alpha_live(c);
+    if (!c->var || c->var->live_alpha != live) {
+      c->var = pick_variant(c);
+      if (!c->var) return fail(c, CG_ERR_ARG, "no stage kernel variant fits this grid/order");
+    }
+    var = c->var;
   }
-  a.ntx = (c->p.nx + c->var->ti - 1) / c->var->ti;
-  a.nty = (c->p.ny + c->var->tj - 1) / c->var->tj;
-  a.ntz = (c->p.nz + c->var->tk - 1) / c->var->tk;
+  a.ntx = (c->p.nx + var->ti - 1) / var->ti;
+  a.nty = (c->p.ny + var->tj - 1) / var->tj;
+  a.ntz = (c->p.nz + var->tk - 1) / var->tk;
   if (a.tile_order == 3 && !morton_fits(a.ntx, a.nty)) a.tile_order = 0;
   a.per_xcd = (a.ntx * a.nty * a.ntz + 7) / 8;
   c->last_rows = (long)a.ntx * a.nty * a.ntz;
   if (c->last_rows > c->ext_rows) return fail(c, CG_ERR_STATE, "extra-field partial buffer too small");
   // stage-1 normalisation needs the register path (it transforms the metric on its way into LDS)
-  const bool dma = c->dma_allowed && c->dma_pick && !a.normalize && dma_fits(c, *c->var);
+  const bool dma = fixed || (c->dma_allowed && c->dma_pick && !a.normalize && dma_fits(c, *var));
   if (a.s_norm_out >= 0 && !dma) return fail(c, CG_ERR_STATE, "normalised copy without DMA staging");
-  int rc = (dma ? c->var->launch_dma : c->var->launch)(a, c->stream);
+  int rc = (dma ? var->launch_dma : var->launch)(a, c->stream);
   if (rc != 0) return fail(c, CG_ERR_HIP, std::string("stage launch: ") + hipGetErrorString((hipError_t)rc));
   if (c->timing) {
     HIPCHK(c, hipEventRecord(e1, c->stream));
@@ -1239,8 +1255,9 @@ constexpr int kMqCheck = 2;
 
 int cg_rk4_steps(cg_ctx* c, int nsteps) {
   if (!c || nsteps < 0) return CG_ERR_ARG;
-  if (gauge_pass(c)) {
-    // The shift build runs the reference's method sequence
+  c->svar = shift_variant(c);
+  if (gauge_pass(c) && !c->svar) {
+    // Without a fused form the shift build runs the reference's method sequence
     // (sims/static.cc:74-170): stepInit, the NaN guard, then RKEvolve (stage
     // kernel + gauge pass) and K{n}Finalize per stage.
     for (int s = 0; s < nsteps; ++s) {
@@ -1269,7 +1286,10 @@ int cg_rk4_steps(cg_ctx* c, int nsteps) {
   int prev_in = 0, prev_met = 0, prev_norm = 0;
   double prev_phiF = 0.0;
   // Accumulator-free form (no _f sweeps)
-  const bool incr = fused_incr(c) && c->incr_pick;
+  // (the shift build's four slots hold p, f, the stage's input and the gauge
+  // pass's terms: the reference's accumulator)
+  const bool shift = c->svar != nullptr;
+  const bool incr = fused_incr(c) && c->incr_pick && !shift;
   auto stage = [&](int n, int rin, int rout, int normalize, int in_norm = -1, int norm_out = -1, int sf = 1,
                    int sa2 = -1) -> int {
     StageArgs a = make_args(c, n, rin, 0, sf, rout, normalize);
@@ -1291,10 +1311,18 @@ int cg_rk4_steps(cg_ctx* c, int nsteps) {
       prev_norm = normalize;
       prev_phiF = c->frw.g_phi;
     }
+    if (shift) {
+      // the terms go to the slot the stage writes, at stage 4 (which writes
+      // _p) to the dead one
+      a.s_add = n == 4 ? Y : rout;
+      a.auxB = c->p.shift == CG_SHIFT_GAMMA_DRIVER ? c->xreg + (long)XAUXB1 * 4 * c->rstride : nullptr;
+      a.gd_eta = c->gd_eta;
+      if (int rc = gauge_terms(c, a)) return rc;
+    }
     src4 = SrcArgs{c->DIFFD, c->p.matter, c->frw.g_phi, c->frw.g_rho, c->lambda, c->rho_src};
     c->frw.stage(n, c->p.dt);
     a.phi_F_next = c->frw.g_phi;
-    int rc = launch(c, a);
+    int rc = launch(c, a, c->svar);
     return (rc || !flrw) ? rc : ext_combine(c, c->last_rows, false);
   };
   c->ext_lazy = false;
@@ -1309,11 +1337,12 @@ int cg_rk4_steps(cg_ctx* c, int nsteps) {
     // fixed-point metric: exponents checked every kMqCheck steps (a field's
     // words stay below 2^MQ_BITS; twice that saturates)
     if (c->mq && s % kMqCheck == 0 && (rc = mq_check(c))) return rc;
-    const bool pre = c->p.normalize_metric && s + 1 < nsteps && c->var &&
-                     c->dma_allowed && c->dma_pick && dma_fits(c, *c->var);
-    if (ko_norm && !have_norm) {
-      // KO needs normalised A_ij at halo points, which stage 1 does not form
-      // on the fly: the copy is materialised where no stage 4 wrote one
+    const bool pre = c->p.normalize_metric && s + 1 < nsteps &&
+                     (shift || (c->var && c->dma_allowed && c->dma_pick && dma_fits(c, *c->var)));
+    if ((ko_norm || (shift && c->p.normalize_metric)) && !have_norm) {
+      // KO and the advection need normalised A_ij at halo points, which stage
+      // 1 does not form on the fly: the copy is materialised where no stage 4
+      // wrote one
       if ((rc = norm_copy(c, 0, Y))) return rc;
       have_norm = true;
       norm_slot = Y;

@@ -40,6 +40,7 @@
 #include <cmath>
 
 #include "bssn_stage.h"
+#include "bssn_stage_kernel.h"
 #include "runtime.h"
 #include "stencil.h"
 
@@ -63,6 +64,11 @@ struct GaugeArgs {
   double phi_F, K_F;
   const double* ext;  // [K_min, K_avg, avg_vol, rho_avg] (device)
   int nseq;           // number of staged arrays (see staged())
+  // k_gauge_terms: DIFFgamma_ij and A_ij are read from slot s_in_norm; the
+  // shift registers' RK4 update of stage `stage` (slots s_p, s_f, s_xout, as
+  // StageArgs); per_xcd tiles per XCD
+  int s_in_norm, s_p, s_f, s_xout, stage, live_alpha, per_xcd;
+  double cf, ca;
 };
 
 // Materialises a value in registers at this point: the per-point sums
@@ -408,6 +414,377 @@ __global__ void __launch_bounds__(GNT) __attribute__((amdgpu_waves_per_eu(2))) k
     for (int I = 0; I < 3; ++I) xr(XBETA1 + I, a.s_out)[idx] = sh[I];
 }
 
+// The same terms for the fused steps (cg_rk4_steps), into slot s_out instead
+// of on top of a right-hand side: the stage kernel that follows adds them in
+// its epilogue and steps every field, and this kernel steps beta^i and expN
+// itself.  (auxB^i is stepped there, from the complete d_t Gamma^i.)  Against
+// the method sequence this saves the reads and writes of _c and the finalize
+// passes.
+//
+// Staging as in the stage kernels' LDS-DMA path (bssn_stage_kernel.h): 4x4x16
+// tiles of 256 threads, three LDS buffers, two arrays ahead.  Only beta needs
+// the full halo (mixed derivatives); every other array is differentiated along
+// the axes only and staged in three parts, each with the halo of one axis.
+// Two blocks of 4 waves per CU (57.6 KB of LDS, 2 waves per SIMD), where one
+// 512-thread block of the 8x8x8 tile left the CU idle at each of its barriers:
+// 0.297 ms per launch at 112^3, order 4, FP64, against 0.529 ms, and without
+// the 0.28 ms of the finalize passes.  Orders 2, 4 and 6 (halo 3), nz % 4 == 0.
+constexpr int TTI = 4, TTJ = 4, TTK = 16, TNT = TTI * TTJ * TTK, TH = 3, TKH = 4;
+template <typename E>
+__device__ __forceinline__ double el(const void* T, int c) {
+  return (double)reinterpret_cast<const E*>(T)[c];
+}
+template <int R, typename E>
+__device__ __forceinline__ double dax(const void* T, int c, int st) {
+  double acc = c1<R>(1) * (el<E>(T, c + st) - el<E>(T, c - st));
+#pragma unroll
+  for (int m = 2; m <= R; ++m) acc += c1<R>(m) * (el<E>(T, c + m * st) - el<E>(T, c - m * st));
+  return acc;
+}
+// `upwind` on a tile of either type; the reach of 3 is read in both directions
+// and the branch picks the stencil
+template <int R, typename E>
+__device__ __forceinline__ double upw(const void* T, int c, int st, double v, double i1) {
+  double w[7];
+#pragma unroll
+  for (int m = 0; m < 7; ++m) w[m] = el<E>(T, c + (m - 3) * st);
+  return upwind<R>(w, 3, 1, v, i1);
+}
+
+template <typename TS, int R>
+__global__ void __launch_bounds__(TNT) __attribute__((amdgpu_waves_per_eu(2))) k_gauge_terms(GaugeArgs a) {
+  constexpr bool ADV = R <= 2, F32 = sizeof(TS) == 4;
+  constexpr int KO = R == 1 ? 2 : 0;
+  constexpr int HI = TTI + 2 * TH, HJ = TTJ + 2 * TH, HK = TTK + 2 * TKH;
+  constexpr int HV = HI * HJ * HK, SI = HJ * HK, SJ = HK;
+  // axis-only parts
+  constexpr int AX = HI * TTJ * TTK, AY = TTI * HJ * TTK, AZ = TTI * TTJ * HK, AV = AX + AY + AZ;
+  constexpr int NW = TNT / 64;
+  constexpr int CF = (HV / 2 + 63) / 64, CA = (AV / 2 + 63) / 64, CQ = (AV / 4 + 63) / 64;  // 1 KB chunks
+  constexpr int MF = (CF + NW - 1) / NW, MA = (CA + NW - 1) / NW, MQ4 = (CQ + NW - 1) / NW;  // per wave
+  constexpr int BUF = CF * 1024;
+  static_assert(HV % 2 == 0 && AX % 4 == 0 && AY % 4 == 0 && AV % 4 == 0 && CA <= CF, "whole 16-byte groups");
+  __shared__ __align__(16) char lds[3 * BUF];
+
+  const int b = blockIdx.x, t = (b & 7) * a.per_xcd + (b >> 3);
+  if (t >= a.ntx * a.nty * a.ntz) return;
+  int tx, ty;
+  const int tz = t % a.ntz;
+  {  // strips of 4 tile rows along j, as the stage kernels' tile order 5
+    const int r = t / a.ntz, sidx = r / (4 * a.ntx), w = r - sidx * 4 * a.ntx;
+    const int wc = a.nty - sidx * 4 < 4 ? a.nty - sidx * 4 : 4;
+    ty = sidx * 4 + w % wc;
+    tx = w / wc;
+  }
+  const int i0 = tx * TTI, j0 = ty * TTJ, k0 = tz * TTK;
+  const int tid = threadIdx.x;
+  const int lk = tid % TTK, lj = (tid / TTK) % TTJ, li = tid / (TTK * TTJ);
+  const int px = i0 + li, py = j0 + lj, pz = k0 + lk;
+  const bool valid = px < a.nx && py < a.ny && pz < a.nz;
+  const unsigned idx = valid ? (unsigned)((px * a.ny + py) * a.nz + pz) : 0u;
+  const int c = ((li + TH) * HJ + (lj + TH)) * HK + (lk + TKH);
+  // the point in the three parts and their strides
+  const int ca[3] = {((li + TH) * TTJ + lj) * TTK + lk, AX + (li * HJ + lj + TH) * TTK + lk,
+                     AX + AY + (li * TTJ + lj) * HK + lk + TKH};
+  constexpr int sa[3] = {TTJ * TTK, TTK, 1};
+  const double i1 = a.inv_dx, i2 = a.inv_dx2;
+
+  // DMA offsets of this wave's chunks: element offset of each lane's group
+  // (surplus chunks repeat the last one, surplus lanes load element 0 into the
+  // padding)
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6), ln = tid & 63;
+  auto chunk = [&](int m, int n) { const int ch = wv + m * NW; return ch < n ? ch : n - 1; };
+  auto axis_off = [&](int e) -> unsigned {
+    if (e < AX) return box_off<TTK, TTJ>(e, i0 - TH, j0, k0, a.nx, a.ny, a.nz);
+    if (e < AX + AY) return box_off<TTK, HJ>(e - AX, i0, j0 - TH, k0, a.nx, a.ny, a.nz);
+    return box_off<HK, TTJ>(e - AX - AY, i0, j0, k0 - TKH, a.nx, a.ny, a.nz);
+  };
+  unsigned foff[MF], aoff[MA], qoff[F32 ? MQ4 : 1];
+#pragma unroll
+  for (int m = 0; m < MF; ++m) {
+    const int g = chunk(m, CF) * 64 + ln;
+    foff[m] = box_off<HK, HJ>(2 * (g < HV / 2 ? g : 0), i0 - TH, j0 - TH, k0 - TKH, a.nx, a.ny, a.nz);
+  }
+#pragma unroll
+  for (int m = 0; m < MA; ++m) {
+    const int g = chunk(m, CA) * 64 + ln;
+    aoff[m] = axis_off(2 * (g < AV / 2 ? g : 0));
+  }
+  if constexpr (F32) {
+#pragma unroll
+    for (int m = 0; m < MQ4; ++m) {
+      const int g = chunk(m, CQ) * 64 + ln;
+      qoff[m] = axis_off(4 * (g < AV / 4 ? g : 0));
+    }
+  }
+  typedef __attribute__((address_space(3))) char lds_char;
+  const unsigned lds0 = (unsigned)(size_t)(lds_char*)lds;
+  const int na = 10 + (a.need_phi ? 1 : 0);  // FP64 arrays: beta^1..3, expN, metric, [phi]
+  // array q of the sequence (as k_gauge_rhs) into buffer buf
+  auto dma = [&](int q, int buf) {
+    const unsigned dst = lds0 + (unsigned)buf * BUF;
+    if (q < 3) {
+      const void* src = a.xreg + ((long)(XBETA1 + q) * 4 + a.s_in) * a.rstride;
+#pragma unroll
+      for (int m = 0; m < MF; ++m) dma16(src, foff[m] * 8u, dst + chunk(m, CF) * 1024);
+    } else if (q < na || !F32) {
+      const int r = q - na, f = r < 0 ? 0 : ADV && r < 10 ? r : ALPHA - 7;
+      const void* src = q == 3   ? (const void*)(a.xreg + ((long)XEXPN * 4 + a.s_in) * a.rstride)
+                        : q < na ? (const void*)(a.met + ((long)(q - 4) * 4 + (q < 10 ? a.s_in_norm : a.s_in)) * a.rstride)
+                                 : (const void*)((const TS*)a.regs + ((long)f * 4 + (f < 6 ? a.s_in_norm : a.s_in)) * a.rstride);
+#pragma unroll
+      for (int m = 0; m < MA; ++m) dma16(src, aoff[m] * 8u, dst + chunk(m, CA) * 1024);
+    } else {
+      const int r = q - na, f = ADV && r < 10 ? r : ALPHA - 7;
+      const void* src = (const TS*)a.regs + ((long)f * 4 + (f < 6 ? a.s_in_norm : a.s_in)) * a.rstride;
+#pragma unroll
+      for (int m = 0; m < (F32 ? MQ4 : 1); ++m) dma16(src, qoff[m] * 4u, dst + chunk(m, CQ) * 1024);
+    }
+  };
+  // array k has landed for every wave; the one two ahead is issued into the
+  // buffer that was read before the barrier
+  int k = 0, bsel = 0;
+  const char* T = lds;
+  auto next = [&]() {
+    const int n = k + 1;  // at most its chunks are still outstanding
+    if (n >= a.nseq) dma_wait_barrier<0>();
+    else if (n < 3) dma_wait_barrier<MF>();
+    else if (n < na || !F32) dma_wait_barrier<MA>();
+    else dma_wait_barrier<MQ4>();
+    const int b2 = bsel == 0 ? 2 : bsel - 1;
+    if (k + 2 < a.nseq) dma(k + 2, b2);
+    T = lds + bsel * BUF;
+    bsel = bsel == 2 ? 0 : bsel + 1;
+    ++k;
+  };
+
+  auto met = [&](int f, int s) -> double* { return a.met + ((long)f * 4 + s) * a.rstride; };
+  auto reg = [&](int f, int s) -> TS* { return (TS*)a.regs + ((long)(f - 7) * 4 + s) * a.rstride; };
+  auto xr = [&](int q, int s) -> double* { return a.xreg + ((long)q * 4 + s) * a.rstride; };
+  auto stc = [&](int f, double x) {
+    if (!valid) return;
+    if (f < 7) sto(met(f, a.s_out), idx, x);
+    else sto(reg(f, a.s_out), idx, (TS)x);
+  };
+  // K{n}Finalize of a shift register (RK4Register.h:129-176)
+  auto step_x = [&](int q, double cc) {
+    if (!valid) return;
+    const double p = ldo((const double*)xr(q, a.s_p), idx);
+    const double fo = a.stage >= 2 ? ldo((const double*)xr(q, a.s_f), idx) : 0.0;
+    const double inc = a.cf * cc;
+    sto(xr(q, a.s_xout), idx, a.stage == 4 ? fo + (inc + p) : p + a.ca * cc);
+    if (a.stage != 4) sto(xr(q, a.s_f), idx, fo + inc);
+  };
+
+  // point values
+  double gm[6], am[6];
+#pragma unroll
+  for (int q = 0; q < 6; ++q) gm[q] = ldo((const double*)met(G11 + q, a.s_in_norm), idx);
+#pragma unroll
+  for (int q = 0; q < 6; ++q) am[q] = (double)ldo((const TS*)reg(A11 + q, a.s_in_norm), idx);
+  const double alpha = 1.0 + (double)ldo((const TS*)reg(ALPHA, a.s_in), idx),
+               K = (double)ldo((const TS*)reg(KK, a.s_in), idx) + a.K_F,
+               phi = ldo((const double*)met(PHI, a.s_in), idx) + a.phi_F;
+  const bool dw = a.shift == SHIFT_DAMPED_WAVE;
+  double gq[3] = {0, 0, 0}, bx[3] = {0, 0, 0};
+  if (dw)
+#pragma unroll
+    for (int I = 0; I < 3; ++I) gq[I] = (double)ldo((const TS*)reg(GAM1 + I, a.s_in), idx);
+  if (a.shift == SHIFT_GAMMA_DRIVER)
+#pragma unroll
+    for (int I = 0; I < 3; ++I) bx[I] = ldo((const double*)xr(XAUXB1 + I, a.s_in), idx);
+  dma(0, 0);
+  dma(1, 1);
+  // inverse conformal metric from the DIFF variables (bssn.cc:447-455)
+  double gi[6];
+  gi[0] = 1.0 + gm[3] + gm[5] - gm[4] * gm[4] + gm[3] * gm[5];
+  gi[3] = 1.0 + gm[0] + gm[5] - gm[2] * gm[2] + gm[0] * gm[5];
+  gi[5] = 1.0 + gm[0] + gm[3] - gm[1] * gm[1] + gm[0] * gm[3];
+  gi[1] = gm[2] * gm[4] - gm[1] * (1.0 + gm[5]);
+  gi[2] = gm[1] * gm[4] - gm[2] * (1.0 + gm[3]);
+  gi[4] = gm[1] * gm[2] - gm[4] * (1.0 + gm[0]);
+#pragma unroll
+  for (int q = 0; q < 6; ++q) {
+    pin(gi[q]);
+    pin(gm[q]);
+    pin(am[q]);
+  }
+  auto GI = [&](int p, int q) { return gi[sym(p, q)]; };
+  auto GM = [&](int p, int q) { return gm[sym(p, q)] + (p == q ? 1.0 : 0.0); };
+  auto AM = [&](int p, int q) { return am[sym(p, q)]; };
+  const double e4 = dw ? exp(-4.0 * phi) : 0.0;
+
+  // ---- beta^m (see k_gauge_rhs)
+  double bv[3], db[3][3], lapb[3], ddivb[3] = {0, 0, 0}, sh[3];
+#pragma unroll
+  for (int m = 0; m < 3; ++m) {
+    next();
+    const double* L = reinterpret_cast<const double*>(T);
+    bv[m] = L[c];
+    db[0][m] = fd1<R>(L, c, SI) * i1;
+    db[1][m] = fd1<R>(L, c, SJ) * i1;
+    db[2][m] = fd1<R>(L, c, 1) * i1;
+    double h[6];
+    h[0] = fd2<R>(L, c, SI) * i2;
+    h[3] = fd2<R>(L, c, SJ) * i2;
+    h[5] = fd2<R>(L, c, 1) * i2;
+    h[1] = fdm<R>(L, c, SI, SJ) * i2;
+    h[2] = fdm<R>(L, c, SI, 1) * i2;
+    h[4] = fdm<R>(L, c, SJ, 1) * i2;
+    lapb[m] = gi[0] * h[0] + gi[3] * h[3] + gi[5] * h[5] + 2.0 * (gi[1] * h[1] + gi[2] * h[2] + gi[4] * h[4]);
+#pragma unroll
+    for (int j = 0; j < 3; ++j) ddivb[j] += h[sym(m, j)];
+    sh[m] = -(a.ko_pref * ko_sum<KO, double>(L, c, SI, SJ, 1));
+    pin(sh[m]);
+    pin(lapb[m]);
+    pin(bv[m]);
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      pin(db[j][m]);
+      pin(ddivb[j]);
+    }
+  }
+  double divb = db[0][0] + db[1][1] + db[2][2];
+  pin(divb);
+  double gx[3];
+#pragma unroll
+  for (int I = 0; I < 3; ++I) {
+    gx[I] = lapb[I] + (1.0 / 3.0) * (GI(I, 0) * ddivb[0] + GI(I, 1) * ddivb[1] + GI(I, 2) * ddivb[2]);
+    pin(gx[I]);
+  }
+#pragma unroll
+  for (int I = 0; I < 3; ++I) {
+    if (a.shift == SHIFT_GAMMA_DRIVER) {
+      sh[I] += bx[I];
+    } else if (dw) {
+      sh[I] += bv[0] * db[0][I] + bv[1] * db[1][I] + bv[2] * db[2][I] - a.dw_mu_s * alpha * bv[I] +
+               alpha * (-a.dw_mu_l * (12.0 * phi * a.dw_p - log(alpha)) * bv[I]);
+    } else if (a.shift == SHIFT_AWA_SHIFTED_WAVE) {
+      sh[I] += a.wave_dir == I + 1 ? -2.0 * K * alpha : 0.0;
+    }
+    pin(sh[I]);
+  }
+
+  // ---- expN (bssn.cc:871-875)
+  next();
+  step_x(XEXPN, bv[0] * dax<R, double>(T, ca[0], sa[0]) * i1 + bv[1] * dax<R, double>(T, ca[1], sa[1]) * i1 +
+                    bv[2] * dax<R, double>(T, ca[2], sa[2]) * i1 - alpha * K / 3.0);
+
+  auto adv64 = [&]() -> double {
+    return upw<R, double>(T, ca[0], sa[0], bv[0], i1) + upw<R, double>(T, ca[1], sa[1], bv[1], i1) +
+           upw<R, double>(T, ca[2], sa[2], bv[2], i1);
+  };
+  auto advs = [&]() -> double {
+    return upw<R, TS>(T, ca[0], sa[0], bv[0], i1) + upw<R, TS>(T, ca[1], sa[1], bv[1], i1) +
+           upw<R, TS>(T, ca[2], sa[2], bv[2], i1);
+  };
+
+  // ---- metric (bssn_macros.h:292-312) and Gd^I
+  double Gd[3] = {0, 0, 0};
+#pragma unroll
+  for (int p = 0; p < 3; ++p)
+#pragma unroll
+    for (int q = p; q < 3; ++q) {
+      next();
+      double d[3];
+#pragma unroll
+      for (int x = 0; x < 3; ++x) d[x] = dax<R, double>(T, ca[x], sa[x]) * i1;
+      const double w = p == q ? 0.5 : 1.0;
+#pragma unroll
+      for (int I = 0; I < 3; ++I) {
+        double tt = -w * GI(p, q) * (GI(I, 0) * d[0] + GI(I, 1) * d[1] + GI(I, 2) * d[2]);
+#pragma unroll
+        for (int m = 0; m < 3; ++m) tt += d[m] * (GI(m, p) * GI(I, q) + (p != q ? GI(m, q) * GI(I, p) : 0.0));
+        Gd[I] += tt;
+        pin(Gd[I]);
+      }
+      double cv = 0.0;
+      if constexpr (ADV) cv = adv64();
+      cv += GM(p, 0) * db[q][0] + GM(p, 1) * db[q][1] + GM(p, 2) * db[q][2] + GM(q, 0) * db[p][0] +
+            GM(q, 1) * db[p][1] + GM(q, 2) * db[p][2] - (2.0 / 3.0) * GM(p, q) * divb;
+      stc(G11 + sym(p, q), cv);
+    }
+
+  // ---- phi (bssn.cc:806-812)
+  {
+    double cv = (1.0 / 6.0) * divb;
+    if (a.need_phi) {
+      next();
+      if constexpr (ADV) cv += adv64();
+      if (dw) {
+        double d[3];
+#pragma unroll
+        for (int x = 0; x < 3; ++x) d[x] = dax<R, double>(T, ca[x], sa[x]) * i1;
+#pragma unroll
+        for (int I = 0; I < 3; ++I)
+          sh[I] += -2.0 * alpha * alpha * e4 * (GI(I, 0) * d[0] + GI(I, 1) * d[1] + GI(I, 2) * d[2]);
+      }
+    }
+    stc(PHI, cv);
+  }
+
+  // ---- A_ij (bssn_macros.h:313-333)
+#pragma unroll
+  for (int p = 0; p < 3; ++p)
+#pragma unroll
+    for (int q = p; q < 3; ++q) {
+      double cv = 0.0;
+      if constexpr (ADV) {
+        next();
+        cv = advs();
+      }
+      cv += AM(p, 0) * db[q][0] + AM(p, 1) * db[q][1] + AM(p, 2) * db[q][2] + AM(q, 0) * db[p][0] +
+            AM(q, 1) * db[p][1] + AM(q, 2) * db[p][2] - (2.0 / 3.0) * AM(p, q) * divb;
+      stc(A11 + sym(p, q), cv);
+    }
+
+  // ---- DIFFK
+  if constexpr (ADV) {
+    next();
+    stc(KK, advs());
+  }
+
+  // ---- Gt^i (bssn_macros.h:363-382); DampedWaveShift2 reads Gt^3 where Gt^2
+  // is meant (BSSNGaugeHandler.cc:185), kept
+#pragma unroll
+  for (int I = 0; I < 3; ++I) {
+    double cv = 0.0;
+    if constexpr (ADV) {
+      next();
+      cv = advs();
+    }
+    cv += -Gd[0] * db[0][I] - Gd[1] * db[1][I] - Gd[2] * db[2][I] + (2.0 / 3.0) * Gd[I] * divb + gx[I];
+    stc(GAM1 + I, cv);
+    if (dw) {
+      const double tt = alpha * alpha * e4 * gq[I];
+      if (I == 0) sh[0] += tt;
+      if (I == 2) { sh[1] += tt; sh[2] += tt; }
+    }
+  }
+
+  // ---- the lapse: beta.d alpha in OnePlusLog and DampedWave
+  // (BSSNGaugeHandler.cc:64-68, 151-155)
+  if (a.live_alpha) {
+    double cv = 0.0;
+    if (a.need_alpha) {
+      next();
+      double d[3];
+#pragma unroll
+      for (int x = 0; x < 3; ++x) d[x] = dax<R, TS>(T, ca[x], sa[x]) * i1;
+      if (a.lapse == LAPSE_ONE_PLUS_LOG || a.lapse == LAPSE_DAMPED_WAVE) cv = bv[0] * d[0] + bv[1] * d[1] + bv[2] * d[2];
+      if constexpr (ADV) cv += advs();
+      if (dw)
+#pragma unroll
+        for (int I = 0; I < 3; ++I) sh[I] += -alpha * e4 * (GI(I, 0) * d[0] + GI(I, 1) * d[1] + GI(I, 2) * d[2]);
+    }
+    stc(ALPHA, cv);
+  }
+
+  // ---- d_t beta^i (bssn.cc:852-869)
+#pragma unroll
+  for (int I = 0; I < 3; ++I) step_x(XBETA1 + I, sh[I]);
+}
+
 // TestKDriverLapse without the shift build: d_t alpha gains
 // -k ((d_t K - (K_avg^2/3 + 4 pi rho_avg)) + (K - K_avg)) (BSSNGaugeHandler.cc:93-102),
 // which reads the complete d_t DIFFK; nothing else changes
@@ -468,6 +845,75 @@ int launch_gauge_order(int order, const GaugeArgs& g, hipStream_t s) {
 
 }  // namespace
 
+static GaugeArgs gauge_args(cg_ctx* c, int s_in, int s_out) {
+  GaugeArgs g{};
+  g.met = c->met;
+  g.regs = c->regs;
+  g.xreg = c->xreg;
+  g.rstride = c->rstride;
+  g.s_in = s_in;
+  g.s_out = s_out;
+  g.nx = c->p.nx; g.ny = c->p.ny; g.nz = c->p.nz;
+  g.inv_dx = 1.0 / c->p.dx;
+  g.inv_dx2 = 1.0 / (c->p.dx * c->p.dx);
+  const double dx = c->p.dx, ko = c->p.ko_coeff;
+  // KO_dissipation_Q (math.h:36-72): ko*dx^3/64 * sum/dx^4 ; -ko*dx^9/1024 * sum/dx^10
+  g.ko_pref = c->p.stencil_order == 2 ? ko / (64.0 * dx) : c->p.stencil_order == 8 ? -ko / (1024.0 * dx) : 0.0;
+  g.shift = c->p.shift; g.lapse = c->p.lapse; g.nxf = c->nxf; g.wave_dir = c->gauge_wave_dir;
+  g.gd_eta = c->gd_eta; g.dw_mu_s = c->dw_mu_s; g.dw_mu_l = c->dw_mu_l; g.dw_p = c->dw_p; g.k_driver = c->k_driver;
+  g.phi_F = c->frw.g_phi; g.K_F = c->frw.g_K;
+  g.ext = c->ext;
+  // the staging sequence, in the kernels' order: beta^1..3, expN, the
+  // metric, then phi, A_ij, K, Gt^i and alpha where their derivatives or
+  // their advection are needed (advection only at orders 2 and 4)
+  const bool adv = c->p.stencil_order <= 4;
+  const bool dw = c->p.shift == SHIFT_DAMPED_WAVE;
+  g.need_phi = adv || dw;
+  g.need_alpha = adv || dw || c->p.lapse == LAPSE_ONE_PLUS_LOG || c->p.lapse == LAPSE_DAMPED_WAVE;
+  g.nseq = 4 + 6 + (g.need_phi ? 1 : 0) + (adv ? 10 : 0) + (g.need_alpha ? 1 : 0);
+  return g;
+}
+
+bool gauge_fusable(const cg_ctx* c) {
+  // AijDriverShift and TestKDriverLapse read other fields' complete
+  // right-hand sides, which no slot holds in the fused steps
+  if (!c->nxf || c->p.shift == CG_SHIFT_AIJ_DRIVER || c->p.lapse == LAPSE_TEST_K_DRIVER) return false;
+  // k_gauge_terms: its halo of 3 (KO of beta at order 8 needs 5), whole
+  // 16-byte groups along k, one wrap per axis, 24-bit offsets (the 32-bit byte
+  // offsets follow from cg_create's bound on the grid)
+  if (c->p.stencil_order > 6 || !c->dma_allowed) return false;
+  return c->p.nz % 4 == 0 && c->p.nz > TTK + TKH - 2 && c->p.nx > TTI + TH - 2 && c->p.ny > TTJ + TH - 2 &&
+         (long long)c->p.nx * c->p.ny < (1ll << 24);
+}
+
+int gauge_terms(cg_ctx* c, const StageArgs& st) {
+  GaugeArgs g = gauge_args(c, st.s_in, st.s_add);
+  g.phi_F = st.phi_F; g.K_F = st.K_F;
+  g.ntx = (c->p.nx + TTI - 1) / TTI; g.nty = (c->p.ny + TTJ - 1) / TTJ; g.ntz = (c->p.nz + TTK - 1) / TTK;
+  const int tiles = g.ntx * g.nty * g.ntz;
+  g.per_xcd = (tiles + 7) / 8;
+  g.s_in_norm = st.s_in_norm >= 0 ? st.s_in_norm : st.s_in;
+  g.s_p = st.s_p; g.s_f = st.s_f; g.s_xout = st.s_out; g.stage = st.stage;
+  g.cf = st.cf; g.ca = st.ca;
+  g.live_alpha = alpha_live(c) ? 1 : 0;
+  if (!g.live_alpha && g.need_alpha && c->p.shift != SHIFT_DAMPED_WAVE) {
+    g.need_alpha = 0;  // a lapse identically 1: nothing to advect
+    g.nseq -= 1;
+  }
+  auto go = [&](auto ts, auto r) {
+    hipLaunchKernelGGL((k_gauge_terms<decltype(ts), decltype(r)::value>), dim3(8 * g.per_xcd), dim3(TNT), 0, c->stream, g);
+  };
+  auto order = [&](auto ts) {
+    if (c->p.stencil_order == 2) go(ts, std::integral_constant<int, 1>{});
+    else if (c->p.stencil_order == 4) go(ts, std::integral_constant<int, 2>{});
+    else go(ts, std::integral_constant<int, 3>{});
+  };
+  if (c->prec == CG_FP64) order(double());
+  else order(float());
+  HIPCHK(c, hipGetLastError());
+  return CG_OK;
+}
+
 int gauge_rhs(cg_ctx* c, int s_in, int s_out) {
   const bool f32 = c->prec != CG_FP64;
   const size_t w = f32 ? sizeof(float) : sizeof(double);
@@ -489,32 +935,8 @@ int gauge_rhs(cg_ctx* c, int s_in, int s_out) {
     HIPCHK(c, hipGetLastError());
     return CG_OK;
   }
-  GaugeArgs g{};
-  g.met = c->met;
-  g.regs = c->regs;
-  g.xreg = c->xreg;
-  g.rstride = c->rstride;
-  g.s_in = s_in;
-  g.s_out = s_out;
-  g.nx = c->p.nx; g.ny = c->p.ny; g.nz = c->p.nz;
+  GaugeArgs g = gauge_args(c, s_in, s_out);
   g.ntx = (c->p.nx + GT - 1) / GT; g.nty = (c->p.ny + GT - 1) / GT; g.ntz = (c->p.nz + GT - 1) / GT;
-  g.inv_dx = 1.0 / c->p.dx;
-  g.inv_dx2 = 1.0 / (c->p.dx * c->p.dx);
-  const double dx = c->p.dx, ko = c->p.ko_coeff;
-  // KO_dissipation_Q (math.h:36-72): ko*dx^3/64 * sum/dx^4 ; -ko*dx^9/1024 * sum/dx^10
-  g.ko_pref = c->p.stencil_order == 2 ? ko / (64.0 * dx) : c->p.stencil_order == 8 ? -ko / (1024.0 * dx) : 0.0;
-  g.shift = c->p.shift; g.lapse = c->p.lapse; g.nxf = c->nxf; g.wave_dir = c->gauge_wave_dir;
-  g.gd_eta = c->gd_eta; g.dw_mu_s = c->dw_mu_s; g.dw_mu_l = c->dw_mu_l; g.dw_p = c->dw_p; g.k_driver = c->k_driver;
-  g.phi_F = c->frw.g_phi; g.K_F = c->frw.g_K;
-  g.ext = c->ext;
-  // the staging sequence, in the kernel's order: beta^1..3, expN, the
-  // metric, then phi, A_ij, K, Gt^i and alpha where their derivatives or
-  // their advection are needed (advection only at orders 2 and 4)
-  const bool adv = c->p.stencil_order <= 4;
-  const bool dw = c->p.shift == SHIFT_DAMPED_WAVE;
-  g.need_phi = adv || dw;
-  g.need_alpha = adv || dw || c->p.lapse == LAPSE_ONE_PLUS_LOG || c->p.lapse == LAPSE_DAMPED_WAVE;
-  g.nseq = 4 + 6 + (g.need_phi ? 1 : 0) + (adv ? 10 : 0) + (g.need_alpha ? 1 : 0);
   int rc = f32 ? launch_gauge_order<float>(c->p.stencil_order, g, c->stream)
                : launch_gauge_order<double>(c->p.stencil_order, g, c->stream);
   if (rc) return fail(c, CG_ERR_HIP, std::string("gauge pass: ") + hipGetErrorString((hipError_t)rc));

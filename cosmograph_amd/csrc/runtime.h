@@ -105,6 +105,7 @@ struct cg_ctx {
   int R = 2, H = 2;
   int req_ti = 0, req_tj = 0, req_tk = 0;  // requested tile (0 = automatic)
   const StageVariant* var = nullptr;     // stage kernel in use
+  const StageVariant* svar = nullptr;    // ... of the shift build's fused steps
   // tile traversal order (autotuned).  Default: strips of 4 tile rows along
   // j, the fastest or within 2% of it on every grid from 64^3 up (256^3 fixed
   // point 1.63 ms per stage against 1.70 in order 0)
@@ -211,6 +212,11 @@ const void* field_ptr(cg_ctx* c, const char* name, size_t* esz, int* err);
 // that read the complete right-hand side of other fields
 inline bool gauge_pass(const cg_ctx* c) { return c->nxf > 0 || c->p.lapse == LAPSE_TEST_K_DRIVER; }
 int gauge_rhs(cg_ctx* c, int s_in, int s_out);  // after the stage kernel's RHS into s_out: adds to it, fills the shift s_out
+// fused steps of the shift build: whether this context's gauge and grid have
+// them, and the gauge pass of the stage whose arguments are given (terms into
+// slot st.s_add, beta^i and expN stepped)
+bool gauge_fusable(const cg_ctx* c);
+int gauge_terms(cg_ctx* c, const StageArgs& st);
 int gauge_step_init(cg_ctx* c);           // RK4Register::stepInit of the shift registers
 int gauge_finalize(cg_ctx* c, int n);     // RK4Register::K{n}Finalize of the shift registers (no swap)
 // the register the output step's passes read (stepInit's _a, materialised

@@ -132,11 +132,13 @@ struct StageArgs {
   const double* cons_means;
   int cons_pass;
   int tile_base, tile_count;
-  // fixed-point metric (MODE_MQ): scale 2^e and its inverse of field f < 7,
-  // the scale times 1/dx and 1/dx^2 rounded to FP32 (the stencils' factors),
+  // fixed-point metric (MODE_MQ): exponent e of field f < 7 (value = word 2^e),
+  // the factors of the stencils' sums, rounded to FP32: scale times weight
+  // times 1/dx or 1/dx^2 of the first, pure second and mixed derivatives (of
+  // DIFFgamma_ij, the last two times -1/2 and -1, as they enter the Ricci tensor),
   // and the count of saturated words
-  double msc[7], minv[7];
-  float msd1[7], msd2[7];
+  int mexp[7];
+  float msd1[7], msd2[7], msdm[7];
   // shift build, fused stages (MODE_SHIFT): the gauge pass's terms of every
   // field's right-hand side lie in slot s_add, at this point read before
   // anything is written there; with the Gamma driver the auxB^i registers

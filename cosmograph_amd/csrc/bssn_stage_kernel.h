@@ -213,10 +213,13 @@ template <int RK, int RJ>
 __device__ __forceinline__ unsigned box_off(int e, int x0, int y0, int z0, int nx, int ny, int nz) {
   const unsigned r = div13<RK>((unsigned)e), hi = div13<RJ>(r);
   int x = x0 + (int)hi, y = y0 + (int)(r - (unsigned)__umul24(hi, RJ)), z = z0 + (int)((unsigned)e - (unsigned)__umul24(r, RK));
-  x += x < 0 ? nx : 0; x -= x >= nx ? nx : 0;
-  y += y < 0 ? ny : 0; y -= y >= ny ? ny : 0;
-  z += z < 0 ? nz : 0; z -= z >= nz ? nz : 0;
-  return (unsigned)__umul24((unsigned)__umul24(x, ny) + y, nz) + (unsigned)z;
+  // unsigned minima: of x and x + n the one in range is the smaller for
+  // x < 0 (x wraps to a large value), of x and x - n for x >= n
+  auto wrap = [](int v, int n) -> unsigned {
+    const unsigned u = min((unsigned)v, (unsigned)v + (unsigned)n);
+    return min(u, u - (unsigned)n);
+  };
+  return (unsigned)__umul24((unsigned)__umul24(wrap(x, nx), ny) + wrap(y, ny), nz) + wrap(z, nz);
 }
 
 // End of one step of the DMA staging: this wave's vector memory operations
@@ -243,6 +246,9 @@ __device__ __forceinline__ void morton_xy(int m, int lx, int ly, int& x, int& y)
   const int hi = m >> (2 * l);
   if (lx > ly) x |= hi << l; else y |= hi << l;
 }
+
+// kinds of the stage kernel's epilogue (stage_body)
+enum { EP_RHS, EP_INC, EP_INC4, EP_ACC1, EP_ACC, EP_ACC4 };
 
 // WPE: minimum waves per SIMD the register allocation must allow.
 // LIVE_ALPHA = false: synchronous gauge with DIFFalpha identically zero (Static
@@ -380,7 +386,13 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
 
   const int tid = threadIdx.x;
   __builtin_assume(tid >= 0 && tid < NT);
-  const int lk = tid % TK, lj = (tid / TK) % TJ, li = tid / (TK * TJ);
+  // Point of a thread.  On 4x4x16 tiles of 4-byte words the halo rows are 24
+  // words apart, so the two rows of 16 lanes that one LDS cycle serves would
+  // meet in 8 of the 32 banks (818 conflict cycles per wave of 3200); with rows
+  // j and j + 2 in one half of the wave they are 16 banks apart instead.
+  constexpr bool JPERM = DMA && M32 && TJ == 4 && TK == 16 && HK4 % 32 == 24;
+  auto row_j = [](int r) { return JPERM ? (r & 1) * 2 + (r >> 1) : r; };  // 0, 2, 1, 3
+  const int lk = tid % TK, lj = row_j((tid / TK) % TJ), li = tid / (TK * TJ);
   const int px = i0 + li, py = j0 + lj, pz = k0 + lk;
   const bool valid = (px < a.nx) && (py < a.ny) && (pz < a.nz);
   const unsigned idx = valid ? (unsigned)((px * a.ny + py) * a.nz + pz) : 0u;
@@ -419,6 +431,10 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
     }
   };
 
+  // the fixed-point metric's scales 2^e and 2^-e, formed where they are used:
+  // held as doubles they are 28 SGPRs that spill into VGPR lanes
+  auto msc = [&](int f) { return __hiloint2double((a.mexp[f] + 1023) << 20, 0); };
+  auto minv = [&](int f) { return __hiloint2double((1023 - a.mexp[f]) << 20, 0); };
   auto RM = [&](int f, int slot) -> double* { return a.met + ((long)f * 4 + slot) * a.rstride; };
   auto RS = [&](int f, int slot) -> TS* { return (TS*)a.regs + ((long)(f - 7) * 4 + slot) * a.rstride; };
   // stencil / point input of field f: DIFFgamma_ij and A_ij come from the
@@ -446,8 +462,8 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
           for (int m = 0; m < 6; ++m) {
             TS g0, g1;
             pair(INS(G11 + m), q, g0, g1);
-            g[m][0] = MQ ? (double)__float_as_int(g0) * a.msc[G11 + m] : (double)g0;
-            g[m][1] = MQ ? (double)__float_as_int(g1) * a.msc[G11 + m] : (double)g1;
+            g[m][0] = MQ ? (double)__float_as_int(g0) * msc(G11 + m) : (double)g0;
+            g[m][1] = MQ ? (double)__float_as_int(g1) * msc(G11 + m) : (double)g1;
           }
         } else {
 #pragma unroll
@@ -499,7 +515,7 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
         if (pp < HP) {
           if (MQ && !MQW && f < 7) {
             // FP64 compute: the scaled values (normalised at stage 1)
-            const double sc = a.msc[f < 7 ? f : 0];
+            const double sc = msc(f < 7 ? f : 0);
             double w0 = (double)__float_as_int(pf[q][0]) * sc, w1 = (double)__float_as_int(pf[q][1]) * sc;
             if (norm && f <= G33) {
               const double t0 = ldn[2 * pp], t1 = ldn[2 * pp + 1];
@@ -510,7 +526,7 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
             dst[2 * pp + 1] = (TC)w1;
           } else if (MQW && norm && f <= G33) {
             // the normalised halo value, back in the field's fixed point
-            const double t0 = ldn[2 * pp], t1 = ldn[2 * pp + 1], sc = a.msc[f < 7 ? f : 0], iv = a.minv[f < 7 ? f : 0];
+            const double t0 = ldn[2 * pp], t1 = ldn[2 * pp + 1], sc = msc(f < 7 ? f : 0), iv = minv(f < 7 ? f : 0);
             const double w0 = ((double)__float_as_int(pf[q][0]) * sc + (diag6(f) ? t0 : 0.0)) / (1.0 - t0);
             const double w1 = ((double)__float_as_int(pf[q][1]) * sc + (diag6(f) ? t1 : 0.0)) / (1.0 - t1);
             if (fmax(fabs(w0), fabs(w1)) * iv > MQ_WMAX) atomicAdd(a.mq_sat, 1u);
@@ -534,10 +550,10 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
   double gc[7];  // metric at the point in FP64 (DIFFgamma_ij, DIFFphi)
 #pragma unroll
   for (int f = 0; f < 6; ++f)  // idx = 0 outside the grid
-    gc[f] = MQ    ? (double)ldo((const int*)INS(f), idx) * a.msc[f]
+    gc[f] = MQ    ? (double)ldo((const int*)INS(f), idx) * msc(f)
             : M32 ? (double)ldo(INS(f), idx)
                   : ldo(INM(f), idx);
-  const double phi_c = MQ    ? (double)ldo((const int*)INS(PHI), idx) * a.msc[PHI]
+  const double phi_c = MQ    ? (double)ldo((const int*)INS(PHI), idx) * msc(PHI)
                        : M32 ? (double)ldo(INS(PHI), idx)
                              : ldo(INM(PHI), idx);
   gc[6] = phi_c;
@@ -626,7 +642,7 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
 
   // ------------------------------------------------ stencil phase (LDS)
   const double i1 = a.inv_dx, i2 = a.inv_dx2;
-  const TC idx1 = (TC)a.inv_dx;
+  const TC idx1 = (TC)a.inv_dx, idx1n = (TC)(a.inv_dx * c1<R>(1));  // with fd1, fd1n
   TC dg[3][6];      // d_k gamma_ij
   // conformal Ricci tensor, accumulated as its inputs arrive:
   // -1/2 gamma^{kl} d_k d_l gamma_ij per metric field, the d_j Gamma^k terms
@@ -699,7 +715,7 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
   // algebra after the last field, the FP64 kernel held 256 VGPRs and spilled
   // 188 B (0.421 ms per stage at 128^3, order 4; now 242, no spill, 0.285
   // ms), the fixed-point one 157 (1.62 ms at 256^3, order 6; now 126, four
-  // waves, 1.535 ms).
+  // waves).
   TC GL[3][6], G[3][6], Gd[3];
   TC Ac[6], AijAij = TC(0), second[3];  // A^ij, A_ij A^ij, Gamma^i_jk A^jk + 6 A^ij d_j phi
   TC DDa[6], DDaTR = TC(0);             // (D_i D_j alpha)^TF and its trace (without e^{-4 phi})
@@ -880,23 +896,25 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
       const int* __restrict__ LQ = reinterpret_cast<const int*>(BUF);                                                    \
       if (KO_ORDER && f < NF) {                                                                                \
         if (MQW && (f <= G33 || f == PHI))                                                                               \
-          ko[f] = (TC)(a.ko_pref * a.msc[f < 7 ? f : 0] * ko_sumq<KO_ORDER>(LQ, c4, SI4, SJ4, SK));                      \
+          ko[f] = (TC)(a.ko_pref * msc(f < 7 ? f : 0) * ko_sumq<KO_ORDER>(LQ, c4, SI4, SJ4, SK));                      \
         else                                                                                                             \
           ko[f] = (TC)a.ko_pref * ko_sum<KO_ORDER, TC>(L, c4, SI4, SJ4, SK);                                             \
       }                                                                                                                  \
       if (MQW && (f <= G33 || f == PHI)) {                                                                               \
         /* exact integer differences of the words, FP32 sums, the field's scale */                                      \
-        const TC s1 = a.msd1[f < 7 ? f : 0], s2 = a.msd2[f < 7 ? f : 0];                                                \
+        const TC s1 = a.msd1[f < 7 ? f : 0], s2 = a.msd2[f < 7 ? f : 0], sm = a.msdm[f < 7 ? f : 0];                     \
         const TC d0 = fd1qf<R>(LQ, c4, SI4) * s1, d1 = fd1qf<R>(LQ, c4, SJ4) * s1, d2 = fd1qf<R>(LQ, c4, SK) * s1;       \
-        const TC e00 = fd2qf<R>(LQ, c4, SI4) * s2, e11 = fd2qf<R>(LQ, c4, SJ4) * s2, e22 = fd2qf<R>(LQ, c4, SK) * s2;    \
-        const TC e01 = fdmqf<R>(LQ, c4, SI4, SJ4) * s2, e02 = fdmqf<R>(LQ, c4, SI4, SK) * s2,                           \
-                 e12 = fdmqf<R>(LQ, c4, SJ4, SK) * s2;                                                                   \
+        const TC e00 = fd2qf<R>(LQ, c4, SI4), e11 = fd2qf<R>(LQ, c4, SJ4), e22 = fd2qf<R>(LQ, c4, SK);                   \
+        const TC e01 = fdmqf<R>(LQ, c4, SI4, SJ4), e02 = fdmqf<R>(LQ, c4, SI4, SK), e12 = fdmqf<R>(LQ, c4, SJ4, SK);     \
         if (f == PHI) {                                                                                                  \
           dphi[0] = d0; dphi[1] = d1; dphi[2] = d2;                                                                      \
-          ddphi[0] = e00; ddphi[1] = e01; ddphi[2] = e02; ddphi[3] = e11; ddphi[4] = e12; ddphi[5] = e22;                \
+          ddphi[0] = e00 * s2; ddphi[1] = e01 * sm; ddphi[2] = e02 * sm;                                                 \
+          ddphi[3] = e11 * s2; ddphi[4] = e12 * sm; ddphi[5] = e22 * s2;                                                 \
         } else {                                                                                                         \
           dg[0][f] = d0; dg[1][f] = d1; dg[2][f] = d2;                                                                   \
-          add_lap(f, e00, e01, e02, e11, e12, e22);                                                                      \
+          /* -1/2 of the scaled contraction: the factors of the gamma_ij hold the -1/2 and the 2 of the mixed terms */    \
+          ric[f < 6 ? f : 0] += s2 * (gi[0] * e00 + gi[3] * e11 + gi[5] * e22);                                          \
+          ric[f < 6 ? f : 0] += sm * (gi[1] * e01 + gi[2] * e02 + gi[4] * e12);                                          \
         }                                                                                                                \
       } else if (M32 && (f <= G33 || f == PHI)) {                                                                        \
         const TC idx2 = (TC)a.inv_dx2;                                                                                   \
@@ -918,9 +936,9 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
         ddal[1] = fdm<R>(L, c4, SI4, SJ4) * idx2; ddal[2] = fdm<R>(L, c4, SI4, SK) * idx2;                               \
         ddal[4] = fdm<R>(L, c4, SJ4, SK) * idx2;                                                                         \
       } else if (f == KK) {                                                                                              \
-        dK[0] = fd1<R>(L, c4, SI4) * idx1; dK[1] = fd1<R>(L, c4, SJ4) * idx1; dK[2] = fd1<R>(L, c4, SK) * idx1;          \
+        dK[0] = fd1n<R>(L, c4, SI4) * idx1n; dK[1] = fd1n<R>(L, c4, SJ4) * idx1n; dK[2] = fd1n<R>(L, c4, SK) * idx1n;          \
       } else if (f >= GAM1 && f <= GAM3) {                                                                               \
-        add_dG(f - GAM1, fd1<R>(L, c4, SI4) * idx1, fd1<R>(L, c4, SJ4) * idx1, fd1<R>(L, c4, SK) * idx1);                \
+        add_dG(f - GAM1, fd1n<R>(L, c4, SI4) * idx1n, fd1n<R>(L, c4, SJ4) * idx1n, fd1n<R>(L, c4, SK) * idx1n);                \
       } else if (CONS && f >= A11 && f <= A33) {                                                                         \
         const int q = f - A11;                                                                                           \
         add_dA(q, fd1<R>(L, c4, SI4) * idx1, fd1<R>(L, c4, SJ4) * idx1, fd1<R>(L, c4, SK) * idx1);                       \
@@ -930,9 +948,9 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
         const int cz = FGX + FGY + (li * TJ + lj) * HK4 + lk + KH4;                                                      \
         TC dd[2][3];                                                                                                     \
         _Pragma("unroll") for (int h = 0; h < 2; ++h) {                                                                  \
-          dd[h][0] = fd1<R>(L, h * (FGX + FGY + FGZ) + cx, TJ * TK) * idx1;                                              \
-          dd[h][1] = fd1<R>(L, h * (FGX + FGY + FGZ) + cy, TK) * idx1;                                                   \
-          dd[h][2] = fd1<R>(L, h * (FGX + FGY + FGZ) + cz, 1) * idx1;                                                    \
+          dd[h][0] = fd1n<R>(L, h * (FGX + FGY + FGZ) + cx, TJ * TK) * idx1n;                                              \
+          dd[h][1] = fd1n<R>(L, h * (FGX + FGY + FGZ) + cy, TK) * idx1n;                                                   \
+          dd[h][2] = fd1n<R>(L, h * (FGX + FGY + FGZ) + cz, 1) * idx1n;                                                    \
         }                                                                                                                \
         if (f == KG0) {                                                                                                  \
           _Pragma("unroll") for (int d = 0; d < 3; ++d) dK[d] = dd[0][d];                                               \
@@ -944,13 +962,13 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
       } else if (FGRP && f >= FLUXG0) {                                                                                  \
         /* the three fluxes of quantity q, each along its own axis, summed in the order x, y, z */                       \
         const int q = f - FLUXG0;                                                                                        \
-        ddust[q] += fd1<R>(L, ((li + H) * TJ + lj) * TK + lk, TJ * TK) * idx1;                                           \
-        ddust[q] += fd1<R>(L, FGX + (li * HJ + lj + H) * TK + lk, TK) * idx1;                                            \
-        ddust[q] += fd1<R>(L, FGX + FGY + (li * TJ + lj) * HK4 + lk + KH4, 1) * idx1;                                    \
+        ddust[q] += fd1n<R>(L, ((li + H) * TJ + lj) * TK + lk, TJ * TK) * idx1n;                                           \
+        ddust[q] += fd1n<R>(L, FGX + (li * HJ + lj + H) * TK + lk, TK) * idx1n;                                            \
+        ddust[q] += fd1n<R>(L, FGX + FGY + (li * TJ + lj) * HK4 + lk + KH4, 1) * idx1n;                                    \
       } else if (FLUXES && f >= FLUX0) {                                                                                 \
         /* dust.cc:203-224: flux q*3 + i is differentiated along i only */                                               \
         const int q = (f - FLUX0) / 3, dir = (f - FLUX0) % 3;                                                            \
-        ddust[q] += fd1<R>(L, c4, dir == 0 ? SI4 : dir == 1 ? SJ4 : SK) * idx1;                                          \
+        ddust[q] += fd1n<R>(L, c4, dir == 0 ? SI4 : dir == 1 ? SJ4 : SK) * idx1n;                                          \
       }                                                                                                                  \
     }
 
@@ -1104,7 +1122,7 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
         // for them (vmcnt) before its epilogue, while the algebra runs.
         dma_wait_barrier<0>();
         auto poff = [&](int q) -> unsigned {  // element offset of block point q, 0 outside the grid
-          const int qk = q % TK, qj = (q / TK) % TJ, qi = q / (TK * TJ);
+          const int qk = q % TK, qj = row_j((q / TK) % TJ), qi = q / (TK * TJ);
           const int x = i0 + qi, y = j0 + qj, z = k0 + qk;
           return (x < a.nx && y < a.ny && z < a.nz) ? (unsigned)__umul24((unsigned)__umul24(x, a.ny) + y, a.nz) + z
                                                     : 0u;
@@ -1194,16 +1212,16 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
         double m[6];
   #pragma unroll
         for (int q = 0; q < 6; ++q)
-          m[q] = PFD  ? (double)plw[PFD ? q : 0] * a.msc[q]
-                 : MQ ? (double)ldo((const int*)RS(q, a.s_lag_met), idx) * a.msc[q]
+          m[q] = PFD  ? (double)plw[PFD ? q : 0] * msc(q)
+                 : MQ ? (double)ldo((const int*)RS(q, a.s_lag_met), idx) * msc(q)
                       : ldo((const double*)RM(q, a.s_lag_met), idx);
         if (a.lag_mode == 2) {
           const double tn = norm_factor<double>(m[0], m[1], m[2], m[3], m[4], m[5]);
   #pragma unroll
           for (int q = 0; q < 6; ++q) m[q] = (m[q] + (diag6(q) ? tn : 0.0)) / (1.0 - tn);
         }
-        const TC phl = (TC)((PFD  ? (double)plw[PFD ? 6 : 0] * a.msc[PHI]
-                             : MQ ? (double)ldo((const int*)RS(PHI, a.s_lag), idx) * a.msc[PHI]
+        const TC phl = (TC)((PFD  ? (double)plw[PFD ? 6 : 0] * msc(PHI)
+                             : MQ ? (double)ldo((const int*)RS(PHI, a.s_lag), idx) * msc(PHI)
                                   : ldo((const double*)RM(PHI, a.s_lag), idx)) +
                             a.phi_F_lag);
         const TC Dl = PFD ? (TC)pdl[0] : (TC)ldo((const TS*)RD(0, a.s_lag), idx);
@@ -1435,20 +1453,38 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
         if (!SPLIT || (!M32 && f < 7)) return *reinterpret_cast<const double*>(pfr + f * 1024 + kind * 512 + pq * 8);
         const int n = f - F32;
         const char* w = pfr + (N64 + (n >> 1)) * 1024 + (n & 1) * 512 + kind * 256 + pq * 4;
-        if (MQ && f < 7) return (double)*reinterpret_cast<const int*>(w) * a.msc[f < 7 ? f : 0];
+        if (MQ && f < 7) return (double)*reinterpret_cast<const int*>(w) * msc(f < 7 ? f : 0);
         return (double)*reinterpret_cast<const TS*>(w);
       };
       // stage 4: a2 of field f (f - F32 >= A2F) from the prefetch
       auto la2 = [&](int f) -> double {
         const int n = f - F32 - A2F;
         const char* w = pfr + (N64 + CPF + (n >> 2)) * 1024 + (n & 3) * 256 + pq * 4;
-        if (MQ && f < 7) return (double)*reinterpret_cast<const int*>(w) * a.msc[f < 7 ? f : 0];
+        if (MQ && f < 7) return (double)*reinterpret_cast<const int*>(w) * msc(f < 7 ? f : 0);
         return (double)*reinterpret_cast<const TS*>(w);
       };
       if constexpr (PF) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      // one loop per RK4 form, each with only its own loads and stores
-      auto epilogue = [&](auto incr_tag) {
-        constexpr bool INC = decltype(incr_tag)::value;
+      // One copy per kind of stage and RK4 form, without branches, so that its
+      // addresses stay SGPR bases plus one 32-bit offset (with a branch per
+      // field every access added its 64-bit address in VALU):
+      // EP_RHS (stage 0), EP_INC / EP_INC4 (accumulator-free stages 1-3, 4),
+      // EP_ACC1 / EP_ACC / EP_ACC4 (with _f: stage 1, 2-3, 4).
+      // With the sums in units of their first weight, the three-operand
+      // additions and the wrap by minima (4210 to 3976 VALU instructions in
+      // the order-6 fixed-point kernel) a stage takes 1.51 ms at 256^3 instead
+      // of 1.64, FP64 at 128^3 0.324 instead of 0.336, dust at 192^3 0.987
+      // instead of 1.036.
+      bool saturated = false;
+      auto epilogue = [&](auto kind_tag) {
+        constexpr int EP = decltype(kind_tag)::value;
+        constexpr bool INC = EP == EP_INC || EP == EP_INC4, S0 = EP == EP_RHS, S4 = EP == EP_INC4 || EP == EP_ACC4;
+        constexpr bool LF = EP == EP_ACC || EP == EP_ACC4 || EP == EP_INC4;  // _f (or a1) is read
+        // the offset made new in this block (a zero extension shared with the
+        // blocks before it would again be added to every base in 64 bits)
+        unsigned ix = idx;
+#if defined(__HIP_DEVICE_COMPILE__)
+        asm volatile("" : "+v"(ix));
+#endif
         // The epilogue's loads from memory (stage 4 of the accumulator-free
         // form: a2 and a3 of the FP64 metric; without the LDS prefetch also p
         // and f / a1).  The compiler cannot move a load above a store into the
@@ -1462,39 +1498,37 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
         double addv[SHIFT ? NF : 1], bin[SHIFT ? 3 : 1], bp[SHIFT ? 3 : 1], bf[SHIFT ? 3 : 1];
         auto has_add = [](int g) { return SHIFT && !(g == KK && R > 2); };
         auto pre = [&](int g) {
-          if (g >= NF || st == 0 || (g == ALPHA && !LIVE_ALPHA)) return;
+          if (g >= NF || S0 || (g == ALPHA && !LIVE_ALPHA)) return;
           // a storage-type word as FP64 (fixed-point metric words scaled)
           auto lw = [&](int slot) -> double {
-            if (MQ && g < 7) return (double)ldo((const int*)RS(g, slot), idx) * a.msc[g < 7 ? g : 0];
-            return (double)ldo((const TS*)RS(g, slot), idx);
+            if (MQ && g < 7) return (double)ldo((const int*)RS(g, slot), ix) * msc(g < 7 ? g : 0);
+            return (double)ldo((const TS*)RS(g, slot), ix);
           };
           if constexpr (SHIFT) {
             if (has_add(g))
-              addv[g] = mfield<M32>(g) ? ldo((const double*)RM(g, a.s_add), idx) : (double)ldo((const TS*)RS(g, a.s_add), idx);
+              addv[g] = mfield<M32>(g) ? ldo((const double*)RM(g, a.s_add), ix) : (double)ldo((const TS*)RS(g, a.s_add), ix);
             if (g >= GAM1 && g <= GAM3 && a.auxB) {
               const int i = g >= GAM1 && g <= GAM3 ? g - GAM1 : 0;
               const double* xb = a.auxB + (long)i * 4 * a.rstride;
-              bin[i] = ldo(xb + (long)a.s_in * a.rstride, idx);
-              bp[i] = ldo(xb + (long)a.s_p * a.rstride, idx);
-              bf[i] = st >= 2 ? ldo(xb + (long)a.s_f * a.rstride, idx) : 0.0;
+              bin[i] = ldo(xb + (long)a.s_in * a.rstride, ix);
+              bp[i] = ldo(xb + (long)a.s_p * a.rstride, ix);
+              bf[i] = LF ? ldo(xb + (long)a.s_f * a.rstride, ix) : 0.0;
             }
           }
           if constexpr (!PF) {
             const bool m = mfield<M32>(g);
-            pv[g] = m ? ldo((const double*)RM(g, a.s_p), idx) : lw(a.s_p);
-            if (INC ? st == 4 : st >= 2) qv[g] = m ? ldo((const double*)RM(g, a.s_f), idx) : lw(a.s_f);
+            pv[g] = m ? ldo((const double*)RM(g, a.s_p), ix) : lw(a.s_p);
+            if (LF) qv[g] = m ? ldo((const double*)RM(g, a.s_f), ix) : lw(a.s_f);
           }
-          if constexpr (INC) {
-            if (st == 4) {
-              if (mfield<M32>(g)) {
-                a2v[g] = ldo((const double*)RM(g, a.s_a2), idx);
-                a3m[g] = ldo(INM(g), idx);
-              } else {
-                a2v[g] = PF2 && g - F32 >= A2F ? la2(g) : lw(a.s_a2);
-                // the fixed-point metric's stage-4 input, re-read here rather
-                // than kept in registers through the stencil phase
-                if (MQ && g < 7) a3m[g < 7 ? g : 0] = lw(a.s_in);
-              }
+          if constexpr (EP == EP_INC4) {
+            if (mfield<M32>(g)) {
+              a2v[g] = ldo((const double*)RM(g, a.s_a2), ix);
+              a3m[g < 7 ? g : 0] = ldo(INM(g), ix);
+            } else {
+              a2v[g] = PF2 && g - F32 >= A2F ? la2(g) : lw(a.s_a2);
+              // the fixed-point metric's stage-4 input, re-read here rather
+              // than kept in registers through the stencil phase
+              if (MQ && g < 7) a3m[g < 7 ? g : 0] = lw(a.s_in);
             }
           }
         };
@@ -1510,111 +1544,104 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
               const int i = f >= GAM1 && f <= GAM3 ? f - GAM1 : 0;
               double* xb = a.auxB + (long)i * 4 * a.rstride;
               const double cb = 0.75 * cc - a.gd_eta * bin[i], inc = a.cf * cb;
-              sto(xb + (long)a.s_out * a.rstride, idx, st == 4 ? bf[i] + (inc + bp[i]) : bp[i] + a.ca * cb);
-              if (st != 4) sto(xb + (long)a.s_f * a.rstride, idx, bf[i] + inc);
+              sto(xb + (long)a.s_out * a.rstride, ix, S4 ? bf[i] + (inc + bp[i]) : bp[i] + a.ca * cb);
+              if (!S4) sto(xb + (long)a.s_f * a.rstride, ix, bf[i] + inc);
             }
           }
           if (mfield<M32>(f)) {
             double* __restrict__ o = RM(f, a.s_out);
-            if (st == 0) {
-              sto(o, idx, cc);
+            if constexpr (S0) {
+              sto(o, ix, cc);
               continue;
             }
             const double p = PF ? lpf(f, 0) : pv[f];
             double* __restrict__ fr = RM(f, a.s_f);
             double fo = 0.0;
-            if constexpr (!INC) {
-              if (st >= 2) fo = PF ? lpf(f, 1) : qv[f];
-            } else if (st == 4) {
-              const double a1 = PF ? lpf(f, 1) : qv[f];
-              fo = ((a1 - p) + 2.0 * (a2v[f] - p) + (a3m[f] - p)) * (1.0 / 3.0);
-            }
+            if constexpr (LF) fo = PF ? lpf(f, 1) : qv[f];
+            if constexpr (EP == EP_INC4) fo = ((fo - p) + 2.0 * (a2v[f] - p) + (a3m[f < 7 ? f : 0] - p)) * (1.0 / 3.0);
             const double inc = a.cf * cc;
-            const double nv = st == 4 ? fo + (inc + p) : p + a.ca * cc;
+            const double nv = S4 ? fo + (inc + p) : p + a.ca * cc;
             if (f == PHI) phi_new = nv;
             if (f <= G33) gn[f] = nv;
-            sto(o, idx, nv);
-            if (st == 4) {
-              if (f == PHI && nan_as_float(nv)) atomicAdd(a.nan_count, 1u);
-            } else if (!INC) {
-              sto(fr, idx, fo + inc);
-            }
+            sto(o, ix, nv);
+            if (S4 && f == PHI && nan_as_float(nv)) atomicAdd(a.nan_count, 1u);
+            if (!S4 && !INC) sto(fr, ix, fo + inc);
           } else if (MQ && f < 7) {
             // fixed-point metric: the RK4 value in FP64, stored as the
             // field's word; phi_new and gn are the stored values
             int* __restrict__ o = (int*)RS(f, a.s_out);
-            const double sc = a.msc[f < 7 ? f : 0], iv = a.minv[f < 7 ? f : 0];
-            if (st == 0) {
-              sto(o, idx, mq_word(cc, iv));
+            const double sc = msc(f < 7 ? f : 0), iv = minv(f < 7 ? f : 0);
+            if constexpr (S0) {
+              sto(o, ix, mq_word(cc, iv));
               continue;
             }
             const double p = PF ? lpf(f, 0) : pv[f];
             double fo = 0.0;
-            if constexpr (!INC) {
-              if (st >= 2) fo = PF ? lpf(f, 1) : qv[f];
-            } else if (st == 4) {
-              const double a1 = PF ? lpf(f, 1) : qv[f];
-              fo = ((a1 - p) + 2.0 * (a2v[f] - p) + (a3m[f < 7 ? f : 0] - p)) * (1.0 / 3.0);
-            }
+            if constexpr (LF) fo = PF ? lpf(f, 1) : qv[f];
+            if constexpr (EP == EP_INC4) fo = ((fo - p) + 2.0 * (a2v[f] - p) + (a3m[f < 7 ? f : 0] - p)) * (1.0 / 3.0);
             const double inc = a.cf * cc;
-            const double nd = st == 4 ? fo + (inc + p) : p + a.ca * cc;
-            if (fabs(nd * iv) > MQ_WMAX) atomicAdd(a.mq_sat, 1u);
+            const double nd = S4 ? fo + (inc + p) : p + a.ca * cc;
+            saturated |= fabs(nd * iv) > MQ_WMAX;
             const int w = mq_word(nd, iv);
             const double nv = (double)w * sc;
             if (f == PHI) {
               phi_new = nv;
-              if (st == 4 && nan_as_float(nd)) atomicAdd(a.nan_count, 1u);
+              if (S4 && nan_as_float(nd)) atomicAdd(a.nan_count, 1u);
             } else {
               gn[f < 6 ? f : 0] = nv;
             }
-            sto(o, idx, w);
-            if (st != 4 && !INC) sto((int*)RS(f, a.s_f), idx, mq_word(fo + inc, iv));
+            sto(o, ix, w);
+            if (!S4 && !INC) sto((int*)RS(f, a.s_f), ix, mq_word(fo + inc, iv));
           } else {
             TS* __restrict__ o = RS(f, a.s_out);
-            if (st == 0) {
-              sto(o, idx, (TS)cc);
+            if constexpr (S0) {
+              sto(o, ix, (TS)cc);
               continue;
             }
             const double p = PF ? lpf(f, 0) : pv[f];
             TS* __restrict__ fr = RS(f, a.s_f);
             double fo = 0.0;
-            if constexpr (!INC) {
-              if (st >= 2) fo = PF ? lpf(f, 1) : qv[f];
-            } else if (st == 4) {
-              const double a1 = PF ? lpf(f, 1) : qv[f];
+            if constexpr (LF) fo = PF ? lpf(f, 1) : qv[f];
+            if constexpr (EP == EP_INC4) {
               const double a2 = a2v[f];
               // the stored value: v holds it exactly when storage and compute types agree
-              const double a3 = std::is_same<TS, TC>::value ? (double)v[f] : (double)ldo(INS(f), idx);
-              fo = ((a1 - p) + 2.0 * (a2 - p) + (a3 - p)) * (1.0 / 3.0);
+              const double a3 = std::is_same<TS, TC>::value ? (double)v[f] : (double)ldo(INS(f), ix);
+              fo = ((fo - p) + 2.0 * (a2 - p) + (a3 - p)) * (1.0 / 3.0);
             }
             const double inc = a.cf * cc;
-            const TS nv = st == 4 ? (TS)(fo + (inc + p)) : (TS)(p + a.ca * cc);
+            const TS nv = S4 ? (TS)(fo + (inc + p)) : (TS)(p + a.ca * cc);
             if (f == KK) K_new = (double)nv;
             if (f >= A11 && f <= A33) An[f - A11] = (double)nv;
             if (M32 && f == PHI) {
               phi_new = (double)nv;
-              if (st == 4 && nan_as_float(nv)) atomicAdd(a.nan_count, 1u);
+              if (S4 && nan_as_float(nv)) atomicAdd(a.nan_count, 1u);
             }
             if (M32 && f <= G33) gn[f] = (double)nv;
-            sto(o, idx, nv);
-            if (st != 4 && !INC) sto(fr, idx, (TS)(fo + inc));
+            sto(o, ix, nv);
+            if (!S4 && !INC) sto(fr, ix, (TS)(fo + inc));
           }
         }
       };
-      if constexpr (SHIFT) {
-        epilogue(std::false_type{});  // four slots hold p, f, the input and the terms
-      } else {
-        if (a.incr) epilogue(std::true_type{});
-        else epilogue(std::false_type{});
-      }
+      auto run = [&](auto kind) { epilogue(kind); };
+      if (st == 0) run(std::integral_constant<int, EP_RHS>{});
+      else if (!SHIFT && a.incr && st != 4) run(std::integral_constant<int, SHIFT ? EP_ACC : EP_INC>{});
+      else if (!SHIFT && a.incr) run(std::integral_constant<int, SHIFT ? EP_ACC : EP_INC4>{});
+      else if (st == 1) run(std::integral_constant<int, EP_ACC1>{});
+      else if (st == 4) run(std::integral_constant<int, EP_ACC4>{});
+      else run(std::integral_constant<int, EP_ACC>{});  // (the shift build's slots: p, f, the input and the terms)
       if (DMA && st == 4 && a.s_norm_out >= 0) {
         // set_DIFFgamma_Aij_norm (bssn.cc:61-119) of the new state, as the
         // next step's stepInit applies it to _a (DMA kernels only: the
         // launcher pairs the copy with DMA staging)
         const double tn = norm_factor<double>(gn[0], gn[1], gn[2], gn[3], gn[4], gn[5]);
+        unsigned ix = idx;
+#if defined(__HIP_DEVICE_COMPILE__)
+        asm volatile("" : "+v"(ix));
+#endif
         double g[6];
+        const double rden = 1.0 / (1.0 - tn);
     #pragma unroll
-        for (int s = 0; s < 6; ++s) g[s] = (gn[s] + (diag6(s) ? tn : 0.0)) / (1.0 - tn);
+        for (int s = 0; s < 6; ++s) g[s] = (gn[s] + (diag6(s) ? tn : 0.0)) * rden;
         const double i11 = 1.0 + g[3] + g[5] - g[4] * g[4] + g[3] * g[5];
         const double i22 = 1.0 + g[0] + g[5] - g[2] * g[2] + g[0] * g[5];
         const double i33 = 1.0 + g[0] + g[3] - g[1] * g[1] + g[0] * g[3];
@@ -1625,15 +1652,16 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
     #pragma unroll
         for (int s = 0; s < 6; ++s) {
           if constexpr (MQ) {
-            if (fabs(g[s] * a.minv[s]) > MQ_WMAX) atomicAdd(a.mq_sat, 1u);
-            sto((int*)RS(G11 + s, a.s_norm_out), idx, mq_word(g[s], a.minv[s]));
+            saturated |= fabs(g[s] * minv(s)) > MQ_WMAX;
+            sto((int*)RS(G11 + s, a.s_norm_out), ix, mq_word(g[s], minv(s)));
           }
-          else if constexpr (M32) sto(RS(G11 + s, a.s_norm_out), idx, (TS)g[s]);
-          else sto(RM(G11 + s, a.s_norm_out), idx, g[s]);
-          sto(RS(A11 + s, a.s_norm_out), idx,
-              (TS)((An[s] - (1.0 / 3.0) * ((diag6(s) ? 1.0 : 0.0) + g[s]) * trA) / (1.0 - tn)));
+          else if constexpr (M32) sto(RS(G11 + s, a.s_norm_out), ix, (TS)g[s]);
+          else sto(RM(G11 + s, a.s_norm_out), ix, g[s]);
+          sto(RS(A11 + s, a.s_norm_out), ix,
+              (TS)((An[s] - (1.0 / 3.0) * ((diag6(s) ? 1.0 : 0.0) + g[s]) * trA) * rden));
         }
       }
+      if (MQ && saturated) atomicAdd(a.mq_sat, 1u);
     }  // constraint mode / stage
   }  // valid
   if constexpr (CONS) {

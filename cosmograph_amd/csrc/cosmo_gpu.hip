@@ -18,6 +18,7 @@
 #include "../../include/cosmo_gpu.h"
 #include "bssn_stage.h"
 #include "runtime.h"
+#include "stencil.h"
 
 using namespace cg;
 
@@ -931,7 +932,8 @@ StageArgs make_args(cg_ctx* c, int stage, int rin, int rp, int rf, int rout, int
   // regs + (f - 7)*4*rstride addresses the metric fields too
   a.regs = c->met32 ? (void*)((char*)c->regs + 7 * c->fstride * (long)c->ts) : c->regs;
   a.rstride = c->rstride;
-  mq_scales(c, a.msc, a.minv);
+  double msc[7], minv[7];
+  mq_scales(c, msc, minv);
   a.mq_sat = c->mq_sat;
   a.s_in = rin; a.s_p = rp; a.s_f = rf; a.s_out = rout;
   a.s_in_norm = -1; a.s_norm_out = -1;
@@ -948,9 +950,15 @@ StageArgs make_args(cg_ctx* c, int stage, int rin, int rp, int rf, int rout, int
   a.use_H = (c->p.a_adj_amp != 0.0 || c->p.k_damping_amp != 0.0);
   a.inv_dx = 1.0 / c->p.dx;
   a.inv_dx2 = 1.0 / (c->p.dx * c->p.dx);
+  const int R = c->R;
+  const double w1 = R == 1 ? c1<1>(1) : R == 2 ? c1<2>(1) : R == 3 ? c1<3>(1) : c1<4>(1);
+  const double w2 = R == 1 ? c2<1>(1) : R == 2 ? c2<2>(1) : R == 3 ? c2<3>(1) : c2<4>(1);
+  const double wm = R == 1 ? cm<1>(1) : R == 2 ? cm<2>(1) : R == 3 ? cm<3>(1) : cm<4>(1);
   for (int f = 0; f < 7; ++f) {
-    a.msd1[f] = (float)(a.msc[f] * a.inv_dx);
-    a.msd2[f] = (float)(a.msc[f] * a.inv_dx2);
+    a.mexp[f] = c->mq ? c->mq_exp[f] : 0;
+    a.msd1[f] = (float)(msc[f] * a.inv_dx * w1);
+    a.msd2[f] = (float)(msc[f] * a.inv_dx2 * w2 * (f == PHI ? 1.0 : -0.5));
+    a.msdm[f] = (float)(msc[f] * a.inv_dx2 * wm * (f == PHI ? 1.0 : -1.0));
   }
   a.dt = c->p.dt;
   // RK4Register weights (RK4Register.h:129-176)

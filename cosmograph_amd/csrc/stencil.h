@@ -47,6 +47,15 @@ __device__ __forceinline__ T fd1(const T* s, int c, int st) {
   return acc;
 }
 
+// fd1 in units of c1(1): for fields whose factor 1/dx carries the weight
+template <int R, typename T>
+__device__ __forceinline__ T fd1n(const T* s, int c, int st) {
+  T acc = s[c + st] - s[c - st];
+#pragma unroll
+  for (int m = 2; m <= R; ++m) acc += T(c1<R>(m) / c1<R>(1)) * (s[c + m * st] - s[c - m * st]);
+  return acc;
+}
+
 template <int R, typename T>
 __device__ __forceinline__ T fd2(const T* s, int c, int st) {
   T acc = T(c2<R>(0)) * s[c];
@@ -77,26 +86,36 @@ __device__ __forceinline__ T fdm(const T* s, int c, int sa, int sb) {
 // the relative precision of the derivative itself; FP32 storage of the
 // values would instead lose it to the cancellation of neighbouring values.
 __device__ __forceinline__ float qd(int a, int b) { return (float)(int)((unsigned)a - (unsigned)b); }
-// (a - c0) + (b - c0) as (a + b) - 2 c0: the same value in wrap-around
-// arithmetic, one operation fewer (c2 = 2 c0 once per stencil)
-__device__ __forceinline__ float qdd(int a, int b, unsigned c2) {
-  return (float)(int)(((unsigned)a + (unsigned)b) - c2);
+// (a - c0) + (b - c0) as a + b + (-2 c0): the same value in wrap-around
+// arithmetic, one three-operand addition (m2 = -2 c0 once per stencil)
+__device__ __forceinline__ float qdd(int a, int b, unsigned m2) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  unsigned d;  // (the compiler splits the sum into two additions)
+  asm("v_add3_u32 %0, %1, %2, %3" : "=v"(d) : "v"(a), "v"(b), "v"(m2));
+  return (float)(int)d;
+#else
+  return (float)(int)((unsigned)a + (unsigned)b + m2);
+#endif
 }
 
+// These sums are in units of their first weight (c1(1), c2(1), cm(1)): the
+// innermost difference enters unmultiplied, and the caller's factor carries
+// the weight.  That is one multiplication fewer per derivative, 63 per point
+// of the stage kernel, which issues VALU instructions 85% of the time.
 template <int R>
 __device__ __forceinline__ float fd1qf(const int* s, int c, int st) {
-  float acc = float(c1<R>(1)) * qd(s[c + st], s[c - st]);
+  float acc = qd(s[c + st], s[c - st]);
 #pragma unroll
-  for (int m = 2; m <= R; ++m) acc += float(c1<R>(m)) * qd(s[c + m * st], s[c - m * st]);
+  for (int m = 2; m <= R; ++m) acc += float(c1<R>(m) / c1<R>(1)) * qd(s[c + m * st], s[c - m * st]);
   return acc;
 }
 
 template <int R>
 __device__ __forceinline__ float fd2qf(const int* s, int c, int st) {
-  const unsigned q2 = 2u * (unsigned)s[c];
-  float acc = float(c2<R>(1)) * qdd(s[c + st], s[c - st], q2);
+  const unsigned m2 = 0u - 2u * (unsigned)s[c];
+  float acc = qdd(s[c + st], s[c - st], m2);
 #pragma unroll
-  for (int m = 2; m <= R; ++m) acc += float(c2<R>(m)) * qdd(s[c + m * st], s[c - m * st], q2);
+  for (int m = 2; m <= R; ++m) acc += float(c2<R>(m) / c2<R>(1)) * qdd(s[c + m * st], s[c - m * st], m2);
   return acc;
 }
 
@@ -107,7 +126,8 @@ __device__ __forceinline__ float fdmqf(const int* s, int c, int sa, int sb) {
   for (int m = 1; m <= R; ++m) {
     const int p = m * (sa + sb), q = m * (sa - sb);
     const unsigned d = ((unsigned)s[c + p] - (unsigned)s[c + q]) - ((unsigned)s[c - q] - (unsigned)s[c - p]);
-    acc += float(cm<R>(m)) * (float)(int)d;
+    if (m == 1) acc = (float)(int)d;
+    else acc += float(cm<R>(m) / cm<R>(1)) * (float)(int)d;
   }
   return acc;
 }

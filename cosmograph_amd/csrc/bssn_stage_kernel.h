@@ -386,12 +386,19 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
 
   const int tid = threadIdx.x;
   __builtin_assume(tid >= 0 && tid < NT);
-  // Point of a thread.  On 4x4x16 tiles of 4-byte words the halo rows are 24
-  // words apart, so the two rows of 16 lanes that one LDS cycle serves would
-  // meet in 8 of the 32 banks (818 conflict cycles per wave of 3200); with rows
-  // j and j + 2 in one half of the wave they are 16 banks apart instead.
-  constexpr bool JPERM = DMA && M32 && TJ == 4 && TK == 16 && HK4 % 32 == 24;
-  auto row_j = [](int r) { return JPERM ? (r & 1) * 2 + (r >> 1) : r; };  // 0, 2, 1, 3
+  // Point of a thread.  Lanes take the rows along j in an order that keeps the
+  // rows of one LDS cycle (32 words) on different banks:
+  // - 4-byte tiles 4x4x16: rows of 16 lanes 24 words apart, two to a cycle,
+  //   would meet in 8 banks (818 conflict cycles per wave of 3200 in the
+  //   order-6 fixed-point kernel, 96 so); rows j and j + 2 are 16 apart.
+  // - FP64 tiles of 8x8 rows: 8 lanes (16 words) a row, rows 40 or 24 words
+  //   apart meet likewise; rows j and j + 2 are 16 or 48 words apart (order 8
+  //   with KO, 8x8x8 at 96^3: half of the LDS cycles were conflicts, 0.432 ->
+  //   0.401 ms a stage).
+  constexpr bool JPERM = DMA && ((sizeof(TS) == 4 && TJ == 4 && TK == 16 && HK4 % 32 == 24) ||
+                                 (sizeof(TS) == 8 && TJ == 8 && TK == 8 && 2 * HK % 16 == 8));
+  constexpr int JB = TJ == 8 ? 2 : 1;
+  auto row_j = [](int r) { return JPERM ? (r << 1 | r >> JB) & (TJ - 1) : r; };  // 0, 2, (4, 6,) 1, 3, (5, 7)
   const int lk = tid % TK, lj = row_j((tid / TK) % TJ), li = tid / (TK * TJ);
   const int px = i0 + li, py = j0 + lj, pz = k0 + lk;
   const bool valid = (px < a.nx) && (py < a.ny) && (pz < a.nz);

@@ -270,7 +270,7 @@ enum { EP_RHS, EP_INC, EP_INC4, EP_ACC1, EP_ACC, EP_ACC4 };
 // DMA = true: the halo tiles go from memory straight into LDS
 // (global_load_lds, 16 bytes per lane), two fields ahead of the one being
 // differentiated, in three LDS buffers.  No registers hold the loads in
-// flight.  Requires nz % 4 == 0 and no stage-1 normalisation (a.normalize is
+// flight.  Requires rows of whole 16-byte groups and no stage-1 normalisation (a.normalize is
 // ignored); the launcher falls back to DMA = false otherwise.
 template <typename TS, typename TC, int R, int H, int TI, int TJ, int TK, int WPE, bool LIVE_ALPHA, int MODE,
           bool DMA = false>

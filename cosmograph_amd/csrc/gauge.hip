@@ -428,7 +428,7 @@ __global__ void __launch_bounds__(GNT) __attribute__((amdgpu_waves_per_eu(2))) k
 // Two blocks of 4 waves per CU (57.6 KB of LDS, 2 waves per SIMD), where one
 // 512-thread block of the 8x8x8 tile left the CU idle at each of its barriers:
 // 0.297 ms per launch at 112^3, order 4, FP64, against 0.529 ms, and without
-// the 0.28 ms of the finalize passes.  Orders 2, 4 and 6 (halo 3), nz % 4 == 0.
+// the 0.28 ms of the finalize passes.  Orders 2, 4 and 6 (halo 3), rows of whole 16-byte groups.
 constexpr int TTI = 4, TTJ = 4, TTK = 16, TNT = TTI * TTJ * TTK, TH = 3, TKH = 4;
 template <typename E>
 __device__ __forceinline__ double el(const void* T, int c) {
@@ -882,7 +882,7 @@ bool gauge_fusable(const cg_ctx* c) {
   // 16-byte groups along k, one wrap per axis, 24-bit offsets (the 32-bit byte
   // offsets follow from cg_create's bound on the grid)
   if (c->p.stencil_order > 6 || !c->dma_allowed) return false;
-  return c->p.nz % 4 == 0 && c->p.nz > TTK + TKH - 2 && c->p.nx > TTI + TH - 2 && c->p.ny > TTJ + TH - 2 &&
+  return c->p.nz % (c->prec == CG_FP64 ? 2 : 4) == 0 && c->p.nz > TTK + TKH - 2 && c->p.nx > TTI + TH - 2 && c->p.ny > TTJ + TH - 2 &&
          (long long)c->p.nx * c->p.ny < (1ll << 24);
 }
 

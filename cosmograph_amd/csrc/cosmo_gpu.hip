@@ -706,6 +706,28 @@ static bool mq_register(const cg_ctx* c, const void* d, int* f, int* slot) {
   return true;
 }
 
+// After fused steps of the shift build: gives _a and _f registers of their own
+// (copies of _p), as the method sequence leaves them.
+static int unalias(cg_ctx* c) {
+  if (!c->a_is_p || !c->a_raw) return CG_OK;
+  if (int rc = ext_resolve(c)) return rc;  // it reads the slots written here
+  int free_slot[2], n = 0;
+  for (int s = 0; s < 4 && n < 2; ++s)
+    if (s != c->sP && s != c->sC) free_slot[n++] = s;
+  for (int s : free_slot) {
+    for (int f = 0; f < NF; ++f)
+      HIPCHK(c, hipMemcpyAsync(reg_ptr(c, f, s), reg_ptr(c, f, c->sP), (size_t)c->npts * (f < 7 ? 8 : c->ts),
+                               hipMemcpyDeviceToDevice, c->stream));
+    for (int q = 0; q < c->nxf; ++q)
+      HIPCHK(c, hipMemcpyAsync(c->xreg + ((long)q * 4 + s) * c->rstride, c->xreg + ((long)q * 4 + c->sP) * c->rstride,
+                               (size_t)c->npts * 8, hipMemcpyDeviceToDevice, c->stream));
+  }
+  c->sA = free_slot[0];
+  c->sF = free_slot[1];
+  c->a_is_p = false;
+  return CG_OK;
+}
+
 // resolve a reference field-map key to a device pointer and element size
 static void* resolve(cg_ctx* c, const char* name, bool for_write, int* err, size_t* esz) {
   *err = 0;
@@ -739,6 +761,7 @@ static void* resolve(cg_ctx* c, const char* name, bool for_write, int* err, size
   if (s.size() < 3 || s[s.size() - 2] != '_') { *err = 1; return nullptr; }
   const std::string base = s.substr(0, s.size() - 2);
   const char r = s.back();
+  if (for_write && (r == 'a' || r == 'f') && unalias(c)) { *err = 2; return nullptr; }
   auto slot_of = [&](char rr) {
     return rr == 'p' ? c->sP : rr == 'f' ? (c->a_is_p ? c->sP : c->sF) : rr == 'a' ? (c->a_is_p ? c->sP : c->sA)
            : rr == 'c' ? c->sC : -1;
@@ -1189,6 +1212,7 @@ int cg_step_init(cg_ctx* c) {
 
 int cg_rk_evolve(cg_ctx* c) {
   if (!c) return CG_ERR_ARG;
+  if (int rc = unalias(c)) return rc;
   if (c->a_is_p) return fail(c, CG_ERR_STATE, "RKEvolve before stepInit");
   if (c->mq)
     return fail(c, CG_ERR_STATE, "the fixed-point metric holds states, not right-hand sides: step with cg_rk4_steps");
@@ -1233,6 +1257,7 @@ static int finalize_t(cg_ctx* c, int n, const SrcArgs& src) {
 
 int cg_k_finalize(cg_ctx* c, int n) {
   if (!c || n < 1 || n > 4) return CG_ERR_ARG;
+  if (int rc = unalias(c)) return rc;
   if (c->a_is_p) return fail(c, CG_ERR_STATE, "K-finalize before stepInit");
   if (c->mq)
     return fail(c, CG_ERR_STATE, "the fixed-point metric holds states, not right-hand sides: step with cg_rk4_steps");
@@ -1369,7 +1394,7 @@ int cg_rk4_steps(cg_ctx* c, int nsteps) {
       if ((rc = stage(4, s3, 0, 0, -1, pre ? s1 : -1, s1, s2))) return rc;
       have_norm = pre;
       norm_slot = s1;
-      c->sA = 0; c->sC = s3; c->a_is_p = true;
+      c->sA = 0; c->sC = s3; c->a_is_p = true; c->a_raw = shift;
       c->ext_fresh = flrw;
       if (!flrw) {
         c->ext_lazy = true;
@@ -1387,7 +1412,7 @@ int cg_rk4_steps(cg_ctx* c, int nsteps) {
     if ((rc = stage(3, Y, X, 0))) return rc;
     if ((rc = stage(4, X, 0, 0, -1, pre ? Y : -1))) return rc;
     have_norm = pre;
-    c->sA = 0; c->sC = X; c->a_is_p = true;
+    c->sA = 0; c->sC = X; c->a_is_p = true; c->a_raw = shift;
     c->ext_fresh = flrw;
     if (!flrw) {
       c->ext_lazy = true;
@@ -1474,8 +1499,8 @@ int cg::cons_input(cg_ctx* c, int* rin_out) {
   // the pending K4Finalize averages read the dust source this pass rewrites
   if (int rc = ext_resolve(c)) return rc;
   if (int rc = cons_fits(c)) return rc;
-  int rin = c->sA;
-  if (c->a_is_p) {
+  int rin = c->a_is_p ? c->sP : c->sA;
+  if (c->a_is_p && !c->a_raw) {
     rin = spare_slot(c);
     const int bs = 256;
     const long nbk = (c->npts + bs - 1) / bs;
@@ -1504,7 +1529,7 @@ static int cons_args(cg_ctx* c, StageArgs* out, bool* dma) {
   if (int rc = ext_resolve(c)) return rc;
   if (int rc = cons_fits(c)) return rc;
   StageArgs a = make_args(c, 0, c->a_is_p ? c->sP : c->sA, c->sP, c->sF, c->sC, 0);
-  if (c->a_is_p && c->p.normalize_metric) {
+  if (c->a_is_p && !c->a_raw && c->p.normalize_metric) {
     a.s_in_norm = spare_slot(c);
     if (int rc = norm_copy(c, c->sP, a.s_in_norm)) return rc;
   }
@@ -1814,7 +1839,7 @@ int cg_field_stats(cg_ctx* c, const char* name, double out[3]) {
 
 int cg_autotune(cg_ctx* c, int reps, char* report, size_t report_len) {
   if (!c || reps < 1) return CG_ERR_ARG;
-  if (!c->a_is_p) return fail(c, CG_ERR_STATE, "autotune between method-level stages would clobber _a/_c");
+  if (!c->a_is_p || c->a_raw) return fail(c, CG_ERR_STATE, "autotune between method-level stages would clobber _a/_c");
   if (int rc = ext_resolve(c)) return rc;
   // Times stage-1, stage-2 and stage-4 shaped launches per candidate, in
   // each RK4 form the fused step may use, so the evolved state is untouched:

@@ -179,6 +179,11 @@ struct cg_ctx {
   // register roles (physical slot of each reference register)
   int sP = 0, sF = 1, sA = 2, sC = 3;
   bool a_is_p = true;     // after a fused step _a and _f hold the same data as _p
+  // a_is_p after fused steps of the shift build, which stand for the method
+  // sequence: its _a is the step's result as it is (the constraints and the
+  // SVT pass read it without stepInit's normalisation), and _a, _f and the
+  // method calls can be used at once (unalias)
+  bool a_raw = false;
   std::string err;
   bool timing = false;
   std::vector<std::pair<hipEvent_t, hipEvent_t>> ev;

@@ -89,3 +89,45 @@ def test_nan_is_reported(gpu):
     with pytest.raises(gpu.CosmoGpuError) as e:
         g.step(1)
     assert e.value.code == gpu.ERR_NAN
+
+
+def test_registers_after_fused_steps(gpu):
+    """What the method sequence leaves behind stays so: the constraints (and the
+    statistics of det gamma and tr A, which stepInit would remove) are those of
+    the state as it is, autotune is refused, _a can be written and RKEvolve
+    called.  Bars: the registers agree to 1e-12, so the constraints, which are
+    about 1e-3 of the terms they are the difference of, to 1e-8; det gamma - 1
+    and tr A are rounding-sized sums over registers of order 1: 1e-11 absolute."""
+    shape, order = (18, 14, 20), 4
+    st = shift_state(shape, 5)
+    res = []
+    for dma in (True, False):
+        g = gpu.BSSN(gpu.GpuParams(n=shape, order=order, lapse="OnePlusLog", shift="GammaDriver", gd_eta=0.4))
+        g.set_dma(dma)
+        for f in FIELDS + X_ALL:
+            g.upload(f + "_p", st[f])
+        g.upload("DIFFD_a", st["DIFFD"])
+        g.frw_set(0.0, -3.0)
+        g.frw_add_fluid(3.0 / (8.0 * np.pi), 0.0)
+        g.step(2)
+        c = g.setConstraintCalcs()
+        with pytest.raises(gpu.CosmoGpuError):
+            g.autotune()
+        g.RKEvolve()
+        rhs = {f: g.download(f + "_c") for f in FIELDS + x_fields("GammaDriver")}
+        g.upload("DIFFK_a", st["DIFFK"])
+        regs = {f + r: g.download(f + r) for f in ("DIFFK", "A12", "beta1") for r in ("_a", "_f", "_p")}
+        g.step(1)
+        regs["last"] = g.download("A12_p")
+        res.append((c, rhs, regs))
+    (c0, rhs0, r0), (c1, rhs1, r1) = res
+    for k in ("H", "M"):
+        assert np.all(np.abs(np.array(c0[k]) - np.array(c1[k])) <= 1e-8 * np.abs(c1[k])), k
+    print("S", c0["S"], c1["S"], "A", c0["A"], c1["A"])
+    for k in ("A", "S"):
+        n = np.array(c1[k])
+        assert np.all(np.abs(np.array(c0[k]) - n) <= 1e-8 * np.abs(n) + 1e-11 * np.prod(shape)), k
+    for f in rhs0:
+        assert rel_l2(rhs0[f], rhs1[f]) <= 1e-10, f
+    for f in r0:
+        assert rel_l2(r0[f], r1[f]) <= 1e-11, f

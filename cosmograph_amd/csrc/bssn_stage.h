@@ -23,6 +23,9 @@ enum { MODE_STAGE = 0, MODE_CONS = 1, MODE_DUST = 2, MODE_DUST_CONS = 3 };
 enum { MODE_M32 = 4, MODE_M32_CONS = 5, MODE_MQ = 8, MODE_MQ_STAGE = 12, MODE_MQ_CONS = 13 };
 // bit 4: the shift build's fused stages, which add the gauge pass's terms
 enum { MODE_SHIFT = 16 };
+// FP32 fields by LDS-DMA of single words (rows that are no whole 16-byte groups
+// of FP32: nz = 2 mod 4), split precision
+enum { MODE_DW = 32 };
 // fixed-point metric word (MODE_MQ): value / 2^e rounded to the nearest
 // integer, saturated at MQ_WMAX = 2^30 - 1 in magnitude.  After each
 // exponent check the host keeps |word| below 2^MQ_BITS = 2^29, so a field
@@ -319,6 +322,7 @@ struct StageVariant {
   int (*launch_dma)(const StageArgs&, hipStream_t);
   int (*info_dma)(int* vgprs, int* scratch, int* lds);
   int (*launch_batch_dma)(const BatchArgs&, hipStream_t);
+  bool dword = false;     // the twin moves FP32 fields in single words (MODE_DW)
 };
 
 std::vector<StageVariant>& stage_variants();

@@ -177,7 +177,18 @@ __device__ __forceinline__ void dma16(const void* base, unsigned voff, unsigned 
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(bs), "s"(ls)
                : "memory", "m0");
 }
-// The same with a per-lane 64-bit address (lanes may read different arrays).
+// LDS DMA of 4 bytes per lane: lane l copies a word at base + voff (4-byte
+// aligned) into LDS byte lds + 4*l (global_load_lds_dword).
+__device__ __forceinline__ void dma4(const void* base, unsigned voff, unsigned lds) {
+  const unsigned long long bb = (unsigned long long)base;
+  const unsigned hi = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(bb >> 32));
+  const unsigned lo = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)bb);
+  const unsigned long long bs = ((unsigned long long)hi << 32) | (unsigned long long)lo;
+  const unsigned ls = (unsigned)__builtin_amdgcn_readfirstlane((int)lds);
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(voff), "s"(bs), "s"(ls)
+               : "memory", "m0");
+}
+// dma16 with a per-lane 64-bit address (lanes may read different arrays).
 __device__ __forceinline__ void dma16v(const void* addr, unsigned lds) {
   const unsigned ls = (unsigned)__builtin_amdgcn_readfirstlane((int)lds);
   asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(addr), "s"(ls)
@@ -302,6 +313,8 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
   constexpr bool CONS = (MODE & MODE_CONS) != 0;
   constexpr bool DUST = (MODE & MODE_DUST) != 0;
   constexpr bool SHIFT = (MODE & MODE_SHIFT) != 0;
+  constexpr bool DW = (MODE & MODE_DW) != 0;                    // FP32 fields in single words
+  static_assert(!DW || (DMA && SPLIT && !M32 && !CONS && !DUST && !SHIFT), "split-precision stage kernels");
   constexpr int KO_ORDER = (H > R) ? 2 * R : 0;
   // axis-only tiles: the points within H along one axis of the tile's own
   // (x part: HI x TJ x TK, y part: TI x HJ x TK, z part: TI x TJ x HK4)
@@ -322,7 +335,7 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
   static_assert(!MQ || sizeof(TS) == 4, "the fixed-point metric shares the 4-byte storage");
   // epilogue prefetch: the stage kernels, and with every field in 4 bytes
   // the dust ones too (which then load the fluid's point values first)
-  constexpr bool PF = DMA && ((MODE & ~(MODE_M32 | MODE_MQ | MODE_SHIFT)) == 0 ||
+  constexpr bool PF = DMA && ((MODE & ~(MODE_M32 | MODE_MQ | MODE_SHIFT | MODE_DW)) == 0 ||
                               (M32 && (MODE & ~(MODE_M32 | MODE_MQ | MODE_DUST)) == 0));
   constexpr bool PFD = PF && (MODE & MODE_DUST) != 0;
   constexpr int F32 = M32 ? 0 : 7;                              // first field of the FP32 prefetch chunks
@@ -1007,8 +1020,19 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
       const int g = pchunk(m) * 64 + ln;
       poff[m] = box_off<HK, HJ>(2 * (g < NPR ? g : 0), i0 - H, j0 - H, k0 - KH, a.nx, a.ny, a.nz);
     }
-    unsigned qoff[SPLIT ? MQD : 1];
-    if constexpr (SPLIT) {
+    // DW: a chunk of FP32 elements is four loads of 64 words (single elements
+    // wrap by themselves, so rows need not be whole quads).  Four times the
+    // load instructions, still less than register staging costs: 101x90x118,
+    // order 6, 0.205 -> 0.187 ms a stage (0.734 -> 0.649 ms a step), order 4
+    // 0.156 -> 0.149; 256x256x254 order 6 2.71 -> 2.44.
+    unsigned qoff[SPLIT ? MQD * (DW ? 4 : 1) : 1];
+    if constexpr (DW) {
+#pragma unroll
+      for (int m = 0; m < 4 * MQD; ++m) {
+        const int e = qchunk(m / 4) * 256 + m % 4 * 64 + ln;
+        qoff[m] = box_off<HK4, HJ>(e < HV4 ? e : 0, i0 - H, j0 - H, k0 - KH4, a.nx, a.ny, a.nz);
+      }
+    } else if constexpr (SPLIT) {
 #pragma unroll
       for (int m = 0; m < MQD; ++m) {
         const int g = qchunk(m) * 64 + ln;
@@ -1079,8 +1103,13 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
         for (int m = 0; m < MPR; ++m) dma16(src, poff[m] * 8u, dst + pchunk(m) * 1024);
       } else {
         const void* src = (const void*)INS(f);
+        if constexpr (DW) {
 #pragma unroll
-        for (int m = 0; m < MQD; ++m) dma16(src, qoff[m] * 4u, dst + qchunk(m) * 1024);
+          for (int m = 0; m < 4 * MQD; ++m) dma4(src, qoff[m] * 4u, dst + qchunk(m / 4) * 1024 + m % 4 * 256);
+        } else {
+#pragma unroll
+          for (int m = 0; m < MQD; ++m) dma16(src, qoff[m] * 4u, dst + qchunk(m) * 1024);
+        }
       }
     };
     auto seq = [&](int s) {
@@ -1096,7 +1125,7 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
         if (!SPLIT || mfield<M32>(f1)) dma_wait_barrier<MPR>();
         else if (KGRP && f1 >= KG0) dma_wait_barrier<MKG>();
         else if (FGRP && f1 >= FLUXG0) dma_wait_barrier<MFG>();
-        else dma_wait_barrier<MQD>();
+        else dma_wait_barrier<DW ? 4 * MQD : MQD>();
       } else {
         dma_wait_barrier<0>();
       }
@@ -1147,6 +1176,14 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
           const char* b = m < 7 ? (const char*)RM(m, 0) : (const char*)RS(m, 0);
           if (!f64 || need_f) dma16v(b + l64 * 8, reg + m * 1024);
         }
+        if constexpr (DW) {  // the same places, _p and _f of a field in a load each
+          const unsigned o1 = poff(64 * wv + ln) * 4u;
+  #pragma unroll
+          for (int n = 0; n < N32; ++n) {
+            dma4(RS(F32 + n, a.s_p), o1, reg + N64 * 1024 + n * 512);
+            if (need_f) dma4(RS(F32 + n, a.s_f), o1, reg + N64 * 1024 + n * 512 + 256);
+          }
+        } else {
         const bool f32 = ((ln >> 4) & 1) != 0;  // FP32 chunk: lanes 16-31 and 48-63 load _f
         const long l32 = (long)((ln >> 5) * 4 + (f32 ? a.s_f : a.s_p)) * a.rstride + o4;
   #pragma unroll
@@ -1154,6 +1191,7 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
           const int n = 2 * i + (ln >> 5);  // field F32 + n, 4 * rstride elements after field F32 + 2i for odd lanes
           const char* b = (const char*)RS(F32 + 2 * i, 0);
           if (n < N32 && (!f32 || need_f)) dma16v(b + l32 * 4, reg + (N64 + i) * 1024);
+        }
         }
         if (PF2 && a.incr && a.stage == 4) {
           // a2 of field F32 + A2F + 4i + lane/16 in chunk N64 + CPF + i
@@ -1800,6 +1838,14 @@ int cons_launch_t(const StageArgs& a, bool dma, hipStream_t s) {
   CG_REGISTER_STAGE_X(TS, TC, PREC, R, H, TI, TJ, TK, WPE, LA, MODE_STAGE, nullptr,                   \
                       CG_DMA_L(TS, TC, R, H, TI, TJ, TK, WPE, LA, MODE_STAGE),                        \
                       CG_DMA_I(TS, TC, R, H, TI, TJ, TK, WPE, LA, MODE_STAGE), nullptr)
+// the same with the twin for nz = 2 mod 4 (MODE_DW)
+#define CG_REGISTER_STAGE_DW(TS, TC, PREC, R, H, TI, TJ, TK, WPE, LA)                                  \
+  static StageVariantReg CG_CAT(reg_, __COUNTER__)(                                                    \
+      StageVariant{PREC, 2 * R, H, TI, TJ, TK, WPE, LA, false,                                        \
+                   &stage_launch_t<TS, TC, R, H, TI, TJ, TK, WPE, LA, MODE_STAGE>,                    \
+                   &stage_info_t<TS, TC, R, H, TI, TJ, TK, WPE, LA, MODE_STAGE>, nullptr,              \
+                   CG_DMA_L(TS, TC, R, H, TI, TJ, TK, WPE, LA, MODE_DW),                               \
+                   CG_DMA_I(TS, TC, R, H, TI, TJ, TK, WPE, LA, MODE_DW), nullptr, true});
 // single-grid and batched-ensemble kernels, each with its LDS-DMA twin
 #define CG_REGISTER_STAGE_BD(TS, TC, PREC, R, H, TI, TJ, TK, WPE, LA)                                  \
   CG_REGISTER_STAGE_X(TS, TC, PREC, R, H, TI, TJ, TK, WPE, LA, MODE_STAGE,                            \

@@ -482,8 +482,10 @@ bool variant_fits(const cg_ctx* c, const StageVariant& v) {
 // the LDS-DMA twin of v applies to this grid: compiled, rows of whole 16-byte
 // groups, which then never straddle the periodic wrap (nz a multiple of 2 in
 // FP64, of 4 where any field has 4 bytes; FP64 128x128x126, order 4: 0.337 ms a
-// stage against 0.384 with register staging), and one wrap of the k halo (rounded up to 4) suffices; the 4-byte dust kernels address the three
-// fluxes of a quantity from the first one, and the kernels with every field
+// stage against 0.384 with register staging; the split kernels that move their
+// FP32 fields in single words need a multiple of 2 and are for the grids that
+// quads do not fit), and one wrap of the k halo (rounded up to 4) suffices; the
+// 4-byte dust kernels address the three fluxes of a quantity from the first one, and the kernels with every field
 // in 4 bytes Gamma^1 and Gamma^3 from K and Gamma^2, with a 32-bit byte
 // offset; their halo offsets are formed with 24-bit multiplies (nx * ny < 2^24)
 bool dma_fits(const cg_ctx* c, const StageVariant& v) {
@@ -493,7 +495,8 @@ bool dma_fits(const cg_ctx* c, const StageVariant& v) {
   if (v.dust && v.prec != CG_FP64 && 3ull * rs4 > 0xFFFFFFFFull) return false;
   if ((v.prec == CG_FP32_ALL || v.prec == CG_FP32_FIX) && 5ull * rs4 > 0xFFFFFFFFull) return false;
   const int kh = (v.halo + 3) / 4 * 4;
-  const int group = v.prec == CG_FP64 ? 2 : 4;
+  const int group = v.prec == CG_FP64 || v.dword ? 2 : 4;
+  if (v.dword && c->p.nz % 4 == 0) return false;  // quads there
   return c->p.nz % group == 0 && c->p.nz >= kh && c->p.nz > v.tk + kh - 2;
 }
 
@@ -1881,6 +1884,7 @@ int cg_autotune(cg_ctx* c, int reps, char* report, size_t report_len) {
     c->var = &v;
     for (int d = 0; d < 2; ++d) {
       if (d == 1 && !(c->dma_allowed && dma_fits(c, v))) continue;
+      if (d == 0 && v.dword) continue;  // the register-staged kernel of another entry
       c->dma_pick = d == 1;
       for (int order = 0; order < 6; ++order) {
         if (order == 3 && !morton_fits((c->p.nx + v.ti - 1) / v.ti, (c->p.ny + v.tj - 1) / v.tj)) continue;

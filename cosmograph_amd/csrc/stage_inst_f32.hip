@@ -17,4 +17,6 @@ CG_F32(CG_REGISTER_STAGE_BD, 3, 4, 8, 8, 3)
 CG_F32(CG_REGISTER_STAGE_D, 3, 2, 8, 16, 3)
 CG_F32(CG_REGISTER_STAGE_D, 3, 4, 4, 16, 3)
 CG_F32(CG_REGISTER_STAGE, 3, 8, 8, 8, 2)
+CG_F32(CG_REGISTER_STAGE_DW, 2, 4, 4, 16, 3)
+CG_F32(CG_REGISTER_STAGE_DW, 3, 4, 4, 16, 3)
 }  // namespace cg

@@ -58,6 +58,27 @@ def test_stages(gpu, order, shape, lapse, ko):
         assert rel_l2(out[0][f], out[1][f]) <= 1e-14, f
 
 
+@pytest.mark.parametrize("order,shape,lapse,norm", [(4, (17, 13, 22), "Static", 1), (4, (16, 12, 50), "Harmonic", 1),
+                                                    (6, (18, 14, 34), "Static", 1), (6, (9, 11, 30), "OnePlusLog", 1),
+                                                    (6, (16, 16, 22), "Static", 0)])
+def test_split_stages(gpu, order, shape, lapse, norm):
+    """FP32 split: the FP64 metric moves in pairs, the FP32 fields in single
+    words.  Bar: that of the DMA test in split precision (1e-7)."""
+    print(f"case even dma split order {order} {shape} {lapse} norm {norm}", flush=True)
+    st = smooth_random_state(shape, seed=order + 1, with_alpha=lapse != "Static")
+    out, info = [], []
+    for dma in (True, False):
+        g = gpu.BSSN(gpu.GpuParams(n=shape, order=order, lapse=lapse, precision="fp32_split", normalize_metric=norm))
+        g.set_dma(dma)
+        _start(g, st, FIELDS)
+        g.step(3)
+        out.append({f: g.download(f + "_p") for f in FIELDS})
+        info.append(g.kernel_info())
+    assert info[0] != info[1]  # the DMA kernel ran
+    for f in FIELDS:
+        assert rel_l2(out[0][f], out[1][f]) <= 1e-7, f
+
+
 @pytest.mark.parametrize("order,shape", [(4, (17, 13, 22)), (6, (18, 14, 34))])
 def test_constraints(gpu, order, shape):
     print(f"case even dma constraints order {order} {shape}", flush=True)

@@ -1,5 +1,6 @@
 // Instantiations of the stage kernel: orders 2 and 8 (with and without the
-// wider Kreiss-Oliger halo), both precisions, default tile.
+// wider Kreiss-Oliger halo), both precisions: tiles with LDS-DMA twins, and the
+// register-staged 4x8x8 tile for the grids that those do not fit.
 #include "bssn_stage_kernel.h"
 
 namespace cg {

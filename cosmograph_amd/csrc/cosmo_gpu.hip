@@ -709,15 +709,17 @@ static bool mq_register(const cg_ctx* c, const void* d, int* f, int* slot) {
   return true;
 }
 
+static int spare_slot(const cg_ctx* c) { return c->sC == 3 ? 2 : 3; }  // of the two stage registers
+
 // After fused steps of the shift build: gives _a and _f registers of their own
 // (copies of _p), as the method sequence leaves them.
 static int unalias(cg_ctx* c) {
   if (!c->a_is_p || !c->a_raw) return CG_OK;
   if (int rc = ext_resolve(c)) return rc;  // it reads the slots written here
-  int free_slot[2], n = 0;
-  for (int s = 0; s < 4 && n < 2; ++s)
-    if (s != c->sP && s != c->sC) free_slot[n++] = s;
-  for (int s : free_slot) {
+  // _f in slot 1 as everywhere, _a in the stage register that _c leaves
+  c->sF = 1;
+  c->sA = spare_slot(c);
+  for (int s : {c->sA, c->sF}) {
     for (int f = 0; f < NF; ++f)
       HIPCHK(c, hipMemcpyAsync(reg_ptr(c, f, s), reg_ptr(c, f, c->sP), (size_t)c->npts * (f < 7 ? 8 : c->ts),
                                hipMemcpyDeviceToDevice, c->stream));
@@ -725,8 +727,6 @@ static int unalias(cg_ctx* c) {
       HIPCHK(c, hipMemcpyAsync(c->xreg + ((long)q * 4 + s) * c->rstride, c->xreg + ((long)q * 4 + c->sP) * c->rstride,
                                (size_t)c->npts * 8, hipMemcpyDeviceToDevice, c->stream));
   }
-  c->sA = free_slot[0];
-  c->sF = free_slot[1];
   c->a_is_p = false;
   return CG_OK;
 }
@@ -1311,8 +1311,9 @@ int cg_rk4_steps(cg_ctx* c, int nsteps) {
     }
     return CG_OK;
   }
-  // fixed physical slots for the fused path: P=0, F=1, X=2, Y=3
-  c->sP = 0; c->sF = 1;
+  // fixed physical slots for the fused path: P=0, F=1, X=2, Y=3.  No register
+  // role and no pending average changes before the first step begins: a call
+  // of no steps leaves the context as it was.
   const int X = 2, Y = 3;
   const bool ko_norm = ko_norm_path(c);
   // one fused stage: sources and RHS with the current FRW values, then the
@@ -1363,7 +1364,6 @@ int cg_rk4_steps(cg_ctx* c, int nsteps) {
     int rc = launch(c, a, c->svar);
     return (rc || !flrw) ? rc : ext_combine(c, c->last_rows, false);
   };
-  c->ext_lazy = false;
   // With DMA staging, stage 4 also writes the normalised copy of the new
   // state (stepInit's _a) into the dead slot Y, so that the next step's
   // stage 1 runs the DMA kernel instead of normalising halos on the fly.
@@ -1371,10 +1371,11 @@ int cg_rk4_steps(cg_ctx* c, int nsteps) {
   int norm_slot = Y;
   for (int s = 0; s < nsteps; ++s) {
     int rc;
-    c->sP = 0; c->sF = 1;
     // fixed-point metric: exponents checked every kMqCheck steps (a field's
     // words stay below 2^MQ_BITS; twice that saturates)
     if (c->mq && s % kMqCheck == 0 && (rc = mq_check(c))) return rc;
+    c->sP = 0; c->sF = 1;
+    c->ext_lazy = false;  // this step writes the slots they are formed from
     const bool pre = c->p.normalize_metric && s + 1 < nsteps &&
                      (shift || (c->var && c->dma_allowed && c->dma_pick && dma_fits(c, *c->var)));
     if ((ko_norm || (shift && c->p.normalize_metric)) && !have_norm) {
@@ -1493,7 +1494,6 @@ static int cons_fits(cg_ctx* c) {
     return fail(c, CG_ERR_ARG, "grid too small for the constraint kernel tile");
   return CG_OK;
 }
-static int spare_slot(const cg_ctx* c) { return c->sC == 3 ? 2 : 3; }  // of the two stage registers
 
 // The register the SVT pass reads: _a as the reference's output step
 // sees it, after stepInit, i.e. the normalised _p when the last call was a

@@ -713,7 +713,7 @@ static int spare_slot(const cg_ctx* c) { return c->sC == 3 ? 2 : 3; }  // of the
 
 // After fused steps of the shift build: gives _a and _f registers of their own
 // (copies of _p), as the method sequence leaves them.
-static int unalias(cg_ctx* c) {
+int cg::unalias(cg_ctx* c) {
   if (!c->a_is_p || !c->a_raw) return CG_OK;
   if (int rc = ext_resolve(c)) return rc;  // it reads the slots written here
   // _f in slot 1 as everywhere, _a in the stage register that _c leaves
@@ -764,7 +764,7 @@ static void* resolve(cg_ctx* c, const char* name, bool for_write, int* err, size
   if (s.size() < 3 || s[s.size() - 2] != '_') { *err = 1; return nullptr; }
   const std::string base = s.substr(0, s.size() - 2);
   const char r = s.back();
-  if (for_write && (r == 'a' || r == 'f') && unalias(c)) { *err = 2; return nullptr; }
+  if (for_write && r != 'c' && unalias(c)) { *err = 2; return nullptr; }
   auto slot_of = [&](char rr) {
     return rr == 'p' ? c->sP : rr == 'f' ? (c->a_is_p ? c->sP : c->sF) : rr == 'a' ? (c->a_is_p ? c->sP : c->sA)
            : rr == 'c' ? c->sC : -1;

@@ -195,6 +195,7 @@ int cg_ics_static_dust(cg_ctx* c, const double* modes, size_t n_modes, double rm
   const long n = c->npts, nspec = (long)nx * ny * nzc;
   if ((long)n_modes != 2 * nspec) return fail(c, CG_ERR_ARG, "modes must hold nx*ny*(nz/2+1) complex values");
   if (int rc = ext_resolve(c)) return rc;
+  if (int rc = unalias(c)) return rc;
   const double rho_bar = 3.0 / (8.0 * kPi);
   hipStream_t s = c->stream;
   Scratch w;

@@ -182,7 +182,9 @@ struct cg_ctx {
   // a_is_p after fused steps of the shift build, which stand for the method
   // sequence: its _a is the step's result as it is (the constraints and the
   // SVT pass read it without stepInit's normalisation), and _a, _f and the
-  // method calls can be used at once (unalias)
+  // method calls can be used at once (unalias).  The method sequence's _a and
+  // _f are registers of their own: a write to _p leaves them, and what is
+  // evaluated from _a, as they were.
   bool a_raw = false;
   std::string err;
   bool timing = false;
@@ -211,6 +213,9 @@ double variant_weight(const StageVariant& v, bool dma);
 bool alpha_live(const cg_ctx* c);
 StageArgs make_args(cg_ctx* c, int stage, int rin, int rp, int rf, int rout, int normalize);
 int ext_resolve(cg_ctx* c);
+// after fused steps of the shift build: _a and _f registers of their own,
+// before anything is written to them or to _p (cg_ctx::a_raw)
+int unalias(cg_ctx* c);
 // device array of a field-map name for reading (err 1: unknown, 3: filled by cg_constraints)
 const void* field_ptr(cg_ctx* c, const char* name, size_t* esz, int* err);
 // the gauge pass (gauge.hip): shift terms, shift registers and the lapses

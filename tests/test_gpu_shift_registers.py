@@ -79,3 +79,60 @@ def test_no_steps_keep_averages(gpu, shift):
         ext.append(g.extra_field_data())
         assert ext[-1] != before
     assert ext[0] == ext[1]
+
+
+def evaluations(g):
+    """What is formed from _a and _f after the state changed under them."""
+    c = g.setConstraintCalcs()
+    spec = g.power_spectrum("DIFFphi_a")
+    regs = registers(g, "pa")
+    g.RKEvolve()
+    regs.update(registers(g, "c"))
+    g.K1Finalize()
+    regs.update({k + " K1": v for k, v in registers(g, "fc").items()})
+    return c, spec, regs
+
+
+def compare_evaluations(a, b):
+    # H and M are about 1e-3 of the terms they are the difference of
+    for k in ("H", "M"):
+        assert np.all(np.abs(np.array(a[0][k]) - np.array(b[0][k])) <= 1e-8 * np.abs(b[0][k])), k
+    assert np.all(np.abs(a[1] - b[1]) <= 1e-10 * np.abs(b[1]) + 1e-18 * np.abs(b[1]).max())
+    same(a[2], b[2], 1e-10)
+
+
+def test_upload_of_p_leaves_a_and_f(gpu):
+    """An upload to _p between steps changes neither _a nor _f nor what is
+    evaluated from them."""
+    st, other = shift_state(SHAPE, 5), shift_state(SHAPE, 8)
+    out = []
+    for fused in (True, False):
+        g = context(gpu, fused, st)
+        g.step(2)
+        for f in ("DIFFK", "DIFFphi", "beta2"):
+            g.upload(f + "_p", other[f])
+        ev = evaluations(g)
+        g.step(1)
+        out.append((ev, registers(g, "p")))
+    compare_evaluations(out[0][0], out[1][0])
+    same(out[0][1], out[1][1])
+
+
+def test_device_initial_data_leave_a_and_f(gpu):
+    """The device initial data write _p registers: _a, _f and what is evaluated
+    from them stay those of the last step."""
+    st = shift_state(SHAPE, 5)
+    nx, ny, nz = SHAPE
+    rng = np.random.default_rng(3)
+    modes = np.zeros((nx, ny, nz // 2 + 1), dtype=complex)
+    modes[1:3, 1:3, 1:3] = rng.standard_normal((2, 2, 2)) + 1j * rng.standard_normal((2, 2, 2))
+    out = []
+    for fused in (True, False):
+        g = context(gpu, fused, st)
+        g.step(2)
+        g.ics_static_dust(modes, 1e-3)
+        ev = evaluations(g)
+        g.step(1)
+        out.append((ev, registers(g, "p")))
+    compare_evaluations(out[0][0], out[1][0])
+    same(out[0][1], out[1][1])

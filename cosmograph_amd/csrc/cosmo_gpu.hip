@@ -1201,7 +1201,13 @@ static int dust_flux(cg_ctx* c, int slot, int normalize, int mslot = -1) {
 int cg_step_init(cg_ctx* c) {
   if (!c) return CG_ERR_ARG;
   c->ext_lazy = false;  // superseded by this stepInit's averages
-  if (c->a_is_p) { c->a_is_p = false; c->sA = 2; c->sC = 3; }
+  if (c->a_is_p) {
+    // the shift build's _c (stage 4's input) stays where it is, as the method
+    // sequence leaves it; other fused steps leave no register to keep
+    c->sA = c->a_raw ? spare_slot(c) : 2;
+    if (!c->a_raw) c->sC = 3;
+    c->a_is_p = false;
+  }
   if (c->dreg) {
     c->dust_rk = 0;
     if (int rc = dust_reg_init(c, c->sP, c->sA, c->sF)) return rc;

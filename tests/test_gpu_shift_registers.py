@@ -136,3 +136,25 @@ def test_device_initial_data_leave_a_and_f(gpu):
         out.append((ev, registers(g, "p")))
     compare_evaluations(out[0][0], out[1][0])
     same(out[0][1], out[1][1])
+
+
+def test_step_init_keeps_c(gpu):
+    """stepInit writes _a and _f: _c holds what the last step left there."""
+    st = shift_state(SHAPE, 5)
+    out = []
+    for fused in (True, False):
+        g = context(gpu, fused, st)
+        g.step(2)
+        before = registers(g, "c")
+        g.stepInit()
+        after = registers(g, "c")
+        for k in before:
+            assert np.array_equal(before[k], after[k]), k
+        regs = registers(g, "pafc")
+        for fin in (g.K1Finalize, g.K2Finalize, g.K3Finalize, g.K4Finalize):
+            g.RKEvolve()
+            fin()
+        g.step(1)
+        out.append((regs, registers(g, "pc")))
+    same(out[0][0], out[1][0])
+    same(out[0][1], out[1][1])

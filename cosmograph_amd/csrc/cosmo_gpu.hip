@@ -665,6 +665,8 @@ int cg_create(const cg_params* params, cg_ctx** out) {
   if (c->nxf) {
     HIPCHK(c, hipMalloc((void**)&c->xreg, (size_t)c->nxf * 4 * pad * sizeof(double)));
     HIPCHK(c, hipMemsetAsync(c->xreg, 0, (size_t)c->nxf * 4 * pad * sizeof(double), c->stream));
+    HIPCHK(c, hipHostMalloc((void**)&c->nan_host, sizeof(unsigned long long)));
+    HIPCHK(c, hipEventCreateWithFlags(&c->nan_ev, hipEventDisableTiming));
   }
   if (p.matter == CG_MATTER_DUST) {
     HIPCHK(c, hipMalloc(&c->dreg, (size_t)NDUST * 4 * pad * c->ts));
@@ -690,6 +692,8 @@ int cg_destroy(cg_ctx* c) {
   if (c->flux) (void)hipFree(c->flux);
   if (c->rho_src) (void)hipFree(c->rho_src);
   if (c->xreg) (void)hipFree(c->xreg);
+  if (c->nan_host) (void)hipHostFree(c->nan_host);
+  if (c->nan_ev) (void)hipEventDestroy(c->nan_ev);
   if (c->arena) (void)hipFree(c->arena);
   mq_free(c);
   bardeen_free(c);
@@ -1297,6 +1301,19 @@ int cg_k_finalize(cg_ctx* c, int n) {
 
 constexpr int kMqCheck = 2;
 
+// numNaNs (math.h:1524-1541) of a device array into c->nan_cnt
+static int count_nans(cg_ctx* c, const void* d, size_t esz) {
+  HIPCHK(c, hipMemsetAsync(c->nan_cnt, 0, sizeof(unsigned long long), c->stream));
+  const int bs = 256;
+  const long nb = (c->npts + bs - 1) / bs;
+  if (esz == 8)
+    hipLaunchKernelGGL(k_num_nans<double>, dim3(nb), dim3(bs), 0, c->stream, (const double*)d, c->npts, c->nan_cnt);
+  else
+    hipLaunchKernelGGL(k_num_nans<float>, dim3(nb), dim3(bs), 0, c->stream, (const float*)d, c->npts, c->nan_cnt);
+  HIPCHK(c, hipGetLastError());
+  return CG_OK;
+}
+
 int cg_rk4_steps(cg_ctx* c, int nsteps) {
   if (!c || nsteps < 0) return CG_ERR_ARG;
   c->svar = shift_variant(c);
@@ -1370,6 +1387,33 @@ int cg_rk4_steps(cg_ctx* c, int nsteps) {
     int rc = launch(c, a, c->svar);
     return (rc || !flrw) ? rc : ext_combine(c, c->last_rows, false);
   };
+  // The method sequence's NaN guard in the shift build's fused steps: a step
+  // does not change a state whose DIFFphi holds a NaN.  _p and the FRW values
+  // are first written by stage 4, so the count of the state a step starts from
+  // is waited for there, with the stages before it already queued: the guard
+  // costs one small copy per step and no gap (waiting for it before stage 1
+  // leaves the device idle while the host returns).
+  auto guard_begin = [&](bool first) -> int {
+    if (first) {
+      if (int rc = count_nans(c, reg_ptr(c, PHI, 0), 8)) return rc;
+      HIPCHK(c, hipMemcpyAsync(c->nan_host, c->nan_cnt, sizeof(*c->nan_host), hipMemcpyDeviceToHost, c->stream));
+    } else {  // stage 4 of the step before counted them
+      *c->nan_host = 0;
+      HIPCHK(c, hipMemcpyAsync(c->nan_host, c->nan_dev, sizeof(unsigned), hipMemcpyDeviceToHost, c->stream));
+    }
+    HIPCHK(c, hipEventRecord(c->nan_ev, c->stream));
+    return CG_OK;
+  };
+  auto guard_end = [&](bool first, const Frw& before) -> int {
+    HIPCHK(c, hipEventSynchronize(c->nan_ev));
+    const unsigned long long nn = *c->nan_host;
+    if (nn == (first ? 0 : c->nan_seen)) return CG_OK;
+    if (!first) c->nan_seen = (unsigned)nn;
+    // the registers as the guard finds them, after stepInit
+    c->frw = before;
+    if (int rc = cg_step_init(c)) return rc;
+    return fail(c, CG_ERR_NAN, "NAN detected in DIFFphi");
+  };
   // With DMA staging, stage 4 also writes the normalised copy of the new
   // state (stepInit's _a) into the dead slot Y, so that the next step's
   // stage 1 runs the DMA kernel instead of normalising halos on the fly.
@@ -1382,6 +1426,8 @@ int cg_rk4_steps(cg_ctx* c, int nsteps) {
     if (c->mq && s % kMqCheck == 0 && (rc = mq_check(c))) return rc;
     c->sP = 0; c->sF = 1;
     c->ext_lazy = false;  // this step writes the slots they are formed from
+    const Frw frw0 = c->frw;
+    if (shift && (rc = guard_begin(s == 0))) return rc;
     const bool pre = c->p.normalize_metric && s + 1 < nsteps &&
                      (shift || (c->var && c->dma_allowed && c->dma_pick && dma_fits(c, *c->var)));
     if ((ko_norm || (shift && c->p.normalize_metric)) && !have_norm) {
@@ -1420,6 +1466,7 @@ int cg_rk4_steps(cg_ctx* c, int nsteps) {
     if ((rc = have_norm ? stage(1, 0, X, 0, Y) : stage(1, 0, X, c->p.normalize_metric))) return rc;
     if ((rc = stage(2, X, Y, 0))) return rc;
     if ((rc = stage(3, Y, X, 0))) return rc;
+    if (shift && (rc = guard_end(s == 0, frw0))) return rc;
     if ((rc = stage(4, X, 0, 0, -1, pre ? Y : -1))) return rc;
     have_norm = pre;
     c->sA = 0; c->sC = X; c->a_is_p = true; c->a_raw = shift;
@@ -1462,14 +1509,7 @@ int cg_num_nans(cg_ctx* c, const char* name, long long* count) {
     *count = 0;
     return CG_OK;
   }
-  HIPCHK(c, hipMemsetAsync(c->nan_cnt, 0, sizeof(unsigned long long), c->stream));
-  const int bs = 256;
-  const long nb = (c->npts + bs - 1) / bs;
-  if (esz == 8)
-    hipLaunchKernelGGL(k_num_nans<double>, dim3(nb), dim3(bs), 0, c->stream, (const double*)d, c->npts, c->nan_cnt);
-  else
-    hipLaunchKernelGGL(k_num_nans<float>, dim3(nb), dim3(bs), 0, c->stream, (const float*)d, c->npts, c->nan_cnt);
-  HIPCHK(c, hipGetLastError());
+  if (int rc = count_nans(c, d, esz)) return rc;
   unsigned long long n = 0;
   HIPCHK(c, hipMemcpyAsync(&n, c->nan_cnt, sizeof n, hipMemcpyDeviceToHost, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));

@@ -173,6 +173,9 @@ struct cg_ctx {
   SrcArgs ext_lazy_src{};
   double ext_lazy_phiF = 0;
   unsigned long long* nan_cnt = nullptr;  // numNaNs counter
+  // shift build: a NaN count on its way to the host (pinned), and its arrival
+  unsigned long long* nan_host = nullptr;
+  hipEvent_t nan_ev = nullptr;
   hipStream_t stream = nullptr;
   Frw frw;
   double lambda = 0;

@@ -1526,6 +1526,11 @@ int cg_sync(cg_ctx* c) {
 int cg_kernel_info(const cg_ctx* cc, int* vgprs, int* scratch, int* lds, int* ti, int* tj, int* tk) {
   cg_ctx* c = const_cast<cg_ctx*>(cc);
   if (!c) return CG_ERR_ARG;
+  if (const StageVariant* v = shift_variant(c)) {
+    const int rc = v->info_dma(vgprs, scratch, lds);
+    *ti = v->ti; *tj = v->tj; *tk = v->tk;
+    return rc ? CG_ERR_HIP : CG_OK;
+  }
   if (!c->var || c->var->live_alpha != alpha_live(c)) c->var = pick_variant(c);
   if (!c->var) return fail(c, CG_ERR_ARG, "no stage kernel variant fits this grid/order");
   const bool dma = c->dma_allowed && c->dma_pick && dma_fits(c, *c->var);

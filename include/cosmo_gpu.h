@@ -255,7 +255,9 @@ int cg_set_dust_background(cg_ctx* ctx, int on);
 /* Synchronise the context's stream. */
 int cg_sync(cg_ctx* ctx);
 
-/* Kernel resource usage of the stage kernel this context launches. */
+/* Kernel resource usage of the stage kernel that cg_rk4_steps launches: of the
+ * fused steps where the shift build has them (cg_set_dma), else the one that
+ * the method sequence launches too. */
 int cg_kernel_info(const cg_ctx* ctx, int* vgprs, int* scratch_bytes, int* lds_bytes,
                    int* tile_i, int* tile_j, int* tile_k);
 

@@ -1,0 +1,81 @@
+"""Which kernels run: the fused steps of the shift build have a stage kernel of
+their own, so kernel_info tells whether a context has them; and the two forms
+of the constraint kernel split the grid into other tiles, so their sums differ
+in the last bits.  These hold for the contexts of the tests that compare the
+forms with each other, which would pass if both sides ran the same one."""
+import numpy as np
+import pytest
+
+from common import FIELDS, smooth_random_state
+from test_gpu_shift_fused import CASES as FUSED
+from test_gpu_dma_even import _start
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def gpu():
+    import cosmograph_amd as cg
+    cg.load_library()
+    return cg
+
+
+def infos(gpu, shape, shift, order, lapse, prec="fp64", ko=0.0):
+    """kernel_info of the shift context (DMA staging on, off) and of a context
+    without a shift on the same grid."""
+    def one(s, dma):
+        g = gpu.BSSN(gpu.GpuParams(n=shape, order=order, lapse=lapse, shift=s, precision=prec, ko_coeff=ko))
+        if lapse == "Static":
+            g.upload("DIFFalpha_p", np.full(shape, 1e-3))  # as the tests that use these cases: a lapse that is not 1
+        g.set_dma(dma)
+        return g.kernel_info()
+    return one(shift, True), one(shift, False), one("none", True), one("none", False)
+
+
+# the tests of the fused steps
+EVEN = [((18, 14, 22), "GammaDriver", 4, "OnePlusLog", "fp64", 0.0), ((9, 11, 34), "GammaDriver", 6, "OnePlusLog", "fp64", 0.0),
+        ((16, 16, 30), "GammaDriver", 2, "OnePlusLog", "fp64", 0.0)]
+REGISTERS = [((18, 14, 20), "GammaDriver", 4, "OnePlusLog", "fp64", 0.0), ((18, 14, 20), "Static", 4, "OnePlusLog", "fp64", 0.0)]
+
+
+@pytest.mark.parametrize("shape,shift,order,lapse,prec,ko", FUSED + EVEN + REGISTERS)
+def test_fused_kernel_runs(gpu, shape, shift, order, lapse, prec, ko):
+    on, off, plain_on, plain_off = infos(gpu, shape, shift, order, lapse, prec, ko)
+    assert on["tile"] == (4, 4, 16)
+    assert on != plain_on and on != off
+    assert off == plain_off
+
+
+def test_fused_kernel_of_a_frozen_lapse(gpu):
+    def one(shift, dma):
+        g = gpu.BSSN(gpu.GpuParams(n=(18, 14, 20), order=4, lapse="Static", shift=shift, normalize_metric=0))
+        g.set_dma(dma)
+        return g.kernel_info()
+    assert one("GammaDriver", True) != one("none", True)
+    assert one("GammaDriver", True) != one("GammaDriver", False)
+
+
+# other fields' complete right-hand sides; a halo of 4; rows that are no whole 16-byte groups; fewer points than a tile needs
+@pytest.mark.parametrize("shape,shift,order,lapse,prec", [((18, 14, 20), "AijDriverShift", 4, "OnePlusLog", "fp64"),
+                                                          ((18, 14, 20), "GammaDriver", 4, "TestKDriverLapse", "fp64"),
+                                                          ((18, 18, 24), "GammaDriver", 8, "OnePlusLog", "fp64"),
+                                                          ((18, 14, 21), "GammaDriver", 4, "OnePlusLog", "fp64"),
+                                                          ((18, 14, 22), "GammaDriver", 4, "OnePlusLog", "fp32_split"),
+                                                          ((18, 14, 18), "GammaDriver", 4, "OnePlusLog", "fp64")])
+def test_no_fused_kernel(gpu, shape, shift, order, lapse, prec):
+    on, off, plain_on, plain_off = infos(gpu, shape, shift, order, lapse, prec)
+    assert on == plain_on and off == plain_off
+
+
+@pytest.mark.parametrize("order,shape,dma_form", [(4, (17, 13, 22), True), (6, (18, 14, 34), True), (4, (17, 13, 21), False)])
+def test_constraint_forms(gpu, order, shape, dma_form):
+    st = smooth_random_state(shape, seed=9)
+    res = []
+    for dma in (True, False):
+        g = gpu.BSSN(gpu.GpuParams(n=shape, order=order))
+        g.set_dma(dma)
+        _start(g, st, FIELDS)
+        g.stepInit()
+        res.append(g.setConstraintCalcs())
+    equal = all(np.array_equal(res[0][k], res[1][k]) for k in ("H", "M", "G"))
+    assert equal == (not dma_form)

@@ -1022,11 +1022,13 @@ StageArgs make_args(cg_ctx* c, int stage, int rin, int rp, int rf, int rout, int
 }  // namespace cg
 
 // the stage kernel of the shift build's fused steps, or null where the grid,
-// the order or the gauge has none (the method sequence then runs)
+// the order, the gauge or the tile the caller asked for has none (the method
+// sequence then runs).  The autotuner's choice (req_ti) is among the other
+// kernels and decides nothing here.
 static const StageVariant* shift_variant(const cg_ctx* c) {
   if (!gauge_fusable(c)) return nullptr;
   for (const auto& v : shift_variants())
-    if (v.prec == c->prec && v.order == c->p.stencil_order && v.halo == c->H && v.live_alpha == alpha_live(c) &&
+    if ((c->p.tile_i <= 0 || (v.ti == c->p.tile_i && v.tj == c->p.tile_j && v.tk == c->p.tile_k)) && v.prec == c->prec && v.order == c->p.stencil_order && v.halo == c->H && v.live_alpha == alpha_live(c) &&
         variant_fits(c, v) && dma_fits(c, v))
       return &v;
   return nullptr;

@@ -6,9 +6,10 @@ forms with each other, which would pass if both sides ran the same one."""
 import numpy as np
 import pytest
 
-from common import FIELDS, smooth_random_state
+from common import FIELDS, rel_l2, smooth_random_state
 from test_gpu_shift_fused import CASES as FUSED
 from test_gpu_dma_even import _start
+from test_gpu_shift import X_ALL, shift_state
 
 pytestmark = pytest.mark.gpu
 
@@ -79,3 +80,33 @@ def test_constraint_forms(gpu, order, shape, dma_form):
         res.append(g.setConstraintCalcs())
     equal = all(np.array_equal(res[0][k], res[1][k]) for k in ("H", "M", "G"))
     assert equal == (not dma_form)
+
+
+def test_requested_tile(gpu):
+    """A tile asked for at creation is the one that runs (the method sequence
+    where the fused steps have no such tile), or an error where nothing has it."""
+    shape, st = (18, 14, 20), shift_state((18, 14, 20), 5)
+
+    def ctx(tile, shift="GammaDriver"):
+        g = gpu.BSSN(gpu.GpuParams(n=shape, order=4, lapse="OnePlusLog", shift=shift, gd_eta=0.4, tile=tile))
+        _start(g, st, FIELDS + (X_ALL if shift != "none" else []))
+        return g
+
+    fused = ctx((4, 4, 16)).kernel_info()
+    assert fused == ctx((0, 0, 0)).kernel_info() and fused != ctx((4, 4, 16), "none").kernel_info()
+    g = ctx((4, 8, 8))
+    assert g.kernel_info() == ctx((4, 8, 8), "none").kernel_info()
+    g.step(2)
+    h = ctx((0, 0, 0))
+    h.set_dma(False)  # the method sequence
+    h.step(2)
+    for f in FIELDS + X_ALL:
+        assert rel_l2(g.download(f + "_p"), h.download(f + "_p")) <= 1e-12, f
+    for shift in ("none", "GammaDriver"):
+        with pytest.raises(gpu.CosmoGpuError) as e:
+            ctx((4, 4, 4), shift).step(1)
+        assert e.value.code == -1  # CG_ERR_ARG
+    # the autotuner's pick is no request
+    a = ctx((0, 0, 0))
+    a.autotune(1)
+    assert a.kernel_info() == fused

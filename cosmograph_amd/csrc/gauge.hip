@@ -896,8 +896,10 @@ int gauge_terms(cg_ctx* c, const StageArgs& st) {
   g.s_p = st.s_p; g.s_f = st.s_f; g.s_xout = st.s_out; g.stage = st.stage;
   g.cf = st.cf; g.ca = st.ca;
   g.live_alpha = alpha_live(c) ? 1 : 0;
-  if (!g.live_alpha && g.need_alpha && c->p.shift != SHIFT_DAMPED_WAVE) {
-    g.need_alpha = 0;  // a lapse identically 1: nothing to advect
+  if (!g.live_alpha && g.need_alpha) {
+    // a lapse identically 1 has no derivatives.  The kernel takes every array
+    // that is staged (next()), so that none is in flight when it ends.
+    g.need_alpha = 0;
     g.nseq -= 1;
   }
   auto go = [&](auto ts, auto r) {

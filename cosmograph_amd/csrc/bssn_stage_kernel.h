@@ -1668,7 +1668,9 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
         }
       };
       auto run = [&](auto kind) { epilogue(kind); };
-      if (st == 0) run(std::integral_constant<int, EP_RHS>{});
+      // (the shift build's kernels run stages 1-4 only: a right-hand side alone
+      // comes from the others and the gauge pass)
+      if (!SHIFT && st == 0) run(std::integral_constant<int, SHIFT ? EP_ACC : EP_RHS>{});
       else if (!SHIFT && a.incr && st != 4) run(std::integral_constant<int, SHIFT ? EP_ACC : EP_INC>{});
       else if (!SHIFT && a.incr) run(std::integral_constant<int, SHIFT ? EP_ACC : EP_INC4>{});
       else if (st == 1) run(std::integral_constant<int, EP_ACC1>{});

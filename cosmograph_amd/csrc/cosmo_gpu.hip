@@ -505,29 +505,54 @@ double tiled_points(const cg_ctx* c, const StageVariant& v) {
   return up(c->p.nx, v.ti) * up(c->p.ny, v.tj) * up(c->p.nz, v.tk);
 }
 
-// Relative time per tiled point, measured with the autotuner on grids whose
-// extents are multiples of 16 (ms per stage):
-//   LDS-DMA: 4x4x16 is the fastest tile, or within 2% of it: rows of 64 or
-//     128 bytes along k, and the smallest halo of the 256-point tiles.  128^3
-//     FP64, order 4: 4x4x16 0.283, 2x8x16 0.278, 4x8x8 0.314; order 6: 0.329,
-//     0.336, 0.368.  256^3 fixed point, order 6: 1.51, 4x8x8 1.79.  96^3
-//     FP64, order 8: 0.217, 8x8x8 0.242.
-//   Register staging: FP64 order 4 0.372, 0.377, 4x8x8 0.386; order 6 0.453,
-//     0.464, 0.455; split order 6 (101x90x118) 0.208, 0.256, 0.217; order 8
-//     (LDS-bound occupancy): FP64 4x4x16 0.343, 4x8x8 0.360, 8x8x8 0.273,
-//     split 0.334, 0.210, 0.247.
-//   Halo 5 (KO at order 8), FP64, 96^3: 8x8x8 0.457 (DMA), 0.537 (register),
-//     4x8x8 0.650.
+// Relative time per tiled point, in units of the LDS-DMA 4x4x16 kernel of the
+// same precision and order (of the DMA 8x8x8 one at halo 5, where that is the
+// only one).  Ratios of the autotuner's mean stage time in tile order 5,
+// frozen / live lapse, at 128^3 (orders 4, 6) and 96^3 (2, 8), where every
+// tile divides the grid; register staging was measured there too and has the
+// same ratios among its tiles on 127x128x125 and 95x96x97.
+//   LDS-DMA                4x8x8          2x8x16         8x8x8
+//     FP64 order 4, 6      1.13/1.08, 1.23/1.15   1.10/1.05, 1.12/1.12
+//     FP64 order 8                                       1.13/1.14
+//     split order 4, 6     1.21/1.22, 1.25/1.20   1.05/1.06, 1.23/1.06
+//     split order 8                                      1.51/1.49
+//     4-byte order 4, 6    1.27/1.40, 1.28/1.43
+//   Register staging       4x4x16         4x8x8          2x8x16, 8x8x8
+//     FP64 order 2         1.24/1.22      1.36/1.81 (1 wave)
+//     FP64 order 4         1.31/1.26      1.46/1.39      1.37/1.46
+//     FP64 order 6         1.40/1.46      1.49/1.48      1.45/1.62
+//     FP64 order 8         1.45/1.49      1.59/1.53 (1)  1.25/1.29
+//     FP64 halo 5                         1.84/1.49 (1)  1.48/1.34
+//     split order 2        1.05/1.03      1.26/1.23 (1)
+//     split order 4        1.18/1.07      1.41/1.28      1.23/1.11, 1.92/1.75
+//     split order 6        1.34/1.15      1.50/1.32      1.60/1.39, 2.03/1.76
+//     split order 8        2.20/2.22      1.49/1.49 (1)  1.73/1.72
+//     split halo 5                        1.90/1.91 (1)  1.24/1.26
+//     4-byte order 4       1.30/1.79      1.61/1.54      (1.23/1.69, 1.43/1.51 all-FP32)
+//     4-byte order 6       1.58/1.52      1.75/1.69
+// The live-lapse 4-byte kernel of order 4 spills 22 registers at the budget
+// of four waves with register staging, and only there.  (1): compiled for one
+// wave per SIMD; at orders 4 and 6 that budget costs the live FP64 kernels
+// another 30% and is no faster anywhere.
 double variant_weight(const StageVariant& v, bool dma) {
-  const bool f64 = v.prec == CG_FP64;
+  const bool f64 = v.prec == CG_FP64, split = v.prec == CG_FP32_SPLIT, wide = v.halo >= 4;
+  const bool t4416 = v.ti == 4 && v.tj == 4, t2816 = v.ti == 2, t888 = v.ti == 8;  // else 4x8x8
+  if (dma) {
+    if (t4416) return 1.0;
+    if (t2816) return 1.1;
+    if (t888) return v.halo > 4 ? 1.0 : f64 ? 1.13 : 1.5;
+    return f64 ? 1.15 : 1.25;
+  }
   double w;
-  if (v.ti == 4 && v.tj == 4) w = 1.0;
-  else if (v.ti == 2) w = dma ? 1.02 : f64 ? 1.03 : 1.2;
-  else if (v.ti == 8) w = dma ? 1.15 : v.halo >= 4 && f64 ? 0.8 : 1.3;
-  else w = dma ? 1.15 : v.halo >= 4 && !f64 ? 0.7 : 1.04;
-  if (!dma) w *= 1.35;  // register staging against LDS-DMA: 1.31 to 1.65 in the figures above
-  // a register budget for one wave per SIMD only pays where nothing else fits
-  return v.wpe == 1 ? 1.02 * w : w;
+  if (wide) w = t888 ? (v.halo > 4 ? (f64 ? 1.4 : 1.25) : f64 ? 1.27 : 1.73)
+                : t4416 ? (f64 ? 1.47 : 2.2)
+                        : (v.halo > 4 ? (f64 ? 1.65 : 1.9) : f64 ? 1.56 : 1.49);
+  else if (t4416) w = f64 ? 1.35 : split ? 1.2 : v.order == 4 ? (v.live_alpha ? 1.75 : 1.3) : 1.55;
+  else if (t2816) w = 1.45;
+  else if (t888) w = 1.9;
+  else w = f64 ? 1.47 : split ? 1.4 : v.order == 4 ? 1.55 : 1.7;
+  if (v.wpe == 1 && !wide) w *= f64 && v.live_alpha ? 1.3 : 1.02;
+  return w;
 }
 
 // tile order 3 (Morton columns) needs power-of-two tile counts along i and j

@@ -17,6 +17,7 @@
 
 #include "../../include/cosmo_gpu.h"
 #include "bssn_stage.h"
+#include "fftplan.h"
 #include "runtime.h"
 #include "stencil.h"
 
@@ -622,6 +623,7 @@ int cg_create(const cg_params* params, cg_ctx** out) {
   if (p.shift != CG_SHIFT_NONE && p.matter == CG_MATTER_DUST) return CG_ERR_ARG;  // shift build: BSSN + static dust
   if (!(p.dx > 0) || !std::isfinite(p.dt)) return CG_ERR_ARG;
   cg_ctx* c = new cg_ctx();
+  fft_pool_enter();
   c->p = p;
   c->prec = p.precision;
   c->ts = p.precision == CG_FP64 ? 8 : 4;
@@ -723,6 +725,7 @@ int cg_destroy(cg_ctx* c) {
   mq_free(c);
   bardeen_free(c);
   if (c->stream) (void)hipStreamDestroy(c->stream);
+  fft_pool_leave();
   delete c;
   return CG_OK;
 }

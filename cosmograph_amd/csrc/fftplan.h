@@ -7,7 +7,9 @@
 // any number of threads and streams may hold plans of one size.  The pool
 // holds at most kIdlePlans unused plans of the process, the oldest is
 // destroyed first, and none of them holds a work area: that is allocated by
-// the FftPlan and freed with it.
+// the FftPlan and freed with it.  Contexts are counted: with the last one the
+// unused plans go too, so a program that has destroyed its contexts holds
+// nothing on the device.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <hipfft/hipfft.h>
@@ -15,6 +17,9 @@
 #include "runtime.h"
 
 namespace cg {
+
+void fft_pool_enter();  // a context begins
+void fft_pool_leave();  // a context, its FftPlans put back, ends
 
 class FftPlan {
  public:

@@ -15,6 +15,7 @@ struct Idle {
   hipfftHandle h;
 };
 std::mutex g_mu;
+int g_contexts = 0;
 // never destroyed: at process end the runtime may already be gone
 std::vector<Idle>& idle() {
   static std::vector<Idle>* v = new std::vector<Idle>();
@@ -22,6 +23,29 @@ std::vector<Idle>& idle() {
 }
 
 }  // namespace
+
+void fft_pool_enter() {
+  std::lock_guard<std::mutex> lock(g_mu);
+  idle().reserve(kIdlePlans + 1);  // put_back, which a destructor calls, does not allocate
+  ++g_contexts;
+}
+
+void fft_pool_leave() {
+  std::vector<Idle> drop;
+  {
+    std::lock_guard<std::mutex> lock(g_mu);
+    if (--g_contexts > 0) return;
+    drop.swap(idle());
+  }
+  if (drop.empty()) return;
+  int dev = 0;
+  const bool have_dev = hipGetDevice(&dev) == hipSuccess;
+  for (const Idle& e : drop) {
+    (void)hipSetDevice(e.key[0]);
+    (void)hipfftDestroy(e.h);
+  }
+  if (have_dev) (void)hipSetDevice(dev);
+}
 
 int FftPlan::take(cg_ctx* c, hipfftType type, hipStream_t s) {
   put_back();

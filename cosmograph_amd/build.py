@@ -23,7 +23,7 @@ HIP_FLAGS = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}",
              "-Wno-unused-result"]
 # The fixed-point stage kernel has exactly the 128 registers that four blocks a
 # CU leave it.  Pairing its LDS reads (ds_read2) needs a base address each and
-# spills four of them: 1.60 ms a stage at 256^3, 1.54 ms with single reads.  The
+# spills four of them: 1.60 ms a stage at 256^3, 1.51 ms with single reads.  The
 # other kernels are no faster without the pairs, so they keep them.
 FILE_FLAGS = {"stage_inst_f32fix.hip": ["-Xclang", "-target-feature", "-Xclang", "-load-store-opt"]}
 SOURCES = ["stage_inst_f32.hip", "stage_inst_f32all.hip", "stage_inst_f32fix.hip", "stage_inst_f64.hip", "stage_inst_misc.hip", "stage_inst_dust.hip", "stage_inst_dustfix.hip", "stage_inst_shift.hip", "cons_inst.hip",

@@ -733,9 +733,10 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
   // remaining fields are staged only the sums below stay live.  The kernels
   // are bound by how many waves their registers allow: with the whole
   // algebra after the last field, the FP64 kernel held 256 VGPRs and spilled
-  // 188 B (0.421 ms per stage at 128^3, order 4; now 242, no spill, 0.285
-  // ms), the fixed-point one 157 (1.62 ms at 256^3, order 6; now 126, four
-  // waves).
+  // 188 B (0.421 ms per stage at 128^3, order 4; now 236, no spill, 0.302
+  // ms), the fixed-point one 157 (1.62 ms at 256^3, order 6; now 127, four
+  // waves, 1.505 ms).  With a live lapse the FP64 kernels still hold 256 and
+  // spill 52 to 64 B (4x4x16, orders 2 to 6 without KO).
   TC GL[3][6], G[3][6], Gd[3];
   TC Ac[6], AijAij = TC(0), second[3];  // A^ij, A_ij A^ij, Gamma^i_jk A^jk + 6 A^ij d_j phi
   TC DDa[6], DDaTR = TC(0);             // (D_i D_j alpha)^TF and its trace (without e^{-4 phi})
@@ -1515,10 +1516,11 @@ __device__ __forceinline__ void stage_body(const StageArgs& a, const int t, cons
       // EP_RHS (stage 0), EP_INC / EP_INC4 (accumulator-free stages 1-3, 4),
       // EP_ACC1 / EP_ACC / EP_ACC4 (with _f: stage 1, 2-3, 4).
       // With the sums in units of their first weight, the three-operand
-      // additions and the wrap by minima (4210 to 3976 VALU instructions in
-      // the order-6 fixed-point kernel) a stage takes 1.51 ms at 256^3 instead
-      // of 1.64, FP64 at 128^3 0.324 instead of 0.336, dust at 192^3 0.987
-      // instead of 1.036.
+      // additions and the wrap by minima (from 4210 to 3976 VALU instructions
+      // in the code of the order-6 fixed-point kernel, all its epilogues
+      // counted; a wave executes 2270) a stage took 1.51 ms at 256^3 instead of
+      // 1.64, FP64 order 4 at 128^3 0.324 instead of 0.336, dust at 192^3 0.987
+      // instead of 1.036, each pair on one card; now 1.505, 0.302 and 0.962.
       bool saturated = false;
       auto epilogue = [&](auto kind_tag) {
         constexpr int EP = decltype(kind_tag)::value;

@@ -482,13 +482,14 @@ bool variant_fits(const cg_ctx* c, const StageVariant& v) {
 
 // the LDS-DMA twin of v applies to this grid: compiled, rows of whole 16-byte
 // groups, which then never straddle the periodic wrap (nz a multiple of 2 in
-// FP64, of 4 where any field has 4 bytes; FP64 128x128x126, order 4: 0.337 ms a
-// stage against 0.384 with register staging; the split kernels that move their
+// FP64, of 4 where any field has 4 bytes; FP64 128x128x126, order 4: 0.288 ms a
+// stage against 0.357 with register staging; the split kernels that move their
 // FP32 fields in single words need a multiple of 2 and are for the grids that
 // quads do not fit), and one wrap of the k halo (rounded up to 4) suffices; the
 // 4-byte dust kernels address the three fluxes of a quantity from the first
 // one, and the kernels with every field in 4 bytes Gamma^1 and Gamma^3 from K
-// and Gamma^2, with a 32-bit byte offset; their halo offsets are formed with 24-bit multiplies (nx * ny < 2^24)
+// and Gamma^2, with a 32-bit byte offset; their halo offsets are formed with
+// 24-bit multiplies (nx * ny < 2^24)
 bool dma_fits(const cg_ctx* c, const StageVariant& v) {
   if (!v.launch_dma) return false;
   if ((long long)c->p.nx * c->p.ny >= (1ll << 24)) return false;

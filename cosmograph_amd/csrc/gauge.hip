@@ -427,8 +427,10 @@ __global__ void __launch_bounds__(GNT) __attribute__((amdgpu_waves_per_eu(2))) k
 // the axes only and staged in three parts, each with the halo of one axis.
 // Two blocks of 4 waves per CU (57.6 KB of LDS, 2 waves per SIMD), where one
 // 512-thread block of the 8x8x8 tile left the CU idle at each of its barriers:
-// 0.297 ms per launch at 112^3, order 4, FP64, against 0.529 ms, and without
-// the 0.28 ms of the finalize passes.  Orders 2, 4 and 6 (halo 3), rows of whole 16-byte groups.
+// 0.296 ms per launch at 112^3, order 4, FP64, against 0.529 ms, and without
+// the 0.28 ms of the finalize passes.  It needs 59 FP64 words per point (0.66
+// GB there) and moves 1.04 GB, the halos among them: 3.5 TB/s, 2.2 times what
+// its bytes would take at the rate of a large copy.  Orders 2, 4 and 6 (halo 3), rows of whole 16-byte groups.
 constexpr int TTI = 4, TTJ = 4, TTK = 16, TNT = TTI * TTJ * TTK, TH = 3, TKH = 4;
 template <typename E>
 __device__ __forceinline__ double el(const void* T, int c) {

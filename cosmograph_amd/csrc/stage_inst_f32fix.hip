@@ -16,9 +16,11 @@ namespace cg {
   REG(float, float, 3, R, R, TI, TJ, TK, WPE, true)
 CG_F32Q(CG_REGISTER_MQ, 2, 4, 8, 8, 1)
 CG_F32Q(CG_REGISTER_MQ_D, 2, 4, 8, 8, 3)
-// 4 waves per SIMD: the frozen-lapse kernel is at 126 VGPRs and its 40 KB of
-// LDS let four blocks share a CU (256^3, order 6: 1.535 ms per stage against
-// 1.616 ms at 3 waves with 48 KB)
+// 4 waves per SIMD: the frozen-lapse kernel is at 127 VGPRs and its 40 KB of
+// LDS let four blocks share a CU (256^3, order 6, when this was chosen: 1.535
+// ms per stage against 1.616 ms at 3 waves with 48 KB; now 1.505).  With a live
+// lapse the DMA kernels run three (139 to 140 VGPRs, 41.6 KB), and register
+// staging at order 4 spills (variant_weight).
 CG_F32Q(CG_REGISTER_MQ_D, 2, 4, 4, 16, 4)
 CG_F32Q(CG_REGISTER_MQ, 3, 4, 8, 8, 1)
 CG_F32Q(CG_REGISTER_MQ_D, 3, 4, 8, 8, 3)

@@ -125,7 +125,9 @@ int cg_k_finalize(cg_ctx* ctx, int n);
 /* One or more whole RK4 steps in the StaticSim sequence
  * (sims/static.cc:74-170: initStaticStep + runStaticStep, without output),
  * fused into four stage kernels per step.  Returns CG_ERR_NAN if DIFFphi
- * turned NaN (the guard of sims/sim.cc:179-183). */
+ * turned NaN (the guard of sims/sim.cc:179-183): at the end of the call, all
+ * steps done; with a shift also before a step whose state holds a NaN, which
+ * then stays as it is (_a and _f as stepInit leaves them). */
 int cg_rk4_steps(cg_ctx* ctx, int nsteps);
 
 /* BSSN::setConstraintCalcs (bssn.cc:965-1071) on the _a register as the
@@ -264,16 +266,24 @@ int cg_kernel_info(const cg_ctx* ctx, int* vgprs, int* scratch_bytes, int* lds_b
 /* Project autotuner: times every compiled stage-kernel variant (tile shape x
  * register budget) that fits this grid on the context's own data and keeps
  * the fastest.  The evolved state is untouched; must be called between whole
- * steps.  `report` (optional) receives a JSON list of the timings. */
+ * steps.  `report` (optional) receives a JSON list of the timings.  The fused
+ * steps of the shift build have one kernel, which is not among those timed:
+ * there the choice applies to the method calls (and its tile order to both). */
 int cg_autotune(cg_ctx* ctx, int reps, char* report, size_t report_len);
 
 /* Halo staging of the stage kernel.  on = 1 (default): a launch without
- * stage-1 metric normalisation, on a grid with nz % 4 == 0, uses the
- * kernel's LDS-DMA twin where one is compiled: halo tiles go from memory
- * straight into LDS (global_load_lds), two fields ahead of the one being
+ * stage-1 metric normalisation uses the kernel's LDS-DMA twin where one is
+ * compiled and rows are whole 16-byte groups: nz % 2 == 0 in FP64, nz % 4 == 0
+ * where fields are stored in 4 bytes (in split precision at orders 4 and 6 also
+ * nz % 4 == 2, without the dust fluid).  Halo tiles go from memory straight
+ * into LDS (global_load_lds), two fields ahead of the one being
  * differentiated; the autotuner times both paths and keeps the faster.
  * on = 0: register staging everywhere.  The two paths agree to rounding
  * (the kernels may contract a few multiply-adds differently).
+ * Contexts with a shift: cg_rk4_steps has fused steps at orders 2, 4 and 6 on
+ * such grids (4 bytes: nz % 4 == 0), with nz > 18, nx and ny > 5, tile 4x4x16
+ * or none asked for, and any gauge but AijDriverShift and TestKDriverLapse;
+ * with on = 0, and elsewhere, it runs the method sequence.
  * No counterpart in the reference (its stencils read memory directly). */
 int cg_set_dma(cg_ctx* ctx, int on);
 

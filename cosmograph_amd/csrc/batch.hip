@@ -104,9 +104,9 @@ static const StageVariant* batch_pick(const cg_batch* b) {
   for (const auto& v : stage_variants()) {
     if (!batch_fits(b, v)) continue;
     if (b->req_ti && (v.ti != b->req_ti || v.tj != b->req_tj || v.tk != b->req_tk)) continue;
-    double pts = 0.0;
-    for (auto* c : b->m) pts += tiled_points(c, v);
-    const double t = pts * variant_weight(v, batch_dma_fits(b, v));
+    double tiles = 0.0;
+    for (auto* c : b->m) tiles += (double)tile_count(c, v);
+    const double t = stage_estimate(v, batch_dma_fits(b, v), tiles);
     if (!best || t < least) { best = &v; least = t; }
   }
   return best;

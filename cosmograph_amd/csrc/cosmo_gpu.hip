@@ -502,9 +502,32 @@ bool dma_fits(const cg_ctx* c, const StageVariant& v) {
   return c->p.nz % group == 0 && c->p.nz >= kh && c->p.nz > v.tk + kh - 2;
 }
 
-double tiled_points(const cg_ctx* c, const StageVariant& v) {
-  auto up = [](int n, int t) { return (double)((n + t - 1) / t * t); };
+long tile_count(const cg_ctx* c, const StageVariant& v) {
+  auto up = [](int n, int t) { return (long)((n + t - 1) / t); };
   return up(c->p.nx, v.ti) * up(c->p.ny, v.tj) * up(c->p.nz, v.tk);
+}
+
+// Time of a stage over so many tiles, in units of variant_weight's points: the
+// CUs take a tile each in turn, so it goes by whole rounds of 256 tiles.  From
+// 64^3 up that is the number of points, padding included; below, few rounds
+// decide, and in the only round it is the time of one tile (us a stage):
+//   40x40x39, order 8, live lapse: 125 8x8x8 tiles 46.7, 250 4x8x8 ones 31.3;
+//     with KO 65.4 and 43.5; 24^3, 27 8x8x8 tiles by DMA 30.6, 4x4x16 16.6
+//   43x47x52, FP64 order 4: 528 4x4x16 tiles (three rounds) 24.4, 462 4x8x8 18.1
+// Over 260 random grids of 20 to 137 points a side the default took 1.007 of
+// the best variant's time in the mean, 1.18 at most; by points alone 1.019, 1.8.
+double stage_estimate(const StageVariant& v, bool dma, double tiles) {
+  return variant_weight(v, dma) * (v.ti * v.tj * v.tk) * std::ceil(tiles / 256.0);
+}
+
+// A wave of which no more than 8 lanes lie inside the grid takes up to 1.6
+// times as long as one that is full (why was not found): 20x22x20, order 4,
+// the corner waves of 4x4x16 (2 rows of 4 points) 16.1 us a stage, of 4x8x8
+// 9.8; 20x23x20 (3 rows of 4) 10.0 and 9.8.  It only shows where all tiles run
+// at once: counted as part of a round.
+static double corner_wave(const cg_ctx* c, const StageVariant& v) {
+  const int rows = 64 / v.tk;  // of tk points along k, neighbours along j
+  return ((c->p.ny - 1) % rows + 1) * ((c->p.nz - 1) % v.tk + 1) <= 8 ? 0.35 : 0.0;
 }
 
 // Relative time per tiled point, in units of the LDS-DMA 4x4x16 kernel of the
@@ -535,7 +558,11 @@ double tiled_points(const cg_ctx* c, const StageVariant& v) {
 // The live-lapse 4-byte kernel of order 4 spills 22 registers at the budget
 // of four waves with register staging, and only there.  (1): compiled for one
 // wave per SIMD; at orders 4 and 6 that budget costs the live FP64 kernels
-// another 30% and is no faster anywhere.
+// another 30% and is no faster anywhere.  4x8x8 at halo 5 stands at 2.05: a
+// DMA tile of 8x8x8 takes less than two of its, also with the CU to itself
+// (32^3: FP64 30 us against 38, split 29 against 34).  FP64 order 8 by
+// registers: 4x4x16 stands beside 4x8x8, as their times do where either is
+// taken (32x32x31: 25.7 and 25.5 us, live 28.3 and 28.0; 8x8x8 beyond that).
 double variant_weight(const StageVariant& v, bool dma) {
   const bool f64 = v.prec == CG_FP64, split = v.prec == CG_FP32_SPLIT, wide = v.halo >= 4;
   const bool t4416 = v.ti == 4 && v.tj == 4, t2816 = v.ti == 2, t888 = v.ti == 8;  // else 4x8x8
@@ -547,8 +574,8 @@ double variant_weight(const StageVariant& v, bool dma) {
   }
   double w;
   if (wide) w = t888 ? (v.halo > 4 ? (f64 ? 1.4 : 1.25) : f64 ? 1.27 : 1.73)
-                : t4416 ? (f64 ? 1.47 : 2.2)
-                        : (v.halo > 4 ? (f64 ? 1.65 : 1.9) : f64 ? 1.56 : 1.49);
+                : t4416 ? (f64 ? 1.58 : 2.2)
+                        : (v.halo > 4 ? 2.05 : f64 ? 1.56 : 1.49);
   else if (t4416) w = f64 ? 1.35 : split ? 1.2 : v.order == 4 ? (v.live_alpha ? 1.75 : 1.3) : 1.55;
   else if (t2816) w = 1.45;
   else if (t888) w = 1.9;
@@ -579,15 +606,16 @@ static bool variant_matches(const cg_ctx* c, const StageVariant& v) {
 }
 
 // The variant without an autotuner run: among those that fit (and have the
-// requested tile, if any), the one with the least estimated time of a stage,
-// the points of all its tiles (padding included) times variant_weight.
+// requested tile, if any), the one with the least estimated time of a stage.
 static const StageVariant* pick_variant(const cg_ctx* c) {
   const StageVariant* best = nullptr;
   double least = 0.0;
   for (const auto& v : stage_variants()) {
     if (!variant_matches(c, v)) continue;
     if (c->req_ti && (v.ti != c->req_ti || v.tj != c->req_tj || v.tk != c->req_tk)) continue;
-    const double t = tiled_points(c, v) * variant_weight(v, c->dma_allowed && c->dma_pick && dma_fits(c, v));
+    const bool dma = c->dma_allowed && c->dma_pick && dma_fits(c, v);
+    const double tiles = (double)tile_count(c, v);
+    const double t = stage_estimate(v, dma, tiles) * (1.0 + corner_wave(c, v) / std::ceil(tiles / 256.0));
     if (!best || t < least) { best = &v; least = t; }
   }
   return best;

@@ -210,9 +210,11 @@ int halo_for(int order, double ko);
 bool variant_fits(const cg_ctx* c, const StageVariant& v);
 bool dma_fits(const cg_ctx* c, const StageVariant& v);
 bool morton_fits(int ntx, int nty);
-// default choice of a stage kernel: points of all tiles, and time per tiled point
-double tiled_points(const cg_ctx* c, const StageVariant& v);
+// default choice of a stage kernel: relative time per tiled point, tiles of a
+// grid, and the time of a stage over so many tiles
 double variant_weight(const StageVariant& v, bool dma);
+long tile_count(const cg_ctx* c, const StageVariant& v);
+double stage_estimate(const StageVariant& v, bool dma, double tiles);
 bool alpha_live(const cg_ctx* c);
 StageArgs make_args(cg_ctx* c, int stage, int rin, int rp, int rf, int rout, int normalize);
 int ext_resolve(cg_ctx* c);

@@ -38,7 +38,13 @@ PICKS = [
     ("fp32_split", 8, 0.0, "Static", (32, 32, 32), (4, 4, 16), True), ("fp32_split", 8, 0.0, "Harmonic", (32, 32, 48), (4, 4, 16), True),
     ("fp32_split", 8, 0.05, "Static", (32, 32, 32), (8, 8, 8), True), ("fp32_split", 8, 0.05, "Harmonic", (32, 24, 40), (8, 8, 8), True),
     # ... and where rows are no whole 16-byte groups
-    ("fp32_split", 8, 0.0, "Harmonic", (31, 32, 33), (4, 8, 8), False), ("fp32_split", 8, 0.05, "Harmonic", (31, 32, 33), (8, 8, 8), False),
+    ("fp32_split", 8, 0.0, "Harmonic", (31, 32, 33), (4, 8, 8), False), ("fp32_split", 8, 0.05, "Harmonic", (63, 64, 65), (8, 8, 8), False),
+    # few tiles: a CU to each, so a tile of 512 points loses, and a round more or less decides
+    ("fp64", 8, 0.0, "Static", (24, 24, 24), (4, 4, 16), True), ("fp64", 8, 0.0, "Harmonic", (40, 40, 39), (4, 8, 8), False),
+    ("fp64", 8, 0.05, "Static", (30, 32, 25), (4, 8, 8), False), ("fp64", 8, 0.05, "Harmonic", (63, 64, 65), (8, 8, 8), False),
+    ("fp64", 8, 0.05, "Static", (32, 32, 32), (8, 8, 8), True), ("fp64", 4, 0.0, "Static", (43, 47, 52), (4, 8, 8), True),
+    # ... and corner waves of 8 points: 2 rows of 4 in the 4x4x16 tile, 3 rows of 4 are full speed
+    ("fp64", 4, 0.0, "Static", (20, 22, 20), (4, 8, 8), True), ("fp64", 4, 0.0, "Static", (20, 23, 20), (4, 4, 16), True),
     # order 2: the register budget of several waves outweighs some padding
     ("fp64", 2, 0.0, "Harmonic", (23, 24, 97), (4, 4, 16), False), ("fp32_split", 2, 0.0, "Static", (23, 24, 97), (4, 4, 16), False),
     # four-byte fields by registers, order 4: the kernel for four waves spills with a live lapse

@@ -508,26 +508,31 @@ long tile_count(const cg_ctx* c, const StageVariant& v) {
 }
 
 // Time of a stage over so many tiles, in units of variant_weight's points: the
-// CUs take a tile each in turn, so it goes by whole rounds of 256 tiles.  From
-// 64^3 up that is the number of points, padding included; below, few rounds
-// decide, and in the only round it is the time of one tile (us a stage):
+// CUs take a tile each in turn, so on few tiles it goes by whole rounds of 256,
+// and in the only round it is the time of one tile (us a stage):
 //   40x40x39, order 8, live lapse: 125 8x8x8 tiles 46.7, 250 4x8x8 ones 31.3;
 //     with KO 65.4 and 43.5; 24^3, 27 8x8x8 tiles by DMA 30.6, 4x4x16 16.6
 //   43x47x52, FP64 order 4: 528 4x4x16 tiles (three rounds) 24.4, 462 4x8x8 18.1
-// Over 260 random grids of 20 to 137 points a side the default took 1.007 of
-// the best variant's time in the mean, 1.18 at most; by points alone 1.019, 1.8.
+// Beyond two rounds the tiles of a CU overlap and the last round counts half
+// (59x51x56, split order 4: 780 4x4x16 tiles take 0.89 of the time of 735 4x8x8 ones);
+// from 64^3 up it is the number of points, padding included.  Over 680 random
+// grids of 20 to 111 points a side the default took 1.005 of the best
+// variant's time in the mean, 1.21 at most; by points alone 1.015, 1.82.
 double stage_estimate(const StageVariant& v, bool dma, double tiles) {
-  return variant_weight(v, dma) * (v.ti * v.tj * v.tk) * std::ceil(tiles / 256.0);
+  const double r = tiles / 256.0, up = std::ceil(r);
+  return variant_weight(v, dma) * (v.ti * v.tj * v.tk) * (r <= 2.0 ? up : 0.5 * (r + up));
 }
 
-// A wave of which no more than 8 lanes lie inside the grid takes up to 1.6
-// times as long as one that is full (why was not found): 20x22x20, order 4,
-// the corner waves of 4x4x16 (2 rows of 4 points) 16.1 us a stage, of 4x8x8
-// 9.8; 20x23x20 (3 rows of 4) 10.0 and 9.8.  It only shows where all tiles run
-// at once: counted as part of a round.
-static double corner_wave(const cg_ctx* c, const StageVariant& v) {
+// A wave of which no more than 8 lanes lie inside the grid takes 4 to 6 us
+// longer than a full one, with either staging and at every order (why was not
+// found): 20x22x20, order 4, corner waves of 2 rows of 4 points in the 4x4x16
+// tile 16.1 us a stage, 4x8x8 9.8; 20x23x20 (3 rows of 4) 10.0 and 9.8.  It
+// only shows where all tiles run at once.  In stage_estimate's units, a third
+// of a 4x4x16 tile.
+static double corner_wave(const cg_ctx* c, const StageVariant& v, double tiles) {
   const int rows = 64 / v.tk;  // of tk points along k, neighbours along j
-  return ((c->p.ny - 1) % rows + 1) * ((c->p.nz - 1) % v.tk + 1) <= 8 ? 0.35 : 0.0;
+  const int lanes = ((c->p.ny - 1) % rows + 1) * ((c->p.nz - 1) % v.tk + 1);
+  return tiles <= 256.0 && lanes <= 8 ? 90.0 : 0.0;
 }
 
 // Relative time per tiled point, in units of the LDS-DMA 4x4x16 kernel of the
@@ -615,7 +620,7 @@ static const StageVariant* pick_variant(const cg_ctx* c) {
     if (c->req_ti && (v.ti != c->req_ti || v.tj != c->req_tj || v.tk != c->req_tk)) continue;
     const bool dma = c->dma_allowed && c->dma_pick && dma_fits(c, v);
     const double tiles = (double)tile_count(c, v);
-    const double t = stage_estimate(v, dma, tiles) * (1.0 + corner_wave(c, v) / std::ceil(tiles / 256.0));
+    const double t = stage_estimate(v, dma, tiles) + corner_wave(c, v, tiles);
     if (!best || t < least) { best = &v; least = t; }
   }
   return best;

@@ -43,6 +43,7 @@ PICKS = [
     ("fp64", 8, 0.0, "Static", (24, 24, 24), (4, 4, 16), True), ("fp64", 8, 0.0, "Harmonic", (40, 40, 39), (4, 8, 8), False),
     ("fp64", 8, 0.05, "Static", (30, 32, 25), (4, 8, 8), False), ("fp64", 8, 0.05, "Harmonic", (63, 64, 65), (8, 8, 8), False),
     ("fp64", 8, 0.05, "Static", (32, 32, 32), (8, 8, 8), True), ("fp64", 4, 0.0, "Static", (43, 47, 52), (4, 8, 8), True),
+    ("fp64", 8, 0.0, "Static", (34, 42, 43), (8, 8, 8), False), ("fp32_split", 4, 0.0, "Harmonic", (59, 51, 56), (4, 4, 16), True),
     # ... and corner waves of 8 points: 2 rows of 4 in the 4x4x16 tile, 3 rows of 4 are full speed
     ("fp64", 4, 0.0, "Static", (20, 22, 20), (4, 8, 8), True), ("fp64", 4, 0.0, "Static", (20, 23, 20), (4, 4, 16), True),
     # order 2: the register budget of several waves outweighs some padding

@@ -1,8 +1,9 @@
-"""Which kernels run: the fused steps of the shift build have a stage kernel of
-their own, so kernel_info tells whether a context has them; and the two forms
-of the constraint kernel split the grid into other tiles, so their sums differ
-in the last bits.  These hold for the contexts of the tests that compare the
-forms with each other, which would pass if both sides ran the same one."""
+"""Which kernels run: fused steps of the shift build report a NaN that the last
+step of a call produced, which the method sequence leaves to the next call, and
+kernel_info names their 4x4x16 stage kernel; the two forms of the constraint
+kernel split the grid into other tiles, so their sums differ in the last bits.
+These hold for the contexts of the tests that compare the forms with each
+other, which would pass if both sides ran the same one."""
 import numpy as np
 import pytest
 
@@ -21,16 +22,30 @@ def gpu():
     return cg
 
 
+def steps_fused(gpu, g):
+    """Whether the next step is a fused one (the state is lost)."""
+    k = g.download("DIFFK_p")
+    k[5, 6, 7] = np.nan
+    g.upload("DIFFK_p", k)
+    try:
+        g.step(1)
+    except gpu.CosmoGpuError as e:
+        assert e.code == gpu.ERR_NAN
+        return True
+    return False
+
+
 def infos(gpu, shape, shift, order, lapse, prec="fp64", ko=0.0):
     """kernel_info of the shift context (DMA staging on, off) and of a context
-    without a shift on the same grid."""
+    without a shift on the same grid, and whether the shift ones step fused."""
     def one(s, dma):
         g = gpu.BSSN(gpu.GpuParams(n=shape, order=order, lapse=lapse, shift=s, precision=prec, ko_coeff=ko))
         if lapse == "Static":
             g.upload("DIFFalpha_p", np.full(shape, 1e-3))  # as the tests that use these cases: a lapse that is not 1
         g.set_dma(dma)
-        return g.kernel_info()
-    return one(shift, True), one(shift, False), one("none", True), one("none", False)
+        return g.kernel_info(), s != "none" and steps_fused(gpu, g)
+    (on, f_on), (off, f_off) = one(shift, True), one(shift, False)
+    return on, off, one("none", True)[0], one("none", False)[0], f_on, f_off
 
 
 # the tests of the fused steps
@@ -41,19 +56,18 @@ REGISTERS = [((18, 14, 20), "GammaDriver", 4, "OnePlusLog", "fp64", 0.0), ((18, 
 
 @pytest.mark.parametrize("shape,shift,order,lapse,prec,ko", FUSED + EVEN + REGISTERS)
 def test_fused_kernel_runs(gpu, shape, shift, order, lapse, prec, ko):
-    on, off, plain_on, plain_off = infos(gpu, shape, shift, order, lapse, prec, ko)
+    on, off, plain_on, plain_off, f_on, f_off = infos(gpu, shape, shift, order, lapse, prec, ko)
+    assert f_on and not f_off
     assert on["tile"] == (4, 4, 16)
-    assert on != plain_on and on != off
     assert off == plain_off
 
 
 def test_fused_kernel_of_a_frozen_lapse(gpu):
-    def one(shift, dma):
-        g = gpu.BSSN(gpu.GpuParams(n=(18, 14, 20), order=4, lapse="Static", shift=shift, normalize_metric=0))
+    for dma in (True, False):
+        g = gpu.BSSN(gpu.GpuParams(n=(18, 14, 20), order=4, lapse="Static", shift="GammaDriver", normalize_metric=0))
         g.set_dma(dma)
-        return g.kernel_info()
-    assert one("GammaDriver", True) != one("none", True)
-    assert one("GammaDriver", True) != one("GammaDriver", False)
+        assert not dma or g.kernel_info()["tile"] == (4, 4, 16)
+        assert steps_fused(gpu, g) == dma
 
 
 # other fields' complete right-hand sides; a halo of 4; rows that are no whole 16-byte groups; fewer points than a tile needs
@@ -64,7 +78,8 @@ def test_fused_kernel_of_a_frozen_lapse(gpu):
                                                           ((18, 14, 22), "GammaDriver", 4, "OnePlusLog", "fp32_split"),
                                                           ((18, 14, 18), "GammaDriver", 4, "OnePlusLog", "fp64")])
 def test_no_fused_kernel(gpu, shape, shift, order, lapse, prec):
-    on, off, plain_on, plain_off = infos(gpu, shape, shift, order, lapse, prec)
+    on, off, plain_on, plain_off, f_on, f_off = infos(gpu, shape, shift, order, lapse, prec)
+    assert not f_on and not f_off
     assert on == plain_on and off == plain_off
 
 
@@ -93,7 +108,8 @@ def test_requested_tile(gpu):
         return g
 
     fused = ctx((4, 4, 16)).kernel_info()
-    assert fused == ctx((0, 0, 0)).kernel_info() and fused != ctx((4, 4, 16), "none").kernel_info()
+    assert fused == ctx((0, 0, 0)).kernel_info() and fused["tile"] == (4, 4, 16)
+    assert steps_fused(gpu, ctx((4, 4, 16))) and not steps_fused(gpu, ctx((4, 8, 8)))
     g = ctx((4, 8, 8))
     assert g.kernel_info() == ctx((4, 8, 8), "none").kernel_info()
     g.step(2)
@@ -109,4 +125,4 @@ def test_requested_tile(gpu):
     # the autotuner's pick is no request
     a = ctx((0, 0, 0))
     a.autotune(1)
-    assert a.kernel_info() == fused
+    assert a.kernel_info() == fused and steps_fused(gpu, a)
